@@ -25,7 +25,12 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FC = os.environ.get("PDR_FC", "/opt/rocm/bin/amdflang")
 ARCH = "gfx950"
 
-SOURCES = ["pdr_api.hip", "pdr_kernels.hip", "pdr_kernels2.hip", "pdr_host.hip", "pdr_stats.hip", "pdr_pstats.hip", "pdr_sort.hip", "pdr_ens.hip"]
+SPEC_TUS = 8  # kSpecTus of pdr_spec.hpp: pdr_spec.hip is compiled once for each group of line lengths
+# (source, extra defines, object); the costliest first
+SOURCES = [("pdr_ens_passes.hip", [], "pdr_ens_passes.o")]
+SOURCES += [("pdr_spec.hip", [f"-DPDR_SPEC_TU={k}"], f"pdr_spec_{k}.o") for k in range(SPEC_TUS)]
+SOURCES += [(f"{s}.hip", [], f"{s}.o") for s in ("pdr_api", "pdr_kernels", "pdr_spec_dispatch", "pdr_host", "pdr_stats",
+                                                 "pdr_pstats", "pdr_sort", "pdr_ens")]
 
 
 def _run(cmd, cwd=None):
@@ -34,14 +39,14 @@ def _run(cmd, cwd=None):
 
 
 def build_hip(verbose: bool = True) -> str:
-    """Compile every HIP source (in parallel, one hipcc per source) and link the library."""
+    """Compile every HIP source (in parallel, one hipcc per object) and link the library."""
     from concurrent.futures import ThreadPoolExecutor
 
     os.makedirs(LIB, exist_ok=True)
     cmds, objs = [], []
-    for src in SOURCES:
-        obj = os.path.join(LIB, os.path.splitext(src)[0] + ".o")
-        cmds.append([HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-c",
+    for src, defines, name in SOURCES:
+        obj = os.path.join(LIB, name)
+        cmds.append([HIPCC, *defines, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-c",
                      # no packed-FP32 instructions: some of their forms have given wrong results on gfx950
                      "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                      "-Wall", "-Wno-unused-parameter", "-Wno-unused-command-line-argument",

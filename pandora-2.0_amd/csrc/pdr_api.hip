@@ -438,9 +438,7 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     const char* env = std::getenv("PDR_GENERIC_KERNELS");
     const bool generic = env && env[0] && env[0] != '0';
     // NS_R_CONV runs on the generic kernels (its x pass takes twelve rows)
-    c->spec = !generic && !conv_form(c) && spec_supported(nx) && spec_supported(ny) && spec_supported(nz) &&
-              spec_shape_ok(nx, ny, nz) &&
-              spec_lds_need(c->prec, nx, ny, nz) <= c->lds_max;
+    c->spec = !generic && !conv_form(c) && spec_find(c);
   }
   // The x-pencil buffer may hold a chunk of zc planes instead of the whole box
   // (specialised kernels only): the y/x passes then run chunk by chunk.  It
@@ -573,8 +571,8 @@ int pdr_sizes(const pdr_ctx* c, int64_t out[8]) {
 
 int pdr_kernel_forms(const pdr_ctx* c, int32_t out[8]) {
   if (!c || !out) return fail(PDR_ERR_ARG, "pdr_kernel_forms: null argument");
-  int f[5] = {0, 0, 0, 0, 0};
-  if (c->spec) (void)spec_forms(c->prec, c->g.nx, c->g.ny, c->g.nz, f);
+  int f[4] = {0, 0, 0, 0};
+  if (c->spec) spec_forms(c, f);
   out[0] = c->spec ? 1 : 0;
   out[1] = c->g.zc;
   out[2] = c->zs2 ? 1 : 0;

@@ -4,7 +4,7 @@
 // A 32^3 box gives a pass a few dozen workgroups, so stepping each member on
 // its own leaves most of the 256 CUs idle and pays 15 kernel launches per step
 // per member.  Here every pass of an RK3 stage is one launch over the tiles of
-// all members (per-member work descriptors, pdr_kernels2.hip), and the 15
+// all members (per-member work descriptors, pdr_ens_passes.hip), and the 15
 // launches of a step are captured once into a HIP graph and replayed, so a
 // step costs one graph launch for the whole ensemble.  Each member runs the
 // device bodies that pdr_step runs for it, with the same arguments; they are

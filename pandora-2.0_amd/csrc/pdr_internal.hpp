@@ -110,6 +110,8 @@ enum KernelClass {
   K_NCLASS
 };
 
+struct SpecOps;  // pdr_spec.hpp
+
 struct Tables {
   void* twz = nullptr;
   void* twy = nullptr;
@@ -186,7 +188,8 @@ struct pdr_ctx {
   double dt = 99999.0;
   double ucfl = 0.0;
   // launch shapes
-  bool spec = false;  // length-specialised kernels (pdr_kernels2.hip)
+  bool spec = false;  // length-specialised kernels (pdr_passes.hpp)
+  const pdr::SpecOps *ops_x = nullptr, *ops_y = nullptr, *ops_z = nullptr;  // theirs for this box
   bool fuse_zf = true;  // fused z-forward + FormF (specialised path; PDR_FUSE_ZFORMF=0 disables)
   int tj_z = 1, ti_y = 1;
   size_t lds_max = 65536;
@@ -234,7 +237,7 @@ hipError_t launch_tracers(pdr_ctx* c, const TracerFrame& tf, double beta, double
 hipError_t launch_tracers_wrap(pdr_ctx* c, const TracerFrame& tf, hipStream_t s);
 hipError_t launch_remesh(pdr_ctx* c, int bfrot);
 hipError_t launch_remesh_particles(pdr_ctx* c, double lx, double dx);
-// batched ensemble passes (pdr_kernels2.hip)
+// batched ensemble passes (pdr_ens_passes.hip)
 bool ens_size_supported(int n);
 int ens_tiles(int prec, int n, const Geo& g, int fpb_y, int fpb_yf, int nt[5], unsigned blocks[5]);
 size_t ens_lds(int prec, int n, int pass);
@@ -271,11 +274,9 @@ void prof_end(pdr_ctx* c, int cls, hipStream_t s = nullptr);
 
 void fft_plan(FftPlan* p, int n);
 
-// length-specialised kernels (pdr_kernels2.hip)
-bool spec_shape_ok(int nx, int ny, int nz);
-int spec_forms(int prec, int nx, int ny, int nz, int out[5]);
-bool spec_supported(int n);
-size_t spec_lds_need(int prec, int nx, int ny, int nz);
+// length-specialised kernels (pdr_spec_dispatch.hip)
+bool spec_find(pdr_ctx* c);
+void spec_forms(const pdr_ctx* c, int out[4]);
 hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf);
 hipError_t launch2_yinv(pdr_ctx* c, int z0, int nzc);
 hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tracers, bool cfl, int z0, int nzc, double* rsp);

@@ -1,9 +1,10 @@
-// pdr_kernels2.hip -- length-specialised pass kernels (the default path for
-// grid sizes in PDR_SIZES).  Same work split and data layouts as pdr_kernels.hip
+// pdr_passes.hpp -- length-specialised pass kernels (the default path for the
+// grid sizes that pdr_spec.hip instantiates).  Same work split and data layouts as pdr_kernels.hip
 // (pass 1 k_zinv ... pass 5 k_zfwd); see that file for the reference routines
 // each pass replaces.  Differences: compile-time transform length and tile
 // height, in-place LDS transforms, twiddles in LDS, 128-byte tile chunks on
 // 16-element-padded strides, XCD-aware tile order, several x rows per block.
+#pragma once
 #include <type_traits>
 
 #include "pdr_fft2.hpp"
@@ -75,17 +76,19 @@ constexpr int tile_lines_fwd(int n) {
 // i-lines of each) instead of a tile of i-lines of one plane, so that it
 // moves about three thousand points and no tile is left part-empty
 // (PP = 0: tiles of tile_lines i-lines within one plane).
-template <typename T>
+// PL selects these plane tiles; they take the i-lines per plane from the pass's own
+// length (NKI = NY/3 + 1), so boxes with NX/3 != NY/3 run the tiles of i-lines.
+template <typename T, bool PL = true>
 constexpr int y_planes(int n) {
-  return n <= 32 ? 8 : (n <= 48 ? 4 : (n <= 64 ? 2 : (n <= 96 ? 1 : 0)));
+  return !PL ? 0 : n <= 32 ? 8 : (n <= 48 ? 4 : (n <= 64 ? 2 : (n <= 96 ? 1 : 0)));
 }
-template <typename T>
+template <typename T, bool PL = true>
 constexpr int y_lines(int n) {
-  return y_planes<T>(n) ? y_planes<T>(n) * (n / 3 + 1) : tile_lines<T>(n);
+  return y_planes<T, PL>(n) ? y_planes<T, PL>(n) * (n / 3 + 1) : tile_lines<T>(n);
 }
-template <typename T>
+template <typename T, bool PL = true>
 constexpr int y_lines_fwd(int n) {
-  return y_planes<T>(n) ? y_planes<T>(n) * (n / 3 + 1) : tile_lines_fwd<T>(n);
+  return y_planes<T, PL>(n) ? y_planes<T, PL>(n) * (n / 3 + 1) : tile_lines_fwd<T>(n);
 }
 
 // Short lines take more rows per workgroup, so that a workgroup still moves
@@ -110,13 +113,13 @@ template <typename T>
 constexpr int lds_fwd_bytes(int n) {
   return (n + tile_lines_fwd<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
 }
-template <typename T>
+template <typename T, bool PL = true>
 constexpr int lds_y_bytes(int n) {
-  return (n + y_lines<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
+  return (n + y_lines<T, PL>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
 }
-template <typename T>
+template <typename T, bool PL = true>
 constexpr int lds_yf_bytes(int n) {
-  return (n + y_lines_fwd<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
+  return (n + y_lines_fwd<T, PL>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
 }
 // The x tile of lines longer than PDR_X_TWG_MIN points reads its twiddles from
 // the global table (through the caches) instead of staging them in LDS: that
@@ -161,8 +164,7 @@ constexpr bool kNtZfwd = (PDR_NT_WRITES & 16) != 0;
 #define PDR_LINE_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_lines_bytes<T>(N)))))
 #define PDR_FWD_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_fwd_bytes<T>(N)))))
 #define PDR_X_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_x_bytes<T>(N)))))
-#define PDR_Y_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_y_bytes<T>(N)))))
-#define PDR_YF_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_yf_bytes<T>(N)))))
+#define PDR_YF_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_yf_bytes<T, PL>(N)))))
 
 // Line kernels issue all global loads of a field (QE elements per thread)
 // before the LDS stores of that field, so that one HBM latency is exposed per
@@ -411,11 +413,11 @@ __global__ void __launch_bounds__(PDR_ZINV_THREADS) PDR_ZINV_WAVES_T
 // ---------------------------------------------------------------------------
 // pass 2: inverse y FFT, (z, i-tile) per block
 // ---------------------------------------------------------------------------
-template <typename T, int N, int YT = kBlock2>
+template <typename T, int N, bool PL, int YT = kBlock2>
 __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
-  constexpr int PP = y_planes<T>(N);
-  constexpr int L = y_lines<T>(N);
+  constexpr int PP = y_planes<T, PL>(N);
+  constexpr int L = y_lines<T, PL>(N);
   constexpr int LD = lds_ld<T>(N);
   constexpr int K = N / 3;
   constexpr int NKJ = 2 * K + 1;
@@ -525,25 +527,25 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
 #ifndef PDR_YINV_THREADS
 #define PDR_YINV_THREADS 512
 #endif
-template <typename T, int N>
+template <typename T, int N, bool PL>
 constexpr int yinv_threads() {
-  return y_planes<T>(N) ? kBlock2 : PDR_YINV_THREADS;
+  return y_planes<T, PL>(N) ? kBlock2 : PDR_YINV_THREADS;
 }
 // waves per SIMD declared to the register allocator: as for the other passes
 // (at most two 256-thread workgroups), or the two waves per SIMD of each
 // 512-thread workgroup times the workgroups the LDS admits, at most four
-template <typename T, int N>
+template <typename T, int N, bool PL>
 constexpr int yinv_waves() {
-  constexpr int wg = kLdsPerCu / lds_y_bytes<T>(N) < 1 ? 1 : kLdsPerCu / lds_y_bytes<T>(N);
-  return yinv_threads<T, N>() == kBlock2 ? waves_for(lds_y_bytes<T>(N))
-                                          : (wg * (yinv_threads<T, N>() / kBlock2) > 4 ? 4 : wg * (yinv_threads<T, N>() / kBlock2));
+  constexpr int wg = kLdsPerCu / lds_y_bytes<T, PL>(N) < 1 ? 1 : kLdsPerCu / lds_y_bytes<T, PL>(N);
+  return yinv_threads<T, N, PL>() == kBlock2 ? waves_for(lds_y_bytes<T, PL>(N))
+                                          : (wg * (yinv_threads<T, N, PL>() / kBlock2) > 4 ? 4 : wg * (yinv_threads<T, N, PL>() / kBlock2));
 }
 
-template <typename T, int N>
-__global__ void __launch_bounds__((yinv_threads<T, N>())) __attribute__((amdgpu_waves_per_eu(yinv_waves<T, N>())))
+template <typename T, int N, bool PL>
+__global__ void __launch_bounds__((yinv_threads<T, N, PL>())) __attribute__((amdgpu_waves_per_eu(yinv_waves<T, N, PL>())))
     k2_yinv(Geo g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
-  k2_yinv_body<T, N, yinv_threads<T, N>()>(xcd_remap(blockIdx.x, gridDim.x), g, w1, w2, twg, ntile, z0, nzc, fpb);
+  k2_yinv_body<T, N, PL, yinv_threads<T, N, PL>()>(xcd_remap(blockIdx.x, gridDim.x), g, w1, w2, twg, ntile, z0, nzc, fpb);
 }
 
 // ---------------------------------------------------------------------------
@@ -794,11 +796,11 @@ __global__ void __launch_bounds__(kBlock2) PDR_X_WAVES
 // ---------------------------------------------------------------------------
 // pass 4: forward y FFT + truncation, (z, i-tile) per block
 // ---------------------------------------------------------------------------
-template <typename T, int N>
+template <typename T, int N, bool PL>
 __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const cx<T>* __restrict__ w2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
-  constexpr int PP = y_planes<T>(N);
-  constexpr int L = y_lines_fwd<T>(N);
+  constexpr int PP = y_planes<T, PL>(N);
+  constexpr int L = y_lines_fwd<T, PL>(N);
   constexpr int LD = lds_ld<T>(N);
   constexpr int K = N / 3;
   constexpr int NKJ = 2 * K + 1;
@@ -865,11 +867,11 @@ __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const c
   }
 }
 
-template <typename T, int N>
+template <typename T, int N, bool PL>
 __global__ void __launch_bounds__(kBlock2) PDR_YF_WAVES
     k2_yfwd(Geo g, const cx<T>* __restrict__ w2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
-  k2_yfwd_body<T, N>(xcd_remap(blockIdx.x, gridDim.x), g, w2, w1, twg, ntile, z0, nzc, fpb);
+  k2_yfwd_body<T, N, PL>(xcd_remap(blockIdx.x, gridDim.x), g, w2, w1, twg, ntile, z0, nzc, fpb);
 }
 
 // ---------------------------------------------------------------------------
@@ -1034,7 +1036,10 @@ size_t lds_fwd() {
 }
 template <typename T, int N>
 size_t lds_y() {
-  return size_t(lds_y_bytes<T>(N) > lds_yf_bytes<T>(N) ? lds_y_bytes<T>(N) : lds_yf_bytes<T>(N));
+  size_t m = 0;
+  for (int b : {lds_y_bytes<T, true>(N), lds_yf_bytes<T, true>(N), lds_y_bytes<T, false>(N), lds_yf_bytes<T, false>(N)})
+    m = size_t(b) > m ? size_t(b) : m;
+  return m;
 }
 template <typename T, int N>
 size_t lds_x() {
@@ -1072,18 +1077,26 @@ hipError_t zinv_n(pdr_ctx* c, const Coef& cf) {
   }
 }
 
-template <typename T, int N>
-hipError_t yinv_n(pdr_ctx* c, int z0, int nzc) {
+template <typename T, int N, bool PL>
+hipError_t yinv_t(pdr_ctx* c, int z0, int nzc) {
   const Geo& g = c->g;
-  constexpr int PP = y_planes<T>(N);
-  constexpr int L = y_lines<T>(N);
+  constexpr int PP = y_planes<T, PL>(N);
+  constexpr int L = y_lines<T, PL>(N);
   const int nt = PP ? (nzc + PP - 1) / PP : (g.nki + L - 1) / L;
-  const size_t lds = size_t(lds_y_bytes<T>(N));
-  hipError_t e = big_lds((const void*)k2_yinv<T, N>, lds);
+  const size_t lds = size_t(lds_y_bytes<T, PL>(N));
+  hipError_t e = big_lds((const void*)k2_yinv<T, N, PL>, lds);
   if (e != hipSuccess) return e;
-  k2_yinv<T, N><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (6 / c->fpb_y))), yinv_threads<T, N>(), lds, c->stream>>>(
+  k2_yinv<T, N, PL><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (6 / c->fpb_y))), yinv_threads<T, N, PL>(), lds, c->stream>>>(
       g, (const cx<T>*)c->w1, (cx<T>*)c->w2, (const cx<T>*)c->tab.twy, nt, z0, nzc, c->fpb_y);
   return hipGetLastError();
+}
+
+template <typename T, int N>
+hipError_t yinv_n(pdr_ctx* c, int z0, int nzc) {
+  if constexpr (y_planes<T>(N) > 0) {
+    if (c->g.nki == N / 3 + 1) return yinv_t<T, N, true>(c, z0, nzc);
+  }
+  return yinv_t<T, N, false>(c, z0, nzc);
 }
 
 template <typename T, int N>
@@ -1106,18 +1119,26 @@ hipError_t xpass_n(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nz
   return hipGetLastError();
 }
 
-template <typename T, int N>
-hipError_t yfwd_n(pdr_ctx* c, int z0, int nzc) {
+template <typename T, int N, bool PL>
+hipError_t yfwd_t(pdr_ctx* c, int z0, int nzc) {
   const Geo& g = c->g;
-  constexpr int PP = y_planes<T>(N);
-  constexpr int L = y_lines_fwd<T>(N);
+  constexpr int PP = y_planes<T, PL>(N);
+  constexpr int L = y_lines_fwd<T, PL>(N);
   const int nt = PP ? (nzc + PP - 1) / PP : (g.nki + L - 1) / L;
-  const size_t lds = size_t(lds_yf_bytes<T>(N));
-  hipError_t e = big_lds((const void*)k2_yfwd<T, N>, lds);
+  const size_t lds = size_t(lds_yf_bytes<T, PL>(N));
+  hipError_t e = big_lds((const void*)k2_yfwd<T, N, PL>, lds);
   if (e != hipSuccess) return e;
-  k2_yfwd<T, N><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (3 / c->fpb_yf))), kBlock2, lds, c->stream>>>(
+  k2_yfwd<T, N, PL><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (3 / c->fpb_yf))), kBlock2, lds, c->stream>>>(
       g, (const cx<T>*)c->w2, (cx<T>*)c->w1, (const cx<T>*)c->tab.twy, nt, z0, nzc, c->fpb_yf);
   return hipGetLastError();
+}
+
+template <typename T, int N>
+hipError_t yfwd_n(pdr_ctx* c, int z0, int nzc) {
+  if constexpr (y_planes<T>(N) > 0) {
+    if (c->g.nki == N / 3 + 1) return yfwd_t<T, N, true>(c, z0, nzc);
+  }
+  return yfwd_t<T, N, false>(c, z0, nzc);
 }
 
 template <typename T, int N>
@@ -1160,413 +1181,6 @@ hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Batched ensemble passes: one launch runs a pass for every member.  Block b
-// (after the XCD remap, so that a member's tiles share one XCD's L2) belongs to
-// the last member whose start is <= b; the member's descriptor supplies the
-// geometry, coefficients, buffers and tile counts, and a switch on its line
-// length selects the compile-time body that the single-box kernel also uses,
-// so each member computes what its own launches would (up to the rounding of
-// multiply-adds that the compiler contracts differently in another kernel).
-// ---------------------------------------------------------------------------
-#define PDR_ENS_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256)
-
-// member of block b of a pass: binary search of the members' first blocks
-__device__ __forceinline__ int ens_member(const EnsMember* __restrict__ mem, int nm, int pass, unsigned b) {
-  int lo = 0, hi = nm - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (mem[mid].start[pass] <= b)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock2) k_ens_zinv(const EnsMember* __restrict__ mem, int nm) {
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const EnsMember& e = mem[ens_member(mem, nm, 0, b)];
-  const unsigned lb = b - e.start[0];
-  switch (e.n) {
-#define PDR_EC(n)                                                                                                \
-  case n:                                                                                                        \
-    k2_zinv_r_body<T, n>(lb, e.g, e.cf, (const cx<T>*)e.u[0], (const cx<T>*)e.u[1], (const cx<T>*)e.u[2],        \
-                         (cx<T>*)e.w1, (const cx<T>*)e.twz, e.nt[0]);                                            \
-    break;
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      break;
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock2) k_ens_yinv(const EnsMember* __restrict__ mem, int nm) {
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const EnsMember& e = mem[ens_member(mem, nm, 1, b)];
-  const unsigned lb = b - e.start[1];
-  switch (e.n) {
-#define PDR_EC(n)                                                                                                \
-  case n:                                                                                                        \
-    k2_yinv_body<T, n>(lb, e.g, (const cx<T>*)e.w1, (cx<T>*)e.w2, (const cx<T>*)e.twy, e.nt[1], 0, e.g.nz,      \
-                       e.fpb_y);                                                                                 \
-    break;
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      break;
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock2) k_ens_xpass(const EnsMember* __restrict__ mem, int nm) {
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const EnsMember& e = mem[ens_member(mem, nm, 2, b)];
-  const unsigned lb = b - e.start[2];
-  switch (e.n) {
-#define PDR_EC(n)                                                                                                \
-  case n:                                                                                                        \
-    k2_xpass_body<T, n, false>(lb, e.g, e.cf, (cx<T>*)e.w2, (T*)nullptr, 0, 0, e.umax, (const cx<T>*)e.twx,      \
-                               e.nt[2], 0, nullptr);                                                             \
-    break;
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      break;
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock2) k_ens_yfwd(const EnsMember* __restrict__ mem, int nm) {
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const EnsMember& e = mem[ens_member(mem, nm, 3, b)];
-  const unsigned lb = b - e.start[3];
-  switch (e.n) {
-#define PDR_EC(n)                                                                                                \
-  case n:                                                                                                        \
-    k2_yfwd_body<T, n>(lb, e.g, (const cx<T>*)e.w2, (cx<T>*)e.w1, (const cx<T>*)e.twy, e.nt[3], 0, e.g.nz,      \
-                       e.fpb_yf);                                                                                \
-    break;
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      break;
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock2) k_ens_zfwd_formf(const EnsMember* __restrict__ mem, int nm, double beta,
-                                                          double gamma) {
-  const unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-  const EnsMember& e = mem[ens_member(mem, nm, 4, b)];
-  const unsigned lb = b - e.start[4];
-  const double gdt = gamma * e.dt;
-  switch (e.n) {
-#define PDR_EC(n)                                                                                                \
-  case n:                                                                                                        \
-    k2_zfwd_formf_body<T, n, kBlock2, 0>(lb, e.g, e.cf, (const cx<T>*)e.w1, (cx<T>*)e.u[0], (cx<T>*)e.u[1],  \
-                             (cx<T>*)e.u[2], (cx<T>*)e.rk[0], (cx<T>*)e.rk[1], (cx<T>*)e.rk[2], nullptr, 0, 0.0, \
-                             beta, gdt,                                                                          \
-                             (const cx<T>*)e.twz, e.nt[4], T(e.norm));                                           \
-    break;
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      break;
-  }
-}
-
-template <typename T, int N>
-int ens_tiles_n(const Geo& g, int fpb_y, int fpb_yf, int nt[5], unsigned blocks[5]) {
-  nt[0] = (g.nkj + zinv_lines<T>(N) - 1) / zinv_lines<T>(N);
-  constexpr int PP = y_planes<T>(N);
-  nt[1] = PP ? (g.nz + PP - 1) / PP : (g.nki + y_lines<T>(N) - 1) / y_lines<T>(N);
-  nt[2] = (g.ny + xrows<T>(N) - 1) / xrows<T>(N);
-  nt[3] = PP ? (g.nz + PP - 1) / PP : (g.nki + y_lines_fwd<T>(N) - 1) / y_lines_fwd<T>(N);
-  nt[4] = (g.nkj + tile_lines_fwd<T>(N) - 1) / tile_lines_fwd<T>(N);
-  blocks[0] = unsigned(nt[0] * g.nki);
-  blocks[1] = unsigned(nt[1] * (PP ? 1 : g.nz) * (6 / fpb_y));
-  blocks[2] = unsigned(nt[2] * g.nz);
-  blocks[3] = unsigned(nt[3] * (PP ? 1 : g.nz) * (3 / fpb_yf));
-  blocks[4] = unsigned(nt[4] * g.nki);
-  return 0;
-}
-
-template <typename T, int N>
-size_t ens_lds_n(int pass) {
-  switch (pass) {
-    case 0: return size_t(lds_zinv_bytes<T>(N));
-    case 1: return size_t(lds_y_bytes<T>(N));
-    case 2: return lds_x<T, N>();
-    case 3: return size_t(lds_yf_bytes<T>(N));
-    default: return lds_fwd<T, N>();
-  }
-}
-
 }  // namespace
-
-bool ens_size_supported(int n) {
-  switch (n) {
-#define PDR_EC(n) case n:
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    return true;
-    default:
-      return false;
-  }
-}
-
-int ens_tiles(int prec, int n, const Geo& g, int fpb_y, int fpb_yf, int nt[5], unsigned blocks[5]) {
-  switch (n) {
-#define PDR_EC(n)                                                                                     \
-  case n:                                                                                             \
-    return prec ? ens_tiles_n<float, n>(g, fpb_y, fpb_yf, nt, blocks)                                 \
-                : ens_tiles_n<double, n>(g, fpb_y, fpb_yf, nt, blocks);
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      return -1;
-  }
-}
-
-size_t ens_lds(int prec, int n, int pass) {
-  switch (n) {
-#define PDR_EC(n) \
-  case n:         \
-    return prec ? ens_lds_n<float, n>(pass) : ens_lds_n<double, n>(pass);
-    PDR_ENS_SIZES(PDR_EC)
-#undef PDR_EC
-    default:
-      return 0;
-  }
-}
-
-template <typename T>
-static hipError_t ens_prepare_t(size_t lds_max) {
-  const void* fns[5] = {(const void*)k_ens_zinv<T>, (const void*)k_ens_yinv<T>, (const void*)k_ens_xpass<T>,
-                        (const void*)k_ens_yfwd<T>, (const void*)k_ens_zfwd_formf<T>};
-  for (const void* f : fns) {
-    hipError_t e = big_lds(f, lds_max);
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
-hipError_t ens_prepare(int prec, size_t lds_max) {
-  return prec ? ens_prepare_t<float>(lds_max) : ens_prepare_t<double>(lds_max);
-}
-
-template <typename T>
-static void ens_launch_t(int pass, const EnsMember* mem, int nm, unsigned nblk, size_t lds, double beta,
-                         double gamma, hipStream_t s) {
-  const dim3 grid(nblk);
-  switch (pass) {
-    case 0: k_ens_zinv<T><<<grid, kBlock2, lds, s>>>(mem, nm); break;
-    case 1: k_ens_yinv<T><<<grid, kBlock2, lds, s>>>(mem, nm); break;
-    case 2: k_ens_xpass<T><<<grid, kBlock2, lds, s>>>(mem, nm); break;
-    case 3: k_ens_yfwd<T><<<grid, kBlock2, lds, s>>>(mem, nm); break;
-    default: k_ens_zfwd_formf<T><<<grid, kBlock2, lds, s>>>(mem, nm, beta, gamma); break;
-  }
-}
-
-hipError_t launch_ens_pass(int prec, int pass, const EnsMember* mem, int nm, unsigned nblk, size_t lds,
-                           double beta, double gamma, hipStream_t s) {
-  if (prec)
-    ens_launch_t<float>(pass, mem, nm, nblk, lds, beta, gamma, s);
-  else
-    ens_launch_t<double>(pass, mem, nm, nblk, lds, beta, gamma, s);
-  return hipGetLastError();
-}
-
-namespace {
-}  // namespace
-
-#define PDR_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024) X(1536)
-
-int xpass_tiles(const pdr_ctx* c) {
-  switch (c->g.nx) {
-#define PDR_XT(n) \
-  case n:         \
-    return c->prec ? (c->g.ny + xrows<float>(n) - 1) / xrows<float>(n) : (c->g.ny + xrows<double>(n) - 1) / xrows<double>(n);
-    PDR_SIZES(PDR_XT)
-#undef PDR_XT
-    default:
-      return c->g.ny;
-  }
-}
-
-// Compile-time forms the specialised kernels take for this box: out[0] x rows
-// per x-pass workgroup, out[1] 1 if the x tile reads its twiddles from the
-// global table, out[2] 1 for the register z inverse (velocity tile loaded once),
-// out[3] lines per z-inverse tile, out[4] lines per inverse y tile (or whole
-// planes x NKI for short lines).  Returns -1 for lengths without a specialised
-// kernel.
-int spec_forms(int prec, int nx, int ny, int nz, int out[5]) {
-  int ok = 0;
-  auto fx = [&](auto tag, auto nn) {
-    using T = decltype(tag);
-    constexpr int n = decltype(nn)::value;
-    out[0] = xrows<T>(n);
-    out[1] = x_tw_global<T>(n) ? 1 : 0;
-    ++ok;
-  };
-  auto fz = [&](auto tag, auto nn) {
-    using T = decltype(tag);
-    constexpr int n = decltype(nn)::value;
-    out[2] = (PDR_ZINV_REG && n <= 512) ? 1 : 0;
-    out[3] = (PDR_ZINV_REG && n <= 512) ? zinv_lines_t<T, PDR_ZINV_THREADS>(n) : tile_lines<T>(n);
-    ++ok;
-  };
-  auto fy = [&](auto tag, auto nn) {
-    using T = decltype(tag);
-    constexpr int n = decltype(nn)::value;
-    out[4] = y_lines<T>(n);
-    ++ok;
-  };
-  auto dispatch = [&](int n, auto f) {
-    switch (n) {
-#define PDR_SF(n)                                                    \
-  case n:                                                            \
-    if (prec)                                                        \
-      f(float(0), std::integral_constant<int, n>{});                 \
-    else                                                             \
-      f(double(0), std::integral_constant<int, n>{});                \
-    break;
-      PDR_SIZES(PDR_SF)
-#undef PDR_SF
-      default:
-        break;
-    }
-  };
-  dispatch(nx, fx);
-  dispatch(nz, fz);
-  dispatch(ny, fy);
-  return ok == 3 ? 0 : -1;
-}
-
-// The whole-plane tiles of the y passes of short lines take the i-lines per
-// plane from the compile-time length of the pass: NKI = NY/3 + 1 must then be
-// the box's NX/3 + 1.
-bool spec_shape_ok(int nx, int ny, int nz) {
-  (void)nz;
-  return y_planes<float>(ny) == 0 || nx / 3 == ny / 3;
-}
-
-bool spec_supported(int n) {
-  switch (n) {
-#define PDR_CASE(n) case n:
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    return true;
-    default:
-      return false;
-  }
-}
-
-size_t spec_lds_need(int prec, int nx, int ny, int nz) {
-  size_t m = 0;
-  auto upd = [&](size_t v) { m = v > m ? v : m; };
-#define PDR_LDS(T, n, fn)            \
-  switch (n) {                       \
-    case 32: upd(fn<T, 32>()); break;     \
-    case 48: upd(fn<T, 48>()); break;     \
-    case 64: upd(fn<T, 64>()); break;     \
-    case 96: upd(fn<T, 96>()); break;     \
-    case 128: upd(fn<T, 128>()); break;   \
-    case 192: upd(fn<T, 192>()); break;   \
-    case 256: upd(fn<T, 256>()); break;   \
-    case 384: upd(fn<T, 384>()); break;   \
-    case 512: upd(fn<T, 512>()); break;   \
-    case 768: upd(fn<T, 768>()); break;   \
-    case 1024: upd(fn<T, 1024>()); break; \
-    case 1536: upd(fn<T, 1536>()); break; \
-    default: break;                  \
-  }
-  if (prec) {
-    PDR_LDS(float, nz, lds_lines)
-    PDR_LDS(float, ny, lds_lines)
-    PDR_LDS(float, nz, lds_fwd)
-    PDR_LDS(float, ny, lds_fwd)
-    PDR_LDS(float, ny, lds_y)
-    PDR_LDS(float, nx, lds_x)
-  } else {
-    PDR_LDS(double, nz, lds_lines)
-    PDR_LDS(double, ny, lds_lines)
-    PDR_LDS(double, nz, lds_fwd)
-    PDR_LDS(double, ny, lds_fwd)
-    PDR_LDS(double, ny, lds_y)
-    PDR_LDS(double, nx, lds_x)
-  }
-#undef PDR_LDS
-  return m;
-}
-
-#define PDR_DISPATCH(n, call_f, call_d) \
-  case n:                               \
-    return c->prec ? call_f : call_d;
-
-hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf) {
-  switch (c->g.nz) {
-#define PDR_CASE(n) PDR_DISPATCH(n, (zinv_n<float, n>(c, cf)), (zinv_n<double, n>(c, cf)))
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch2_yinv(pdr_ctx* c, int z0, int nzc) {
-  switch (c->g.ny) {
-#define PDR_CASE(n) PDR_DISPATCH(n, (yinv_n<float, n>(c, z0, nzc)), (yinv_n<double, n>(c, z0, nzc)))
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nzc, double* rsp) {
-  switch (c->g.nx) {
-#define PDR_CASE(n) \
-  PDR_DISPATCH(n, (xpass_n<float, n>(c, cf, tr, cfl, z0, nzc, rsp)), (xpass_n<double, n>(c, cf, tr, cfl, z0, nzc, rsp)))
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc) {
-  switch (c->g.ny) {
-#define PDR_CASE(n) PDR_DISPATCH(n, (yfwd_n<float, n>(c, z0, nzc)), (yfwd_n<double, n>(c, z0, nzc)))
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch2_zfwd(pdr_ctx* c) {
-  switch (c->g.nz) {
-#define PDR_CASE(n) PDR_DISPATCH(n, (zfwd_n<float, n>(c)), (zfwd_n<double, n>(c)))
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
-  switch (c->g.nz) {
-#define PDR_CASE(n) \
-  PDR_DISPATCH(n, (zfwd_formf_n<float, n>(c, cf, beta, gdt)), (zfwd_formf_n<double, n>(c, cf, beta, gdt)))
-    PDR_SIZES(PDR_CASE)
-#undef PDR_CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
 
 }  // namespace pdr

@@ -1,0 +1,51 @@
+// pdr_spec.hip -- the pass kernels of pdr_passes.hpp for the lengths of one
+// translation unit; compiled once per PDR_SPEC_TU (build_lib.py), so that the
+// lengths build side by side.
+#include "pdr_passes.hpp"
+#include "pdr_spec.hpp"
+
+#ifndef PDR_SPEC_TU
+#define PDR_SPEC_TU 0
+#endif
+#define PDR_CAT2(a, b) a##b
+#define PDR_CAT(a, b) PDR_CAT2(a, b)
+
+namespace pdr {
+
+namespace {
+
+template <typename T, int N>
+SpecOps ops_of() {
+  SpecOps o;
+  o.prec = sizeof(T) == 4 ? 1 : 0;
+  o.n = N;
+  o.zinv = zinv_n<T, N>;
+  o.yinv = yinv_n<T, N>;
+  o.xpass = xpass_n<T, N>;
+  o.yfwd = yfwd_n<T, N>;
+  o.zfwd = zfwd_n<T, N>;
+  o.zfwd_formf = zfwd_formf_n<T, N>;
+  o.lds_z = lds_lines<T, N>() > lds_fwd<T, N>() ? lds_lines<T, N>() : lds_fwd<T, N>();
+  o.lds_y = lds_y<T, N>();
+  o.lds_x = lds_x<T, N>();
+  o.xrows = xrows<T>(N);
+  o.x_tw_global = x_tw_global<T>(N) ? 1 : 0;
+  constexpr bool reg = PDR_ZINV_REG && N <= 512;
+  o.zinv_register = reg ? 1 : 0;
+  o.zinv_lines = reg ? zinv_lines_t<T, PDR_ZINV_THREADS>(N) : tile_lines<T>(N);
+  return o;
+}
+
+}  // namespace
+
+const SpecOps* PDR_CAT(spec_table_, PDR_SPEC_TU)(int* count) {
+  static const SpecOps t[] = {
+#define PDR_ROW(n) ops_of<float, n>(), ops_of<double, n>(),
+      PDR_CAT(PDR_SPEC_SIZES_, PDR_SPEC_TU)(PDR_ROW)
+#undef PDR_ROW
+  };
+  *count = int(sizeof(t) / sizeof(t[0]));
+  return t;
+}
+
+}  // namespace pdr

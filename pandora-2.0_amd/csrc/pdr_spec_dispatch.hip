@@ -1,0 +1,52 @@
+// pdr_spec_dispatch.hip -- from a box's line lengths to the specialised passes.
+#include "pdr_spec.hpp"
+
+namespace pdr {
+
+const SpecOps* spec_ops(int prec, int n) {
+  using Table = const SpecOps* (*)(int*);
+  static const Table tables[kSpecTus] = {spec_table_0, spec_table_1, spec_table_2, spec_table_3,
+                                         spec_table_4, spec_table_5, spec_table_6, spec_table_7};
+  for (Table f : tables) {
+    int count = 0;
+    const SpecOps* t = f(&count);
+    for (int q = 0; q < count; ++q)
+      if (t[q].n == n && t[q].prec == prec) return &t[q];
+  }
+  return nullptr;
+}
+
+// Finds the passes of the box's three lengths; false: a length has none, or its
+// tiles do not fit the LDS of a workgroup.
+bool spec_find(pdr_ctx* c) {
+  c->ops_x = spec_ops(c->prec, c->g.nx);
+  c->ops_y = spec_ops(c->prec, c->g.ny);
+  c->ops_z = spec_ops(c->prec, c->g.nz);
+  return c->ops_x && c->ops_y && c->ops_z && c->ops_x->lds_x <= c->lds_max && c->ops_y->lds_y <= c->lds_max &&
+         c->ops_z->lds_z <= c->lds_max;
+}
+
+// Forms the passes of this box take (pdr_kernel_forms): x rows per x-pass
+// workgroup, 1 if the x tile reads its twiddles from the global table, 1 for the
+// register z inverse (velocity tile loaded once), lines per z-inverse tile.
+void spec_forms(const pdr_ctx* c, int out[4]) {
+  out[0] = c->ops_x->xrows;
+  out[1] = c->ops_x->x_tw_global;
+  out[2] = c->ops_z->zinv_register;
+  out[3] = c->ops_z->zinv_lines;
+}
+
+int xpass_tiles(const pdr_ctx* c) { return (c->g.ny + c->ops_x->xrows - 1) / c->ops_x->xrows; }
+
+hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf) { return c->ops_z->zinv(c, cf); }
+hipError_t launch2_yinv(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yinv(c, z0, nzc); }
+hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nzc, double* rsp) {
+  return c->ops_x->xpass(c, cf, tr, cfl, z0, nzc, rsp);
+}
+hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yfwd(c, z0, nzc); }
+hipError_t launch2_zfwd(pdr_ctx* c) { return c->ops_z->zfwd(c); }
+hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
+  return c->ops_z->zfwd_formf(c, cf, beta, gdt);
+}
+
+}  // namespace pdr
