@@ -437,15 +437,19 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
   {
     const char* env = std::getenv("PDR_GENERIC_KERNELS");
     const bool generic = env && env[0] && env[0] != '0';
-    // NS_R_CONV runs on the generic kernels (its x pass takes twelve rows)
-    c->spec = !generic && !conv_form(c) && spec_find(c);
+    c->spec = !generic && spec_find(c);
   }
   // The x-pencil buffer may hold a chunk of zc planes instead of the whole box
   // (specialised kernels only): the y/x passes then run chunk by chunk.  It
   // costs time (measured at 512^3 FP32: 73 steps/s whole, 66 with 192 MB
   // chunks, 55 with 64 MB), so it is used only when the whole-box buffers
   // would not fit in device memory, or when PDR_ZCHUNK_MB asks for it.
-  if (c->spec) {
+  // NS_R_CONV keeps the whole box.
+  if (c->spec && conv_form(c)) {
+    const int tiles = (g.nki + 15) / 16;
+    c->fpb_y = tiles * g.nz * 2 < 1024 ? 1 : 3;
+    c->fpb_yf = tiles * g.nz < 1024 ? 1 : 3;
+  } else if (c->spec) {
     const char* env = std::getenv("PDR_ZCHUNK_MB");
     double mb = env && env[0] ? std::atof(env) : 0.0;
     const double plane = 6.0 * double(ny) * double(g.ldi) * double(c->csz);
@@ -516,10 +520,10 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     if (rc == PDR_OK) rc = dalloc(c, &c->rk[q], wbytes);
   }
   if (rc == PDR_OK) rc = dalloc(c, &c->w1, 6 * size_t(g.m1) * c->csz);
-  if (rc == PDR_OK) rc = dalloc(c, &c->w2, 6 * size_t(g.m2) * c->csz);
+  if (rc == PDR_OK) rc = dalloc(c, &c->w2, (c->spec && conv_form(c) ? 9 : 6) * size_t(g.m2) * c->csz);
   if (rc == PDR_OK && c->zs2) rc = dalloc(c, &c->w2z, 6 * size_t(g.m2) * c->csz);
   if (rc == PDR_OK) c->nl = static_cast<char*>(c->w1) + 3 * size_t(g.m1) * c->csz;
-  if (rc == PDR_OK && conv_form(c)) {
+  if (rc == PDR_OK && conv_form(c) && !c->spec) {
     for (void** q : {&c->w1b, &c->w1c})
       if (rc == PDR_OK) rc = dalloc(c, q, 6 * size_t(g.m1) * c->csz);
     for (void** q : {&c->w2b, &c->w2c})

@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(kBlock2) k_ens_yinv(const EnsMember* __restric
   switch (e.n) {
 #define PDR_EC(n)                                                                                                \
   case n:                                                                                                        \
-    k2_yinv_body<T, n, true>(lb, e.g, (const cx<T>*)e.w1, (cx<T>*)e.w2, (const cx<T>*)e.twy, e.nt[1], 0, e.g.nz,      \
+    k2_yinv_body<T, n, true, false>(lb, e.g, (const cx<T>*)e.w1, (cx<T>*)e.w2, (const cx<T>*)e.twy, e.nt[1], 0, e.g.nz,      \
                        e.fpb_y);                                                                                 \
     break;
     PDR_ENS_SIZES(PDR_EC)
@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(kBlock2) k_ens_xpass(const EnsMember* __restri
   switch (e.n) {
 #define PDR_EC(n)                                                                                                \
   case n:                                                                                                        \
-    k2_xpass_body<T, n, false>(lb, e.g, e.cf, (cx<T>*)e.w2, (T*)nullptr, 0, 0, e.umax, (const cx<T>*)e.twx,      \
+    k2_xpass_body<T, n, 0>(lb, e.g, e.cf, (cx<T>*)e.w2, (T*)nullptr, 0, 0, e.umax, (const cx<T>*)e.twx,      \
                                e.nt[2], 0, nullptr);                                                             \
     break;
     PDR_ENS_SIZES(PDR_EC)

@@ -131,8 +131,8 @@ struct pdr_ctx {
   void* rk[3] = {nullptr, nullptr, nullptr};
   // work buffers
   void* w1 = nullptr;  // 6 fields x m1 (1r2w layout)
-  void* w2 = nullptr;  // 6 fields x m2 (x-pencil layout, zc planes of z)
-  void *w1b = nullptr, *w1c = nullptr, *w2b = nullptr, *w2c = nullptr;  // NS_R_CONV: du/dy, du/dz sweeps
+  void* w2 = nullptr;  // 6 fields x m2 (x-pencil layout, zc planes of z); 9 with the specialised NS_R_CONV
+  void *w1b = nullptr, *w1c = nullptr, *w2b = nullptr, *w2c = nullptr;  // NS_R_CONV on the generic kernels: du/dy, du/dz sweeps
   void* nl = nullptr;  // NL [c][i][j][k] written by pass 5 (aliases w1 fields 3..5)
   int fpb_y = 6;       // fields per workgroup of the chunked inverse / forward y passes
   int fpb_yf = 3;
@@ -295,6 +295,8 @@ inline size_t conv_xpass_lds(int nx, size_t csz) { return 12 * size_t(nx + 1) * 
 Coef conv_coef(const Coef& cf, int d);  // G selecting field 3 + c = d u_c / d x_d
 hipError_t launch_conv_front(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp);
 hipError_t launch_dealias(pdr_ctx* c);  // no-op for DEALIASING = 1
+hipError_t launch2_yinv_conv(pdr_ctx* c);
+hipError_t launch2_xpass_conv(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp);
 hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc);
 hipError_t launch2_zfwd(pdr_ctx* c);
 hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt);

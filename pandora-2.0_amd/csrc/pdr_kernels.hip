@@ -1036,13 +1036,26 @@ Coef conv_coef(const Coef& cf, int d) {
   return r;
 }
 
-// NS_R_CONV front of a stage (generic kernels, whole box): three inverse z/y
+// NS_R_CONV front of a stage (whole box).  Specialised kernels: the z pass gives u and
+// du/dz, the y pass adds du/dy, the x pass du/dx.  Generic kernels: three inverse z/y
 // sweeps give u with du/dx, du/dy and du/dz (fields 3..5 of w, wb, wc), then
 // the convective x pass leaves NL in fields 0..2 of the x-pencil buffer.
 hipError_t launch_conv_front(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
   void* w1s[3] = {c->w1, c->w1b, c->w1c};
   void* w2s[3] = {c->w2, c->w2b, c->w2c};
   hipError_t e = hipSuccess;
+  if (c->spec) {
+    prof_begin(c, K_ZINV);
+    e = launch2_zinv(c, conv_coef(cf, 2));
+    prof_end(c, K_ZINV);
+    prof_begin(c, K_YINV);
+    if (e == hipSuccess) e = launch2_yinv_conv(c);
+    prof_end(c, K_YINV);
+    prof_begin(c, K_XPASS);
+    if (e == hipSuccess) e = launch2_xpass_conv(c, cf, tr, cfl, rsp);
+    prof_end(c, K_XPASS);
+    return e;
+  }
   prof_begin(c, K_ZINV);
   for (int d = 0; d < 3 && e == hipSuccess; ++d) {
     const Coef cd = conv_coef(cf, d);

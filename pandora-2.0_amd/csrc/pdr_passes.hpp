@@ -24,6 +24,12 @@ template <typename T>
 __device__ __forceinline__ cx<T> czero() {
   return mk<T>(T(0), T(0));
 }
+// i k a for the stored mode k (0..K, then -K..-1)
+template <typename T>
+__device__ __forceinline__ cx<T> mul_ik(cx<T> a, int k, int K) {
+  const T w = T(k <= K ? k : k - (2 * K + 1));
+  return mk<T>(-w * a.y, w * a.x);
+}
 
 // Tile shapes.  Lines per tile of the y/z kernels and rows per block of the x
 // kernel; the build may override the FP32 / FP64 values for lengths <= 512
@@ -413,7 +419,9 @@ __global__ void __launch_bounds__(PDR_ZINV_THREADS) PDR_ZINV_WAVES_T
 // ---------------------------------------------------------------------------
 // pass 2: inverse y FFT, (z, i-tile) per block
 // ---------------------------------------------------------------------------
-template <typename T, int N, bool PL, int YT = kBlock2>
+// DY: nine fields instead of six, fields 6..8 being d/dy of fields 0..2 (their modes
+// times i k2 on the way in)
+template <typename T, int N, bool PL, bool DY, int YT = kBlock2>
 __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
   constexpr int PP = y_planes<T, PL>(N);
@@ -442,7 +450,7 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
   constexpr int QM = PP > 0 ? QE : (EM + YT - 1) / YT;
   cx<T> pre[QM];
   auto load = [&](int f) {
-    const cx<T>* src = w1 + (long long)f * g.m1 + ((long long)i0 * g.nz + z) * g.ldj;
+    const cx<T>* src = w1 + (long long)(DY && f >= 6 ? f - 6 : f) * g.m1 + ((long long)i0 * g.nz + z) * g.ldj;
     if constexpr (PP == 0) {
 #pragma unroll
       for (int q = 0; q < QM; ++q) {
@@ -450,7 +458,7 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
         const int line = e / NKJ;
         cx<T> v = czero<T>();
         if ((EM % YT == 0 || e < EM) && i0 + line < nki) v = get<kNrYinv>(&src[line * lstride + (e - line * NKJ)]);
-        pre[q] = v;
+        pre[q] = DY && f >= 6 ? mul_ik<T>(v, e - line * NKJ, K) : v;
       }
       return;
     }
@@ -471,7 +479,7 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
         if ((L * N % YT == 0 || idx < L * N) && i0 + line < nki && j >= 0)
           v = get<kNrYinv>(&src[line * lstride + j]);
       }
-      pre[q] = v;
+      pre[q] = DY && f >= 6 ? mul_ik<T>(v, j, K) : v;
     }
   };
   for (int f = fg * fpb; f < (fg + 1) * fpb; ++f) {
@@ -541,17 +549,18 @@ constexpr int yinv_waves() {
                                           : (wg * (yinv_threads<T, N, PL>() / kBlock2) > 4 ? 4 : wg * (yinv_threads<T, N, PL>() / kBlock2));
 }
 
-template <typename T, int N, bool PL>
+template <typename T, int N, bool PL, bool DY>
 __global__ void __launch_bounds__((yinv_threads<T, N, PL>())) __attribute__((amdgpu_waves_per_eu(yinv_waves<T, N, PL>())))
     k2_yinv(Geo g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
-  k2_yinv_body<T, N, PL, yinv_threads<T, N, PL>()>(xcd_remap(blockIdx.x, gridDim.x), g, w1, w2, twg, ntile, z0, nzc, fpb);
+  k2_yinv_body<T, N, PL, DY, yinv_threads<T, N, PL>()>(xcd_remap(blockIdx.x, gridDim.x), g, w1, w2, twg, ntile, z0, nzc, fpb);
 }
 
 // ---------------------------------------------------------------------------
 // pass 3: RB rows (z, y0..y0+RB-1) per block: c2r, product, r2c
 // ---------------------------------------------------------------------------
-template <typename T, int N, bool RS, int XT = kBlock2>
+// Real-space moments (RS): 0 none; a thread's own points summed in FP32 (1) or FP64 (2).
+template <typename T, int N, int RS, int XT = kBlock2>
 __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const Coef& cf, cx<T>* __restrict__ w2, T* __restrict__ ur, int want_tr, int want_cfl,
              unsigned long long* __restrict__ umax, const cx<T>* __restrict__ twg, int ntile, int z0,
              double* __restrict__ rsp) {
@@ -662,7 +671,8 @@ __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const 
   T nl[IT][3];
   T lmax = T(0);
   T* urow = ur + ((long long)z * ny + y0) * N * 3;
-  RsAccT<T> acc;
+  using RA = std::conditional_t<RS == 2, double, T>;
+  RsAccT<RA> acc;
   if (RS) rs_init(acc);
   // the product, with the frame's form a compile-time choice (no per-point select)
   auto product = [&](auto form_c) {
@@ -694,7 +704,7 @@ __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const 
         const T s = fabs(v1) + fabs(v2) + fabs(v3);  // lab-frame velocity (src/pf_fluidstats.f90:853-866, 914)
         lmax = s > lmax ? s : lmax;
       }
-      if (RS && y0 + r < ny) rs_add(acc, v1, v2, v3, o1, o2, o3);
+      if (RS && y0 + r < ny) rs_add(acc, RA(v1), RA(v2), RA(v3), RA(o1), RA(o2), RA(o3));
     }
   }
   };
@@ -702,15 +712,15 @@ __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const 
     product(std::true_type{});
   else
     product(std::false_type{});
-  if constexpr (RS) {
+  if constexpr (RS != 0) {
     // partial of this workgroup at its place in the whole box: (z, tile); where
     // the x tile can hold the threads' partials (the product has read it), they
     // are reduced through it
     double* const rso = rsp + ((long long)z * ntile + tile) * kRsWidth;
     __shared__ double rs_lds[kRsWidth * 4];
-    if constexpr (kRsWidth * (XT + 1) * sizeof(T) <= 3 * RB * LD * sizeof(cx<T>)) {
+    if constexpr (kRsWidth * (XT + 1) * sizeof(RA) <= 3 * RB * LD * sizeof(cx<T>)) {
       __syncthreads();
-      rs_block_out_lds<XT>(acc, reinterpret_cast<T*>(buf), rs_lds, rso);
+      rs_block_out_lds<XT>(acc, reinterpret_cast<RA*>(buf), rs_lds, rso);
     } else {
       static_assert(kRsWidth * (XT / 64) <= kRsWidth * 4, "rs_block_out's LDS");
       rs_block_out(acc, rs_lds, rso);
@@ -784,13 +794,191 @@ __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const 
   }
 }
 
-template <typename T, int N, bool RS>
+template <typename T, int N, int RS>
 __global__ void __launch_bounds__(kBlock2) PDR_X_WAVES
     k2_xpass(Geo g, Coef cf, cx<T>* __restrict__ w2, T* __restrict__ ur, int want_tr, int want_cfl,
              unsigned long long* __restrict__ umax, const cx<T>* __restrict__ twg, int ntile, int z0,
              double* __restrict__ rsp) {
   k2_xpass_body<T, N, RS>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w2, ur, want_tr, want_cfl, umax, twg, ntile, z0,
                           rsp);
+}
+
+// ---------------------------------------------------------------------------
+// pass 3, NS_R_CONV: the y pass hands over u, du/dz and du/dy (fields 0..2, 3..5 and
+// 6..8); du/dx is formed here, its modes times i k1 on the way into the tile.  RB rows
+// per block, six complex lines of two real rows each: (u1, u2), (u3, dz u1),
+// (dz u2, dz u3), (dy u1, dy u2), (dy u3, dx u1), (dx u2, dx u3); then
+// NL_i = sum_j sum_k bmat(k,j) du_i/dx_k u_j (f_RK3ComputeNonlinearRConv,
+// src/pf_rk3.f90:1717-1774) and the forward lines of k2_xpass.  Forming each
+// derivative in its own pass moves 6 fields through the z pass and 9 through the y
+// pass, where transforming u and nine gradients from the z pass on moves 18 and 18
+// (three sweeps of six): ten FP64 steps at 96^3 14.7 -> 3.39 ms against the
+// runtime-radix kernels' three sweeps (launch_conv_front).  The moments take u, binv u and du/dx, as the reference's
+// f_FluidstatsRs2D reads u4..u6 (src/pf_fluidstats.f90:846-917), summed in FP64.
+// ---------------------------------------------------------------------------
+template <typename T>
+constexpr int xrows_conv(int n) {  // half the rows of k2_xpass: twice the lines a row
+  return xrows<T>(n) > 4 ? xrows<T>(n) / 2 : 2;
+}
+template <typename T>
+constexpr int lds_xc_bytes(int n) {
+  return ((x_tw_global<T>(n) ? 0 : n) + 6 * xrows_conv<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
+}
+#define PDR_XC_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_xc_bytes<T>(N)))))
+
+template <typename T, int N, bool RS>
+__global__ void __launch_bounds__(kBlock2) PDR_XC_WAVES
+    k2_xpass_conv(Geo g, Coef cf, cx<T>* __restrict__ w2, T* __restrict__ ur, int want_tr, int want_cfl,
+                  unsigned long long* __restrict__ umax, const cx<T>* __restrict__ twg, int ntile,
+                  double* __restrict__ rsp) {
+  constexpr int RB = xrows_conv<T>(N);
+  constexpr int LD = lds_ld<T>(N);
+  constexpr int KI = N / 3;
+  constexpr int NKI = KI + 1;
+  constexpr int IT = (RB * N + kBlock2 - 1) / kBlock2;  // product items per thread
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ T red[kBlock2 / 64];
+  constexpr bool TWG = x_tw_global<T>(N);
+  cx<T>* const lds0 = reinterpret_cast<cx<T>*>(smem);
+  const cx<T>* const tw = TWG ? twg : lds0;
+  cx<T>* const buf = TWG ? lds0 : lds0 + N;
+  const unsigned bid = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = int(bid % unsigned(ntile));
+  const int z = int(bid / unsigned(ntile));
+  const int y0 = tile * RB;
+  const int ny = g.ny;
+  if constexpr (!TWG) load_tw<T, N>(lds0, twg);
+  cx<T>* rowp = w2 + ((long long)z * ny + y0) * g.ldi;
+  // one (row, mode) per thread: nine modes in, twelve out as six packed lines, each
+  // at its mode and its Hermitian image (c2r uses only the real part of the DC term)
+  for (int idx = threadIdx.x; idx < RB * NKI; idx += kBlock2) {
+    const int r = idx / NKI;
+    const int m = idx - r * NKI;
+    cx<T> f[12];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) f[q] = (y0 + r < ny) ? rowp[(long long)q * g.m2 + r * g.ldi + m] : czero<T>();
+#pragma unroll
+    for (int q = 0; q < 3; ++q) f[9 + q] = mk<T>(-T(m) * f[q].y, T(m) * f[q].x);
+    cx<T>* row = buf + 6 * r * LD;
+    const int om = lds_off<T>(m), on = lds_off<T>(N - m);
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+      const cx<T> A = f[2 * p], B = f[2 * p + 1];
+      if (m == 0) {
+        row[p * LD] = mk<T>(A.x, B.x);
+      } else {
+        row[p * LD + om] = mk<T>(A.x - B.y, A.y + B.x);
+        row[p * LD + on] = mk<T>(A.x + B.y, B.x - A.y);
+      }
+    }
+  }
+  zero_band_edges<T, N, 6 * RB, LD, KI>(buf);
+  __syncthreads();
+  fft_ip<T, N, 6 * RB, LD, +1, !TWG, kBlock2, KI>(buf, tw);
+  T V[9], Bk[9];  // masked binv; bmat as [k][j]
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    V[q] = T(cf.V[q]);
+    Bk[q] = T(cf.Bm[q]);
+  }
+  T nl[IT][3];
+  T lmax = T(0);
+  T* urow = ur + ((long long)z * ny + y0) * N * 3;
+  RsAcc acc;
+  if (RS) rs_init(acc);
+#pragma unroll
+  for (int q = 0; q < IT; ++q) {
+    const int idx = int(threadIdx.x) + kBlock2 * q;
+    if ((RB * N) % kBlock2 == 0 || idx < RB * N) {
+      const int r = idx / N;
+      const int x = idx - r * N;
+      T f[12];  // u, du/dz, du/dy, du/dx
+#pragma unroll
+      for (int p = 0; p < 6; ++p) {
+        const cx<T> v = buf[(6 * r + p) * LD + lds_off<T>(x)];
+        f[2 * p] = v.x;
+        f[2 * p + 1] = v.y;
+      }
+      const int at[3] = {9, 6, 3};  // d/dx, d/dy, d/dz
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        T a = T(0);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) a = a + (Bk[3 * k + j] * f[at[k] + i] * f[j]);
+        nl[q][i] = a;
+      }
+      if (want_tr && y0 + r < ny) {
+        T* d = urow + idx * 3;
+        put1<kNtXpass>(d, f[0]);
+        put1<kNtXpass>(d + 1, f[1]);
+        put1<kNtXpass>(d + 2, f[2]);
+      }
+      if (want_cfl || RS) {
+        const T v1 = V[0] * f[0] + V[1] * f[1] + V[2] * f[2];
+        const T v2 = V[3] * f[0] + V[4] * f[1] + V[5] * f[2];
+        const T v3 = V[6] * f[0] + V[7] * f[1] + V[8] * f[2];
+        const T s = fabs(v1) + fabs(v2) + fabs(v3);
+        lmax = s > lmax ? s : lmax;
+        if (RS && y0 + r < ny)
+          rs_add(acc, double(v1), double(v2), double(v3), double(f[9]), double(f[10]), double(f[11]));
+      }
+    }
+  }
+  if constexpr (RS) {
+    __shared__ double rs_lds[kRsWidth * (kBlock2 / 64)];
+    rs_block_out(acc, rs_lds, rsp + ((long long)z * ntile + tile) * kRsWidth);
+  }
+  __syncthreads();
+  // forward lines and stored modes as in k2_xpass: r -> n1 + i n2 of row r,
+  // RB + r/2 -> n3 of rows (r, r+1)
+#pragma unroll
+  for (int q = 0; q < IT; ++q) {
+    const int idx = int(threadIdx.x) + kBlock2 * q;
+    if ((RB * N) % kBlock2 == 0 || idx < RB * N) {
+      const int r = idx / N;
+      const int x = idx - r * N;
+      buf[r * LD + lds_off<T>(x)] = mk<T>(nl[q][0], nl[q][1]);
+      cx<T>* p3 = &buf[(RB + r / 2) * LD + lds_off<T>(x)];
+      if (r & 1)
+        p3->y = nl[q][2];
+      else
+        p3->x = nl[q][2];
+    }
+  }
+  __syncthreads();
+  fft_ip<T, N, 3 * RB / 2, LD, -1, !TWG>(buf, tw);
+  for (int idx = threadIdx.x; idx < RB * NKI; idx += kBlock2) {
+    const int r = idx / NKI;
+    const int m = idx - r * NKI;
+    if (y0 + r >= ny) continue;
+    const int om = lds_off<T>(m), omr = lds_off<T>((m == 0) ? 0 : N - m);
+    const cx<T> Z = buf[r * LD + om], Zr = buf[r * LD + omr];
+    const cx<T> W = buf[(RB + r / 2) * LD + om], Wr = buf[(RB + r / 2) * LD + omr];
+    cx<T>* d0 = rowp + r * g.ldi + m;
+    put<kNtXpass>(d0, mk<T>(T(0.5) * (Z.x + Zr.x), T(0.5) * (Z.y - Zr.y)));
+    put<kNtXpass>(d0 + g.m2, mk<T>(T(0.5) * (Z.y + Zr.y), T(-0.5) * (Z.x - Zr.x)));
+    if (r & 1)
+      put<kNtXpass>(d0 + 2 * g.m2, mk<T>(T(0.5) * (W.y + Wr.y), T(-0.5) * (W.x - Wr.x)));
+    else
+      put<kNtXpass>(d0 + 2 * g.m2, mk<T>(T(0.5) * (W.x + Wr.x), T(0.5) * (W.y - Wr.y)));
+  }
+  if (want_cfl) {
+    T m = lmax;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const T o = __shfl_xor(m, off);
+      m = o > m ? o : m;
+    }
+    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      T r = red[0];
+      for (int w = 1; w < kBlock2 / 64; ++w) r = red[w] > r ? red[w] : r;
+      atomicMax(umax, (unsigned long long)__double_as_longlong(double(r)));
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1077,26 +1265,39 @@ hipError_t zinv_n(pdr_ctx* c, const Coef& cf) {
   }
 }
 
-template <typename T, int N, bool PL>
+template <typename T, int N, bool PL, bool DY>
 hipError_t yinv_t(pdr_ctx* c, int z0, int nzc) {
   const Geo& g = c->g;
   constexpr int PP = y_planes<T, PL>(N);
   constexpr int L = y_lines<T, PL>(N);
   const int nt = PP ? (nzc + PP - 1) / PP : (g.nki + L - 1) / L;
   const size_t lds = size_t(lds_y_bytes<T, PL>(N));
-  hipError_t e = big_lds((const void*)k2_yinv<T, N, PL>, lds);
+  hipError_t e = big_lds((const void*)k2_yinv<T, N, PL, DY>, lds);
   if (e != hipSuccess) return e;
-  k2_yinv<T, N, PL><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (6 / c->fpb_y))), yinv_threads<T, N, PL>(), lds, c->stream>>>(
-      g, (const cx<T>*)c->w1, (cx<T>*)c->w2, (const cx<T>*)c->tab.twy, nt, z0, nzc, c->fpb_y);
+  // nine fields split over workgroups by one or three
+  const int fpb = DY ? (c->fpb_y >= 3 ? 3 : 1) : c->fpb_y;
+  k2_yinv<T, N, PL, DY>
+      <<<dim3(unsigned(nt * (PP ? 1 : nzc) * ((DY ? 9 : 6) / fpb))), yinv_threads<T, N, PL>(), lds, c->stream>>>(
+          g, (const cx<T>*)c->w1, (cx<T>*)c->w2, (const cx<T>*)c->tab.twy, nt, z0, nzc, fpb);
   return hipGetLastError();
 }
 
-template <typename T, int N>
+template <typename T, int N, bool DY>
 hipError_t yinv_n(pdr_ctx* c, int z0, int nzc) {
   if constexpr (y_planes<T>(N) > 0) {
-    if (c->g.nki == N / 3 + 1) return yinv_t<T, N, true>(c, z0, nzc);
+    if (c->g.nki == N / 3 + 1) return yinv_t<T, N, true, DY>(c, z0, nzc);
   }
-  return yinv_t<T, N, false>(c, z0, nzc);
+  return yinv_t<T, N, false, DY>(c, z0, nzc);
+}
+
+// FP32-mixed boxes whose moments a thread sums in FP32 over its own points: cubes
+// and long boxes of 2^a or 3 2^a points; every other shape sums them in FP64 (the
+// sums across threads are FP64 in both).
+constexpr bool rs_fp32_len(int n) {
+  return n >= 32 && ((n & (n - 1)) == 0 || (n % 3 == 0 && ((n / 3) & (n / 3 - 1)) == 0));
+}
+inline bool rs_fp32_box(const Geo& g) {
+  return rs_fp32_len(g.nx) && rs_fp32_len(g.ny) && rs_fp32_len(g.nz) && (g.ny > 96 || g.nx / 3 == g.ny / 3);
 }
 
 template <typename T, int N>
@@ -1105,18 +1306,36 @@ hipError_t xpass_n(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nz
   constexpr int RB = xrows<T>(N);
   const int nt = (g.ny + RB - 1) / RB;
   const size_t lds = lds_x<T, N>();
-  if (rsp) {
-    hipError_t e = big_lds((const void*)k2_xpass<T, N, true>, lds);
+  auto launch = [&](auto rs_c) -> hipError_t {
+    constexpr int RS = decltype(rs_c)::value;
+    hipError_t e = big_lds((const void*)k2_xpass<T, N, RS>, lds);
     if (e != hipSuccess) return e;
-    k2_xpass<T, N, true><<<dim3(unsigned(nt * nzc)), kBlock2, lds, c->stream>>>(
+    k2_xpass<T, N, RS><<<dim3(unsigned(nt * nzc)), kBlock2, lds, c->stream>>>(
         g, cf, (cx<T>*)c->w2, (T*)c->ur, tr ? 1 : 0, cfl ? 1 : 0, c->umax, (const cx<T>*)c->tab.twx, nt, z0, rsp);
     return hipGetLastError();
+  };
+  if (!rsp) return launch(std::integral_constant<int, 0>{});
+  if constexpr (sizeof(T) == 4 && rs_fp32_len(N)) {
+    if (rs_fp32_box(g)) return launch(std::integral_constant<int, 1>{});
   }
-  hipError_t e = big_lds((const void*)k2_xpass<T, N, false>, lds);
-  if (e != hipSuccess) return e;
-  k2_xpass<T, N, false><<<dim3(unsigned(nt * nzc)), kBlock2, lds, c->stream>>>(
-      g, cf, (cx<T>*)c->w2, (T*)c->ur, tr ? 1 : 0, cfl ? 1 : 0, c->umax, (const cx<T>*)c->tab.twx, nt, z0, rsp);
-  return hipGetLastError();
+  return launch(std::integral_constant<int, 2>{});
+}
+
+template <typename T, int N>
+hipError_t xpass_conv_n(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
+  const Geo& g = c->g;
+  constexpr int RB = xrows_conv<T>(N);
+  const int nt = (g.ny + RB - 1) / RB;
+  const size_t lds = size_t(lds_xc_bytes<T>(N));
+  auto launch = [&](auto rs_c) -> hipError_t {
+    constexpr bool RS = decltype(rs_c)::value;
+    hipError_t e = big_lds((const void*)k2_xpass_conv<T, N, RS>, lds);
+    if (e != hipSuccess) return e;
+    k2_xpass_conv<T, N, RS><<<dim3(unsigned(nt * g.nz)), kBlock2, lds, c->stream>>>(
+        g, cf, (cx<T>*)c->w2, (T*)c->ur, tr ? 1 : 0, cfl ? 1 : 0, c->umax, (const cx<T>*)c->tab.twx, nt, rsp);
+    return hipGetLastError();
+  };
+  return rsp ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 template <typename T, int N, bool PL>

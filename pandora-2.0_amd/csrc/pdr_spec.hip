@@ -20,7 +20,9 @@ SpecOps ops_of() {
   o.prec = sizeof(T) == 4 ? 1 : 0;
   o.n = N;
   o.zinv = zinv_n<T, N>;
-  o.yinv = yinv_n<T, N>;
+  o.yinv = yinv_n<T, N, false>;
+  o.yinv_conv = yinv_n<T, N, true>;
+  o.xpass_conv = xpass_conv_n<T, N>;
   o.xpass = xpass_n<T, N>;
   o.yfwd = yfwd_n<T, N>;
   o.zfwd = zfwd_n<T, N>;
@@ -28,7 +30,9 @@ SpecOps ops_of() {
   o.lds_z = lds_lines<T, N>() > lds_fwd<T, N>() ? lds_lines<T, N>() : lds_fwd<T, N>();
   o.lds_y = lds_y<T, N>();
   o.lds_x = lds_x<T, N>();
+  o.lds_xc = size_t(lds_xc_bytes<T>(N));
   o.xrows = xrows<T>(N);
+  o.xrows_conv = xrows_conv<T>(N);
   o.x_tw_global = x_tw_global<T>(N) ? 1 : 0;
   constexpr bool reg = PDR_ZINV_REG && N <= 512;
   o.zinv_register = reg ? 1 : 0;

@@ -10,11 +10,13 @@ struct SpecOps {
   hipError_t (*zinv)(pdr_ctx*, const Coef&);
   hipError_t (*yinv)(pdr_ctx*, int z0, int nzc);
   hipError_t (*xpass)(pdr_ctx*, const Coef&, bool tr, bool cfl, int z0, int nzc, double* rsp);
+  hipError_t (*yinv_conv)(pdr_ctx*, int z0, int nzc);  // NS_R_CONV: also d/dy of the velocity
+  hipError_t (*xpass_conv)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
   hipError_t (*yfwd)(pdr_ctx*, int z0, int nzc);
   hipError_t (*zfwd)(pdr_ctx*);
   hipError_t (*zfwd_formf)(pdr_ctx*, const Coef&, double beta, double gdt);
-  size_t lds_z, lds_y, lds_x;  // the largest workgroup of the z, y and x passes
-  int xrows;                   // rows of an x tile
+  size_t lds_z, lds_y, lds_x, lds_xc;  // the largest workgroup of the z, y, x and NS_R_CONV x passes
+  int xrows, xrows_conv;       // rows of an x tile
   int x_tw_global;             // 1: the x tile reads its twiddles from the global table
   int zinv_register;           // 1: register z inverse
   int zinv_lines;              // lines of a z inverse tile

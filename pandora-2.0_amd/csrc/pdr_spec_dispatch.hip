@@ -22,7 +22,7 @@ bool spec_find(pdr_ctx* c) {
   c->ops_x = spec_ops(c->prec, c->g.nx);
   c->ops_y = spec_ops(c->prec, c->g.ny);
   c->ops_z = spec_ops(c->prec, c->g.nz);
-  return c->ops_x && c->ops_y && c->ops_z && c->ops_x->lds_x <= c->lds_max && c->ops_y->lds_y <= c->lds_max &&
+  return c->ops_x && c->ops_y && c->ops_z && (conv_form(c) ? c->ops_x->lds_xc : c->ops_x->lds_x) <= c->lds_max && c->ops_y->lds_y <= c->lds_max &&
          c->ops_z->lds_z <= c->lds_max;
 }
 
@@ -30,18 +30,25 @@ bool spec_find(pdr_ctx* c) {
 // workgroup, 1 if the x tile reads its twiddles from the global table, 1 for the
 // register z inverse (velocity tile loaded once), lines per z-inverse tile.
 void spec_forms(const pdr_ctx* c, int out[4]) {
-  out[0] = c->ops_x->xrows;
+  out[0] = conv_form(c) ? c->ops_x->xrows_conv : c->ops_x->xrows;
   out[1] = c->ops_x->x_tw_global;
   out[2] = c->ops_z->zinv_register;
   out[3] = c->ops_z->zinv_lines;
 }
 
-int xpass_tiles(const pdr_ctx* c) { return (c->g.ny + c->ops_x->xrows - 1) / c->ops_x->xrows; }
+int xpass_tiles(const pdr_ctx* c) {
+  const int rb = conv_form(c) ? c->ops_x->xrows_conv : c->ops_x->xrows;
+  return (c->g.ny + rb - 1) / rb;
+}
 
 hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf) { return c->ops_z->zinv(c, cf); }
 hipError_t launch2_yinv(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yinv(c, z0, nzc); }
 hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nzc, double* rsp) {
   return c->ops_x->xpass(c, cf, tr, cfl, z0, nzc, rsp);
+}
+hipError_t launch2_yinv_conv(pdr_ctx* c) { return c->ops_y->yinv_conv(c, 0, c->g.nz); }
+hipError_t launch2_xpass_conv(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
+  return c->ops_x->xpass_conv(c, cf, tr, cfl, rsp);
 }
 hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yfwd(c, z0, nzc); }
 hipError_t launch2_zfwd(pdr_ctx* c) { return c->ops_z->zfwd(c); }
