@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "pdr_internal.hpp"
+#include "pdr_spec.hpp"
 
 using namespace pdr;
 
@@ -481,6 +482,7 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     // (1536^3 FP64: 0.750 against 0.771 steps/s).  PDR_ZSTREAMS=2 forces it,
     // 1 turns it off; the same buffer bytes either way.
     const char* zs = std::getenv("PDR_ZSTREAMS");
+    c->plane_separate = (zs && zs[0]) || (env && env[0]);
     c->zs2 = (zs && zs[0] ? zs[0] == '2' : (c->prec == 0 && nz >= 1024 && zc == nz)) && nz > 1;
     if (c->zs2) zc = std::min(zc, (nz + 1) / 2);
     g.zc = zc;
@@ -498,6 +500,11 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     const char* env = std::getenv("PDR_FUSE_ZFORMF");
     c->fuse_zf = !(env && env[0] == '0') && nz <= 512;
   }
+  // fused planes: groups of a plane's parts on their own workgroups until the chip's
+  // 256 CUs have one each (the z forward pass then adds their results; the separate z
+  // forward of long lines reads one).  A step of 64^3 FP64: 180 us with one group, 115
+  // with two, 91 with four; of 32^3 106, 69 and 53.
+  if (plane_fused(c) && c->fuse_zf) c->nl_parts = std::max(1, std::min({kNlParts, c->ops_x->plane_parts, (256 + nz - 1) / nz}));
   fft_plan(&c->pz, nz);
   fft_plan(&c->py, ny);
   fft_plan(&c->px, nx);
@@ -520,7 +527,8 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     if (rc == PDR_OK) rc = dalloc(c, &c->rk[q], wbytes);
   }
   if (rc == PDR_OK) rc = dalloc(c, &c->w1, 6 * size_t(g.m1) * c->csz);
-  if (rc == PDR_OK) rc = dalloc(c, &c->w2, (c->spec && conv_form(c) ? 9 : 6) * size_t(g.m2) * c->csz);
+  if (rc == PDR_OK) rc = dalloc(c, &c->w2, std::max((c->spec && conv_form(c) ? 9 : 6) * size_t(g.m2),
+                                                        3 * size_t(c->nl_parts) * size_t(g.m1)) * c->csz);
   if (rc == PDR_OK && c->zs2) rc = dalloc(c, &c->w2z, 6 * size_t(g.m2) * c->csz);
   if (rc == PDR_OK) c->nl = static_cast<char*>(c->w1) + 3 * size_t(g.m1) * c->csz;
   if (rc == PDR_OK && conv_form(c) && !c->spec) {
@@ -681,13 +689,18 @@ int pdr_synchronize(pdr_ctx* c) {
 }
 
 // f_RK3Remesh (src/pf_rk3.f90:3958-4049) + f_RK3RemeshWaveSpace frame updates (4056-4178)
-static int maybe_remesh(pdr_ctx* c, int tstep, int32_t* done) {
-  if (done) *done = 0;
-  if (c->p.f_type == PDR_F_ISOTROPIC || c->p.rk3_timestep != PDR_RK3_TIMESTEP_DECIDE) return PDR_OK;
+static bool remesh_due(const pdr_ctx* c, int tstep) {
+  if (c->p.f_type == PDR_F_ISOTROPIC || c->p.rk3_timestep != PDR_RK3_TIMESTEP_DECIDE) return false;
   const int b110 = box_stretch(c->p, 1);
   const int a = tstep - (b110 * c->p.f_remesh_t) - 1;
   const int b = 2 * b110 * c->p.f_remesh_t;
-  if (a % b != 0) return PDR_OK;  // Fortran mod truncates toward zero like C %
+  return a % b == 0;  // Fortran mod truncates toward zero like C %
+}
+
+static int maybe_remesh(pdr_ctx* c, int tstep, int32_t* done) {
+  if (done) *done = 0;
+  if (!remesh_due(c, tstep)) return PDR_OK;
+  const int b110 = box_stretch(c->p, 1);
   const TracerFrame tf = make_tracer_frame(c);
   HIPCHK(launch_remesh_particles(c, tf.lx, tf.dx));
   T9(c->binv, 1, 3) = (double(b110) * 0.5) / T9(c->bmat, 3, 3);
@@ -706,8 +719,37 @@ static hipError_t tracers_release(pdr_ctx* c, hipStream_t s) {
   return e;
 }
 
+// How a stage joins its neighbours inside pdr_step and pdr_run: z_ready on entry, the
+// previous stage has left this one's inverse z pass in w1; join, the next stage's may
+// be done with this one's z forward pass (z_ready then holds on return).
+struct StageLink {
+  bool z_ready = false;
+  bool join = false;
+  double tstart = 0.0;  // simtime at the start of the step
+};
+
+// Operator of the stage that follows, from the frame that pdr_update_b will set then.
+static Coef next_coef(pdr_ctx* c, int stage, int32_t tstep, double tstart, double dt) {
+  double b[9], bi[9];
+  std::memcpy(b, c->bmat, sizeof(b));
+  std::memcpy(bi, c->binv, sizeof(bi));
+  const double frac = stage == 1 ? 1.0 / 3.0 : (stage == 2 ? 3.0 / 4.0 : 1.0);
+  pdr_update_b(c, tstep, tstart + frac * dt);
+  const Coef f = make_coef(c);
+  std::memcpy(c->bmat, b, sizeof(b));
+  std::memcpy(c->binv, bi, sizeof(bi));
+  return f;
+}
+
+static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, StageLink* link);
+
 int pdr_stage(pdr_ctx* c, int32_t stage, int32_t tstep, double time, double* dt) {
   (void)time;
+  StageLink alone;
+  return stage_run(c, stage, tstep, dt, &alone);
+}
+
+static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, StageLink* link) {
   if (!c || !dt) return fail(PDR_ERR_ARG, "pdr_stage: null argument");
   if (stage < 1 || stage > 3) return fail(PDR_ERR_ARG, "stage must be 1, 2 or 3");
   if (stage == 1) {
@@ -746,8 +788,12 @@ int pdr_stage(pdr_ctx* c, int32_t stage, int32_t tstep, double time, double* dt)
     if (need_cfl) HIPCHK(hipMemsetAsync(c->umax, 0, sizeof(unsigned long long), c->stream));
     HIPCHK(launch_conv_front(c, cf, field, need_cfl, rsp));
     HIPCHK(launch_yfwd(c, 0, c->g.nz));
+  } else if (plane_fused(c)) {
+    if (!link->z_ready) HIPCHK(launch_zinv(c, cf));
+    if (need_cfl) HIPCHK(hipMemsetAsync(c->umax, 0, sizeof(unsigned long long), c->stream));
+    HIPCHK(launch_plane(c, cf, field, need_cfl, rsp));
   } else {
-    HIPCHK(launch_zinv(c, cf));
+    if (!link->z_ready) HIPCHK(launch_zinv(c, cf));
     if (need_cfl) HIPCHK(hipMemsetAsync(c->umax, 0, sizeof(unsigned long long), c->stream));
     // chunks touch disjoint planes of w1 and the tracer field; with two in
     // flight the odd ones run on zstream with their own x-pencil buffer
@@ -838,7 +884,12 @@ int pdr_stage(pdr_ctx* c, int32_t stage, int32_t tstep, double time, double* dt)
   // pdr_particles_finish_step
   if (c->forcing) HIPCHK(launch_force(c, tstep, *dt));  // f_ForceCalc (src/pf_rk3.f90:2063)
   if (c->spec && c->fuse_zf) {
-    HIPCHK(launch_zfwd_formf(c, cf, beta, gdt));
+    if (link->join) {
+      const Coef next = next_coef(c, stage, tstep, link->tstart, *dt);
+      HIPCHK(launch_zfwd_formf(c, cf, &next, beta, gdt));
+    } else {
+      HIPCHK(launch_zfwd_formf(c, cf, nullptr, beta, gdt));
+    }
   } else {
     HIPCHK(launch_zfwd(c));
     HIPCHK(launch_formf(c, cf, beta, gdt));
@@ -846,6 +897,7 @@ int pdr_stage(pdr_ctx* c, int32_t stage, int32_t tstep, double time, double* dt)
   // and at the end of f_RK3SolveNavierStokes (src/pf_rk3.f90:2101-2109)
   HIPCHK(launch_dealias(c));
   if (tracers) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_tr, 0));
+  link->z_ready = link->join;
   return PDR_OK;
 }
 
@@ -951,29 +1003,41 @@ int pdr_update_b(pdr_ctx* c, int32_t tstep, double simtime) {
   return PDR_OK;
 }
 
-// g_RK3Calc (src/pg_rk3.f90:82-129)
-int pdr_step(pdr_ctx* c, int32_t tstep, double* simtime) {
-  if (!c || !simtime) return fail(PDR_ERR_ARG, "pdr_step: null argument");
+// g_RK3Calc (src/pg_rk3.f90:82-129).  Its stages are joined where one kernel can end a
+// stage and start the next (short z lines, no truncation of the state between them);
+// more: so is the next step's first stage.
+static int step_run(pdr_ctx* c, int32_t tstep, double* simtime, StageLink* link, bool more) {
   const double tstart = *simtime;
-  int rc = pdr_stage(c, 1, tstep, *simtime, &c->dt);
+  const bool zz = zz_fused(c) && c->p.dealiasing == PDR_DEALIASING_TWOTHIRD;
+  link->tstart = tstart;
+  link->join = zz;
+  int rc = stage_run(c, 1, tstep, &c->dt, link);
   if (rc != PDR_OK) return rc;
   *simtime = tstart + (1.0 / 3.0) * c->dt;
   pdr_update_b(c, tstep, *simtime);
-  rc = pdr_stage(c, 2, tstep, *simtime, &c->dt);
+  rc = stage_run(c, 2, tstep, &c->dt, link);
   if (rc != PDR_OK) return rc;
   *simtime = tstart + (3.0 / 4.0) * c->dt;
   pdr_update_b(c, tstep, *simtime);
-  rc = pdr_stage(c, 3, tstep, *simtime, &c->dt);
+  link->join = zz && more && !remesh_due(c, tstep + 1);
+  rc = stage_run(c, 3, tstep, &c->dt, link);
   if (rc != PDR_OK) return rc;
   *simtime = tstart + c->dt;
   pdr_update_b(c, tstep, *simtime);
   return PDR_OK;
 }
 
+int pdr_step(pdr_ctx* c, int32_t tstep, double* simtime) {
+  if (!c || !simtime) return fail(PDR_ERR_ARG, "pdr_step: null argument");
+  StageLink link;
+  return step_run(c, tstep, simtime, &link, false);
+}
+
 int pdr_run(pdr_ctx* c, int32_t tstep0, int32_t nsteps, double* simtime) {
   if (!c || !simtime || nsteps < 0) return fail(PDR_ERR_ARG, "pdr_run: bad argument");
+  StageLink link;
   for (int32_t s = 0; s < nsteps; ++s) {
-    int rc = pdr_step(c, tstep0 + s, simtime);
+    int rc = step_run(c, tstep0 + s, simtime, &link, s + 1 < nsteps);
     if (rc != PDR_OK) return rc;
   }
   return PDR_OK;

@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(kBlock2) k_ens_zfwd_formf(const EnsMember* __r
   switch (e.n) {
 #define PDR_EC(n)                                                                                                \
   case n:                                                                                                        \
-    k2_zfwd_formf_body<T, n, kBlock2, 0>(lb, e.g, e.cf, (const cx<T>*)e.w1, (cx<T>*)e.u[0], (cx<T>*)e.u[1],  \
+    k2_zfwd_formf_body<T, n, kBlock2, 0>(lb, e.g, e.cf, (const cx<T>*)e.w1, 1, (cx<T>*)e.u[0], (cx<T>*)e.u[1],  \
                              (cx<T>*)e.u[2], (cx<T>*)e.rk[0], (cx<T>*)e.rk[1], (cx<T>*)e.rk[2], nullptr, 0, 0.0, \
                              beta, gdt,                                                                          \
                              (const cx<T>*)e.twz, e.nt[4], T(e.norm));                                           \

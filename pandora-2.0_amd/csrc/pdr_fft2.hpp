@@ -74,6 +74,15 @@ __device__ __forceinline__ int lds_off(int o) {
   return o + (o >> lds_pad_shift<T>());
 }
 
+// A thread index that the compiler takes as new: index arithmetic made from it is
+// neither shared with earlier phases of a kernel nor moved out of a loop, where its
+// results would stay in registers (a plane of 96 points spilled 250 of them).
+__device__ __forceinline__ int fresh_tid() {
+  int t = int(threadIdx.x);
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // One radix-R Stockham pass over LINES lines of length N held in LDS (line
 // stride LD, padded layout above).  The per-element offsets o(r) = B + r*S are
 // turned into a base plus compile-time constants wherever the pad positions
@@ -86,7 +95,7 @@ __device__ __forceinline__ int lds_off(int o) {
 // read, so the caller writes zeros only to the band positions of the blocks
 // that hold stored modes as well (zero_band_edges).
 template <typename T, int N, int LINES, int LD, int R, int NS, int SIGN, bool PPT, int NT = kBlock2, int ZB = 0>
-__device__ __forceinline__ void pass_ip(cx<T>* __restrict__ buf, const cx<T>* __restrict__ tw) {
+__device__ __forceinline__ void pass_ip(cx<T>* __restrict__ buf, const cx<T>* __restrict__ tw, int tid) {
   constexpr int NBL = N / R;
   constexpr int TOTAL = NBL * LINES;
   constexpr int NB = (TOTAL + NT - 1) / NT;
@@ -96,7 +105,7 @@ __device__ __forceinline__ void pass_ip(cx<T>* __restrict__ buf, const cx<T>* __
   cx<T> v[NB][R];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const int t = int(threadIdx.x) + NT * b;
+    const int t = tid + NT * b;
     if (TOTAL % NT == 0 || t < TOTAL) {
       const int line = t / NBL;
       const int j = t - line * NBL;
@@ -118,7 +127,7 @@ __device__ __forceinline__ void pass_ip(cx<T>* __restrict__ buf, const cx<T>* __
   __syncthreads();
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const int t = int(threadIdx.x) + NT * b;
+    const int t = tid + NT * b;
     if (TOTAL % NT == 0 || t < TOTAL) {
       const int line = t / NBL;
       const int j = t - line * NBL;
@@ -156,11 +165,11 @@ __device__ __forceinline__ void pass_ip(cx<T>* __restrict__ buf, const cx<T>* __
 
 template <typename T, int N, int LINES, int LD, int SIGN, bool PPT = true, int NT = kBlock2, int ZB = 0, int P = 0,
           int NS = 1>
-__device__ __forceinline__ void fft_ip(cx<T>* __restrict__ buf, const cx<T>* __restrict__ tw) {
+__device__ __forceinline__ void fft_ip(cx<T>* __restrict__ buf, const cx<T>* __restrict__ tw, int tid = int(threadIdx.x)) {
   if constexpr (P < plan_npass(N)) {
     constexpr int R = plan_radix(N, P);
-    pass_ip<T, N, LINES, LD, R, NS, SIGN, PPT, NT, P == 0 ? ZB : 0>(buf, tw);
-    fft_ip<T, N, LINES, LD, SIGN, PPT, NT, ZB, P + 1, NS * R>(buf, tw);
+    pass_ip<T, N, LINES, LD, R, NS, SIGN, PPT, NT, P == 0 ? ZB : 0>(buf, tw, tid);
+    fft_ip<T, N, LINES, LD, SIGN, PPT, NT, ZB, P + 1, NS * R>(buf, tw, tid);
   }
 }
 
@@ -169,7 +178,7 @@ __device__ __forceinline__ void fft_ip(cx<T>* __restrict__ buf, const cx<T>* __r
 // positions each) that also hold stored modes, at most two runs per line
 // ([A, E1] and [S2, B]).  The caller synchronises before the transform.
 template <typename T, int N, int LINES, int LD, int ZB, int NT = kBlock2>
-__device__ __forceinline__ void zero_band_edges(cx<T>* __restrict__ buf) {
+__device__ __forceinline__ void zero_band_edges(cx<T>* __restrict__ buf, int tid = int(threadIdx.x)) {
   constexpr int NBL = N / plan_radix(N, 0);
   constexpr int A = ZB + 1, B = N - ZB - 1;  // the band, inclusive
   constexpr int E1 = (A % NBL == 0) ? A - 1 : ((A / NBL + 1) * NBL - 1 < B ? (A / NBL + 1) * NBL - 1 : B);
@@ -180,7 +189,7 @@ __device__ __forceinline__ void zero_band_edges(cx<T>* __restrict__ buf) {
   // 32 and 48 points) and many lines per tile, which a thread per position
   // would write one after another
   if constexpr (C > 0) {
-    for (int t = threadIdx.x; t < LINES * C; t += NT) {
+    for (int t = tid; t < LINES * C; t += NT) {
       const int line = t / C, p = t - line * C;
       buf[line * LD + lds_off<T>(p < C1 ? A + p : S2 + (p - C1))] = mk<T>(T(0), T(0));
     }
@@ -232,8 +241,9 @@ __device__ __forceinline__ void put1(T* p, T v) {
 // lanes of a butterfly wave (consecutive k) then read at stride R - 1, which is
 // odd for radix 8, 4 and 2 (no bank conflicts), where the plain table's
 // stride k r N / (NS R) puts many lanes on one bank.  The passes' tables tile
-// [0, N - 1) exactly (sum of NS (R - 1) over the passes is N - 1).
-template <typename T, int N, int NT = kBlock2, int P = 0, int NS = 1>
+// [0, N - 1) exactly (sum of NS (R - 1) over the passes is N - 1).  src may be the
+// table of a length SS N.
+template <typename T, int N, int NT = kBlock2, int SS = 1, int P = 0, int NS = 1>
 __device__ __forceinline__ void load_tw(cx<T>* __restrict__ dst, const cx<T>* __restrict__ src) {
   if constexpr (P < plan_npass(N)) {
     constexpr int R = plan_radix(N, P);
@@ -242,10 +252,10 @@ __device__ __forceinline__ void load_tw(cx<T>* __restrict__ dst, const cx<T>* __
       for (int e = threadIdx.x; e < NS * (R - 1); e += NT) {
         const int k = e / (R - 1);
         const int r = e - k * (R - 1) + 1;
-        dst[(NS - 1) + e] = src[k * r * TWS];
+        dst[(NS - 1) + e] = src[k * r * TWS * SS];
       }
     }
-    load_tw<T, N, NT, P + 1, NS * R>(dst, src);
+    load_tw<T, N, NT, SS, P + 1, NS * R>(dst, src);
   }
 }
 

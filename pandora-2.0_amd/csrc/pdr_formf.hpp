@@ -18,6 +18,7 @@ __device__ __forceinline__ double wvn_m(int k, int kmax) {
 
 // Mode (i, j, k) at element e of the wave arrays; a, b, c are its three
 // components of the nonlinear term NL (already normalised and truncated).
+// keep: the mode's new velocity for a caller that goes on with it (or null).
 // FRC: 0 leaves the forcing code out (callers without forcing arrays), so that
 // it costs the fused kernels' unforced runs no registers; 1 the isotropic
 // forcing; 2 that of the deformed isotropic form (cf.fdef).
@@ -26,10 +27,17 @@ __device__ __forceinline__ void formf_mode(const Geo& g, const Coef& cf, int i, 
                                            cx<T> b, cx<T> c, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                                            cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1,
                                            cx<T>* __restrict__ r2, const double2* __restrict__ frc, int fnk,
-                                           double fkf, double beta, double gdt) {
+                                           double fkf, double beta, double gdt, cx<T>* keep = nullptr) {
   const double kv[3] = {wvn_m(i, g.ki), wvn_m(j, g.kj), wvn_m(k, g.kk)};
   const double kmag2 = (kv[0] * kv[0]) + (kv[1] * kv[1]) + (kv[2] * kv[2]);
-  if (!(kmag2 > 0.0)) return;  // the k = 0 mode is never updated (src/pf_rk3.f90:2385)
+  if (!(kmag2 > 0.0)) {  // the k = 0 mode is never updated (src/pf_rk3.f90:2385)
+    if (keep) {
+      keep[0] = u0[e];
+      keep[1] = u1[e];
+      keep[2] = u2[e];
+    }
+    return;
+  }
   cx<T> u[3] = {u0[e], u1[e], u2[e]};
   cx<T> r[3] = {r0[e], r1[e], r2[e]};
   const bool rg = cf.form != 0;  // NS_R_ROT (f_RK3FormFRRot, src/pf_rk3.f90:2680-2856)
@@ -135,6 +143,11 @@ __device__ __forceinline__ void formf_mode(const Geo& g, const Coef& cf, int i, 
     const cx<T> kd = add(add(scl(u[0], T(kv[0])), scl(u[1], T(kv[1]))), scl(u[2], T(kv[2])));
 #pragma unroll
     for (int c = 0; c < 3; ++c) u[c] = sub(u[c], scl(kd, T(kv[c] / kmag2)));
+  }
+  if (keep) {
+    keep[0] = u[0];
+    keep[1] = u[1];
+    keep[2] = u[2];
   }
   u0[e] = u[0];
   u1[e] = u[1];

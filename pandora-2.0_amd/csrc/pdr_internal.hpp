@@ -64,6 +64,9 @@ inline int box_stretch(const pdr_params& p, int m) {
   return b > 0 ? b : 1;
 }
 
+// Most addends that the fused plane pass leaves NL in (pdr_ctx::nl_parts)
+constexpr int kNlParts = 4;
+
 // One member of a batched ensemble (pdr_ens.hip): everything a batched pass
 // kernel needs to run that member's tiles, read from device memory by the
 // workgroups whose block index falls in [start[p], start[p] + blocks[p]).
@@ -134,6 +137,7 @@ struct pdr_ctx {
   void* w2 = nullptr;  // 6 fields x m2 (x-pencil layout, zc planes of z); 9 with the specialised NS_R_CONV
   void *w1b = nullptr, *w1c = nullptr, *w2b = nullptr, *w2c = nullptr;  // NS_R_CONV on the generic kernels: du/dy, du/dz sweeps
   void* nl = nullptr;  // NL [c][i][j][k] written by pass 5 (aliases w1 fields 3..5)
+  int nl_parts = 1;    // > 1: the fused plane pass leaves NL as this many addends of three fields in w2
   int fpb_y = 6;       // fields per workgroup of the chunked inverse / forward y passes
   int fpb_yf = 3;
   void* ur = nullptr;  // real-space velocity for tracers, [z][y][x][3]
@@ -190,6 +194,7 @@ struct pdr_ctx {
   // launch shapes
   bool spec = false;  // length-specialised kernels (pdr_passes.hpp)
   const pdr::SpecOps *ops_x = nullptr, *ops_y = nullptr, *ops_z = nullptr;  // theirs for this box
+  bool plane_separate = false;  // y and x passes asked for as separate launches (PDR_ZCHUNK_MB or PDR_ZSTREAMS set)
   bool fuse_zf = true;  // fused z-forward + FormF (specialised path; PDR_FUSE_ZFORMF=0 disables)
   int tj_z = 1, ti_y = 1;
   size_t lds_max = 65536;
@@ -228,7 +233,9 @@ hipError_t launch_xpass(pdr_ctx* c, const Coef& cf, bool tracers, bool cfl, int 
 hipError_t launch_yfwd(pdr_ctx* c, int z0, int nzc);
 hipError_t launch_zfwd(pdr_ctx* c);
 hipError_t launch_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt);
-hipError_t launch_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt);
+// next: the operator of the following stage, whose inverse z pass is then done as well
+// (where zz_fused), or null
+hipError_t launch_zfwd_formf(pdr_ctx* c, const Coef& cf, const Coef* next, double beta, double gdt);
 hipError_t launch_force(pdr_ctx* c, int32_t tstep, double dt);
 // the tracer advance (interpolation, RK3 update, particle_up); wrap: also the
 // periodic correction of p_ControlFinishTimeStep (moving particle_xp0 with it)
@@ -295,11 +302,16 @@ inline size_t conv_xpass_lds(int nx, size_t csz) { return 12 * size_t(nx + 1) * 
 Coef conv_coef(const Coef& cf, int d);  // G selecting field 3 + c = d u_c / d x_d
 hipError_t launch_conv_front(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp);
 hipError_t launch_dealias(pdr_ctx* c);  // no-op for DEALIASING = 1
+bool plane_fused(const pdr_ctx* c);
+// passes 2 to 4 of every plane in one launch (where plane_fused)
+hipError_t launch_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp);
+hipError_t launch2_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp);
 hipError_t launch2_yinv_conv(pdr_ctx* c);
 hipError_t launch2_xpass_conv(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp);
 hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc);
 hipError_t launch2_zfwd(pdr_ctx* c);
-hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt);
+hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, const Coef* next, double beta, double gdt);
+bool zz_fused(const pdr_ctx* c);
 
 // records the text returned by pdr_last_error() and returns code
 int set_error(int code, const std::string& msg);

@@ -1082,6 +1082,13 @@ hipError_t launch_xpass(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, i
   return e;
 }
 
+hipError_t launch_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
+  prof_begin(c, K_XPASS);
+  hipError_t e = launch2_plane(c, cf, tr, cfl, rsp);
+  prof_end(c, K_XPASS);
+  return e;
+}
+
 template <typename T>
 static hipError_t yfwd_t(pdr_ctx* c) {
   const Geo& g = c->g;
@@ -1154,9 +1161,9 @@ hipError_t launch_force(pdr_ctx* c, int32_t tstep, double dt) {
   return hipGetLastError();
 }
 
-hipError_t launch_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
+hipError_t launch_zfwd_formf(pdr_ctx* c, const Coef& cf, const Coef* next, double beta, double gdt) {
   prof_begin(c, K_ZFF);
-  hipError_t e = launch2_zfwd_formf(c, cf, beta, gdt);
+  hipError_t e = launch2_zfwd_formf(c, cf, next, beta, gdt);
   prof_end(c, K_ZFF);
   return e;
 }

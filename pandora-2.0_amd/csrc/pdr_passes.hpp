@@ -1129,7 +1129,7 @@ __global__ void __launch_bounds__(kBlock2) PDR_FWD_WAVES
 #define PDR_ZFF_PF 1
 #endif
 template <typename T, int N, int FT = kBlock2, int FRC = 2>
-__device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ w1, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
+__device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ w1, int parts, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                   cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1, cx<T>* __restrict__ r2,
                   const double2* __restrict__ frc, int fnk, double fkf, double beta, double gdt,
                   const cx<T>* __restrict__ twg, int ntile, T norm) {
@@ -1158,6 +1158,17 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
       const int z = idx / L;
       const int line = idx - z * L;
       pre[q] = ((L * N % FT == 0 || idx < L * N) && j0 + line < nkj) ? src[z * g.ldj + line] : czero<T>();
+    }
+#pragma unroll 1
+    for (int p = 1; p < parts; ++p) {  // the plane pass left NL as this many addends
+      src += 3 * g.m1;
+#pragma unroll
+      for (int q = 0; q < QE; ++q) {
+        const int idx = int(threadIdx.x) + FT * q;
+        const int z = idx / L;
+        const int line = idx - z * L;
+        if ((L * N % FT == 0 || idx < L * N) && j0 + line < nkj) pre[q] = add(pre[q], src[z * g.ldj + line]);
+      }
     }
   };
   // FP32 lines of 256..512 points: the next field's loads are issued before
@@ -1206,11 +1217,11 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
 // FRC: 0 unforced, 1 isotropic forcing, 2 deformed isotropic forcing
 template <typename T, int N, int FRC>
 __global__ void __launch_bounds__(kBlock2) PDR_FWD_WAVES
-    k2_zfwd_formf(Geo g, Coef cf, const cx<T>* __restrict__ w1, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
+    k2_zfwd_formf(Geo g, Coef cf, const cx<T>* __restrict__ w1, int parts, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                   cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1, cx<T>* __restrict__ r2,
                   const double2* __restrict__ frc, int fnk, double fkf, double beta, double gdt,
                   const cx<T>* __restrict__ twg, int ntile, T norm) {
-  k2_zfwd_formf_body<T, N, kBlock2, FRC>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w1, u0, u1, u2, r0, r1, r2, frc,
+  k2_zfwd_formf_body<T, N, kBlock2, FRC>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w1, parts, u0, u1, u2, r0, r1, r2, frc,
                                          fnk, fkf, beta, gdt, twg, ntile, norm);
 }
 
@@ -1375,7 +1386,7 @@ hipError_t zfwd_n(pdr_ctx* c) {
 }
 
 template <typename T, int N>
-hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
+hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, const Coef*, double beta, double gdt) {
   if constexpr (N > 512) {  // not used above 512 points per line (see pdr_create)
     return hipErrorNotSupported;
   } else {
@@ -1389,8 +1400,8 @@ hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
     hipError_t e = big_lds((const void*)k2_zfwd_formf<T, N, F>, lds);
     if (e != hipSuccess) return e;
     k2_zfwd_formf<T, N, F><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
-        g, cf, (const cx<T>*)c->w1, (cx<T>*)c->u[0], (cx<T>*)c->u[1], (cx<T>*)c->u[2], (cx<T>*)c->rk[0],
-        (cx<T>*)c->rk[1], (cx<T>*)c->rk[2], F ? (const double2*)c->force : nullptr, F ? c->force_nk : 0,
+        g, cf, (const cx<T>*)(c->nl_parts > 1 ? c->w2 : c->w1), c->nl_parts, (cx<T>*)c->u[0], (cx<T>*)c->u[1],
+        (cx<T>*)c->u[2], (cx<T>*)c->rk[0], (cx<T>*)c->rk[1], (cx<T>*)c->rk[2], F ? (const double2*)c->force : nullptr, F ? c->force_nk : 0,
         F ? c->p.force_kf : 0.0, beta, gdt, (const cx<T>*)c->tab.twz, nt, T(norm));
     return hipGetLastError();
   };

@@ -2,7 +2,9 @@
 // translation unit; compiled once per PDR_SPEC_TU (build_lib.py), so that the
 // lengths build side by side.
 #include "pdr_passes.hpp"
+#include "pdr_plane.hpp"
 #include "pdr_spec.hpp"
+#include "pdr_zall.hpp"
 
 #ifndef PDR_SPEC_TU
 #define PDR_SPEC_TU 0
@@ -19,14 +21,24 @@ SpecOps ops_of() {
   SpecOps o;
   o.prec = sizeof(T) == 4 ? 1 : 0;
   o.n = N;
-  o.zinv = zinv_n<T, N>;
   o.yinv = yinv_n<T, N, false>;
   o.yinv_conv = yinv_n<T, N, true>;
   o.xpass_conv = xpass_conv_n<T, N>;
   o.xpass = xpass_n<T, N>;
   o.yfwd = yfwd_n<T, N>;
   o.zfwd = zfwd_n<T, N>;
-  o.zfwd_formf = zfwd_formf_n<T, N>;
+  o.zz = zall_lines<T>(N) > 0;
+  if constexpr (zall_lines<T>(N) > 0) {
+    o.zinv = zall_inv_n<T, N>;
+    o.zfwd_formf = zall_fwd_n<T, N>;
+  } else {
+    o.zinv = zinv_n<T, N>;
+    o.zfwd_formf = zfwd_formf_n<T, N>;
+  }
+  constexpr int parts = plane_parts_box<T>(N);
+  o.plane = parts ? plane_n<T, N> : nullptr;
+  o.plane_parts = parts;
+  o.lds_plane = parts ? size_t(plane_lds_bytes<T>(N, parts)) : 0;
   o.lds_z = lds_lines<T, N>() > lds_fwd<T, N>() ? lds_lines<T, N>() : lds_fwd<T, N>();
   o.lds_y = lds_y<T, N>();
   o.lds_x = lds_x<T, N>();
@@ -36,7 +48,7 @@ SpecOps ops_of() {
   o.x_tw_global = x_tw_global<T>(N) ? 1 : 0;
   constexpr bool reg = PDR_ZINV_REG && N <= 512;
   o.zinv_register = reg ? 1 : 0;
-  o.zinv_lines = reg ? zinv_lines_t<T, PDR_ZINV_THREADS>(N) : tile_lines<T>(N);
+  o.zinv_lines = zall_lines<T>(N) ? zall_lines<T>(N) : reg ? zinv_lines_t<T, PDR_ZINV_THREADS>(N) : tile_lines<T>(N);
   return o;
 }
 

@@ -14,7 +14,14 @@ struct SpecOps {
   hipError_t (*xpass_conv)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
   hipError_t (*yfwd)(pdr_ctx*, int z0, int nzc);
   hipError_t (*zfwd)(pdr_ctx*);
-  hipError_t (*zfwd_formf)(pdr_ctx*, const Coef&, double beta, double gdt);
+  // next: the operator of the stage that follows, whose inverse z pass is then done in the
+  // same kernel; only where zz is true, else null
+  hipError_t (*zfwd_formf)(pdr_ctx*, const Coef&, const Coef* next, double beta, double gdt);
+  bool zz;
+  // passes 2 to 4 of n x n planes in one launch (pdr_plane.hpp), null where they do not fit
+  hipError_t (*plane)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
+  size_t lds_plane;
+  int plane_parts;
   size_t lds_z, lds_y, lds_x, lds_xc;  // the largest workgroup of the z, y, x and NS_R_CONV x passes
   int xrows, xrows_conv;       // rows of an x tile
   int x_tw_global;             // 1: the x tile reads its twiddles from the global table

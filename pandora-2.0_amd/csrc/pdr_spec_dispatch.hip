@@ -36,7 +36,19 @@ void spec_forms(const pdr_ctx* c, int out[4]) {
   out[3] = c->ops_z->zinv_lines;
 }
 
+// Whether the y and x passes of a plane run as one kernel: square planes of a length
+// that has it, unless the environment asks for the chunked passes or their streams.
+bool plane_fused(const pdr_ctx* c) {
+  return c->spec && !conv_form(c) && !c->plane_separate && c->g.nx == c->g.ny && c->ops_x->plane &&
+         c->ops_x->lds_plane <= c->lds_max && c->g.zc == c->g.nz;
+}
+hipError_t launch2_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
+  return c->ops_x->plane(c, cf, tr, cfl, rsp);
+}
+
+// rows of moment partials per z plane: x-pass workgroups, or the parts of a fused plane
 int xpass_tiles(const pdr_ctx* c) {
+  if (plane_fused(c)) return c->ops_x->plane_parts;
   const int rb = conv_form(c) ? c->ops_x->xrows_conv : c->ops_x->xrows;
   return (c->g.ny + rb - 1) / rb;
 }
@@ -52,8 +64,10 @@ hipError_t launch2_xpass_conv(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, dou
 }
 hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yfwd(c, z0, nzc); }
 hipError_t launch2_zfwd(pdr_ctx* c) { return c->ops_z->zfwd(c); }
-hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
-  return c->ops_z->zfwd_formf(c, cf, beta, gdt);
+// Whether the z forward pass can go on with the next stage's z inverse
+bool zz_fused(const pdr_ctx* c) { return c->spec && !conv_form(c) && c->fuse_zf && c->ops_z->zz; }
+hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, const Coef* next, double beta, double gdt) {
+  return c->ops_z->zfwd_formf(c, cf, next, beta, gdt);
 }
 
 }  // namespace pdr

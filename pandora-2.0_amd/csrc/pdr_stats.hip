@@ -786,6 +786,9 @@ int pdr_rs_stats(pdr_ctx* ctx, pdr_rs_stats_t* out) {
   hipError_t e = hipSuccess;
   if (pdr::conv_form(c)) {
     e = pdr::launch_conv_front(c, cf, false, false, part);
+  } else if (pdr::plane_fused(c)) {
+    e = pdr::launch_zinv(c, cf);
+    if (e == hipSuccess) e = pdr::launch_plane(c, cf, false, false, part);
   } else {
     e = pdr::launch_zinv(c, cf);
     for (int z0 = 0; e == hipSuccess && z0 < g.nz; z0 += g.zc) {
