@@ -2,13 +2,15 @@
 // realisations of uneven sizes advanced together.
 //
 // A 32^3 box gives a pass a few dozen workgroups, so stepping each member on
-// its own leaves most of the 256 CUs idle and pays 15 kernel launches per step
-// per member.  Here every pass of an RK3 stage is one launch over the tiles of
-// all members (per-member work descriptors, pdr_ens_passes.hip), and the 15
-// launches of a step are captured once into a HIP graph and replayed, so a
-// step costs one graph launch for the whole ensemble.  Each member runs the
-// device bodies that pdr_step runs for it, with the same arguments; they are
-// compiled into other kernels, where the compiler may contract multiply-adds
+// its own leaves most of the 256 CUs idle and pays its kernel launches per step
+// per member.  Here every pass of an RK3 stage is one launch over all members of
+// one line length (pdr_ens_passes.hip), and the launches of their step are
+// captured once into a HIP graph and replayed.  The members of different lengths
+// have nothing to wait for in each other: each length's steps run on a stream of
+// their own, where one length's kernels fill the CUs that the last workgroups of
+// another's leave idle, and the streams meet at the end of a run.  Each member
+// runs the device bodies that pdr_step runs for it, with the same arguments; they
+// are compiled into other kernels, where the compiler may contract multiply-adds
 // differently, so the results agree with pdr_step to rounding.
 //
 // Scope: members of one precision with the specialised kernels, cubic, line
@@ -18,21 +20,34 @@
 // frames (per-stage coefficients), CFL steps (a host read of the maximum),
 // forcing (per-step draws) and tracers are rejected with PDR_ERR_UNSUPPORTED.
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <string>
 #include <vector>
 
-#include "pdr_internal.hpp"
+#include "pdr_ens_ops.hpp"
+
+namespace {
+
+// The members of one line length.
+struct EnsGroup {
+  const pdr::EnsOps* ops = nullptr;
+  int first = 0, count = 0;  // of the descriptors, which are ordered by length
+  hipStream_t stream = nullptr;
+  // one RK3 step: `joined` leaves the next step's inverse z pass done (lengths with
+  // zz, which then start a run with that pass and end it with `last`)
+  hipGraph_t joined = nullptr, last = nullptr;
+  hipGraphExec_t joined_exec = nullptr, last_exec = nullptr;
+};
+
+}  // namespace
 
 struct pdr_ensemble {
   std::vector<pdr_ctx*> m;
   int prec = 0;
   hipStream_t stream = nullptr;
   pdr::EnsMember* d_mem = nullptr;
-  unsigned nblk[5] = {0, 0, 0, 0, 0};
-  size_t lds[5] = {0, 0, 0, 0, 0};
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  std::vector<EnsGroup> groups;
   int fpb_y = 0, fpb_yf = 0;  // 0: each member's own choice
 };
 
@@ -44,37 +59,57 @@ const double kBeta[3] = {0.0, -5.0 / 9.0, -153.0 / 128.0};
 const double kGamma[3] = {1.0 / 3.0, 15.0 / 16.0, 8.0 / 15.0};
 
 void ens_release(pdr_ensemble* e) {
-  if (e->exec) (void)hipGraphExecDestroy(e->exec);
-  if (e->graph) (void)hipGraphDestroy(e->graph);
-  e->exec = nullptr;
-  e->graph = nullptr;
+  for (EnsGroup& q : e->groups) {
+    if (q.stream) (void)hipStreamSynchronize(q.stream);
+    for (hipGraphExec_t x : {q.joined_exec, q.last_exec})
+      if (x) (void)hipGraphExecDestroy(x);
+    for (hipGraph_t x : {q.joined, q.last})
+      if (x) (void)hipGraphDestroy(x);
+    if (q.stream) (void)hipStreamDestroy(q.stream);
+  }
+  e->groups.clear();
+}
+
+// Captures one RK3 step of a group: 3 stages of the inverse z pass (where the stage
+// before has not done it), the passes of the planes and the z forward + FormF.
+hipError_t ens_capture(pdr_ensemble* e, EnsGroup& q, int fpb_y, int fpb_yf, bool joined, hipGraph_t* graph,
+                       hipGraphExec_t* exec) {
+  const pdr::EnsMember* mem = e->d_mem + q.first;
+  hipError_t r = hipStreamBeginCapture(q.stream, hipStreamCaptureModeThreadLocal);
+  if (r != hipSuccess) return r;
+  hipError_t lr = hipSuccess;
+  for (int st = 0; st < 3 && lr == hipSuccess; ++st) {
+    if (!q.ops->zz) lr = q.ops->zinv(mem, q.count, q.stream);
+    if (lr == hipSuccess) lr = q.ops->mid(mem, q.count, fpb_y, fpb_yf, q.stream);
+    if (lr == hipSuccess)
+      lr = q.ops->zend(mem, q.count, kBeta[st], kGamma[st], q.ops->zz && (joined || st < 2), q.stream);
+  }
+  r = hipStreamEndCapture(q.stream, graph);
+  if (lr != hipSuccess) return lr;
+  if (r != hipSuccess) return r;
+  return hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
 }
 
 int ens_build(pdr_ensemble* e) {
   ens_release(e);
   const int nm = int(e->m.size());
+  std::vector<pdr_ctx*> order = e->m;
+  std::stable_sort(order.begin(), order.end(), [](const pdr_ctx* a, const pdr_ctx* b) { return a->g.nx < b->g.nx; });
   std::vector<pdr::EnsMember> h(static_cast<size_t>(nm));
-  for (int q = 0; q < 5; ++q) {
-    e->nblk[q] = 0;
-    e->lds[q] = 0;
-  }
   for (int k = 0; k < nm; ++k) {
-    pdr_ctx* c = e->m[size_t(k)];
+    pdr_ctx* c = order[size_t(k)];
+    if (k == 0 || c->g.nx != order[size_t(k - 1)]->g.nx) {
+      EnsGroup q;
+      q.ops = pdr::ens_ops(c->prec, c->g.nx);
+      q.first = k;
+      if (!q.ops) return set_error(PDR_ERR_UNSUPPORTED, "ensemble: unsupported line length");
+      e->groups.push_back(q);
+    }
+    ++e->groups.back().count;
     pdr::EnsMember& d = h[size_t(k)];
     std::memset(&d, 0, sizeof(d));
     d.g = c->g;
     d.cf = pdr::make_coef(c);
-    d.n = c->g.nx;
-    d.fpb_y = e->fpb_y ? e->fpb_y : c->fpb_y;
-    d.fpb_yf = e->fpb_yf ? e->fpb_yf : c->fpb_yf;
-    unsigned blocks[5];
-    if (pdr::ens_tiles(c->prec, d.n, c->g, d.fpb_y, d.fpb_yf, d.nt, blocks) != 0)
-      return set_error(PDR_ERR_UNSUPPORTED, "ensemble: unsupported line length");
-    for (int q = 0; q < 5; ++q) {
-      d.start[q] = e->nblk[q];
-      e->nblk[q] += blocks[q];
-      e->lds[q] = std::max(e->lds[q], pdr::ens_lds(c->prec, d.n, q));
-    }
     d.dt = c->p.rk3_dt;
     d.norm = 1.0 / (double(c->g.nx) * double(c->g.ny) * double(c->g.nz));
     for (int q = 0; q < 3; ++q) {
@@ -93,28 +128,37 @@ int ens_build(pdr_ensemble* e) {
     e->d_mem = nullptr;
     return set_error(PDR_ERR_NOMEM, "ensemble: device allocation failed");
   }
-  size_t lmax = 0;
-  for (int q = 0; q < 5; ++q) lmax = std::max(lmax, e->lds[q]);
-  hipError_t r = pdr::ens_prepare(e->prec, lmax);
-  if (r == hipSuccess)
-    r = hipMemcpy(e->d_mem, h.data(), sizeof(pdr::EnsMember) * size_t(nm), hipMemcpyHostToDevice);
-  // capture one RK3 step: 3 stages x 5 batched passes
-  if (r == hipSuccess) r = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal);
-  if (r == hipSuccess) {
-    hipError_t lr = hipSuccess;
-    for (int st = 0; st < 3 && lr == hipSuccess; ++st)
-      for (int q = 0; q < 5 && lr == hipSuccess; ++q)
-        lr = pdr::launch_ens_pass(e->prec, q, e->d_mem, nm, e->nblk[q], e->lds[q], kBeta[st], kGamma[st],
-                                  e->stream);
-    r = hipStreamEndCapture(e->stream, &e->graph);
-    if (lr != hipSuccess) r = lr;
+  hipError_t r = hipMemcpy(e->d_mem, h.data(), sizeof(pdr::EnsMember) * size_t(nm), hipMemcpyHostToDevice);
+  for (EnsGroup& q : e->groups) {
+    const pdr_ctx* c = order[size_t(q.first)];
+    const int fy = e->fpb_y ? e->fpb_y : c->fpb_y, fyf = e->fpb_yf ? e->fpb_yf : c->fpb_yf;
+    if (r == hipSuccess) r = q.ops->prepare();
+    if (r == hipSuccess) r = hipStreamCreateWithFlags(&q.stream, hipStreamNonBlocking);
+    if (r == hipSuccess) r = ens_capture(e, q, fy, fyf, false, &q.last, &q.last_exec);
+    if (r == hipSuccess && q.ops->zz) r = ens_capture(e, q, fy, fyf, true, &q.joined, &q.joined_exec);
   }
-  if (r == hipSuccess) r = hipGraphInstantiate(&e->exec, e->graph, nullptr, nullptr, 0);
   if (r != hipSuccess) {
+    (void)hipGetLastError();
     ens_release(e);
     return set_error(PDR_ERR_HIP, std::string("ensemble set-up: ") + hipGetErrorString(r));
   }
   return PDR_OK;
+}
+
+// Queues nsteps steps of every group and waits for them.  The groups take turns, so
+// that each has work queued while the others run.
+hipError_t ens_steps(pdr_ensemble* e, int nsteps) {
+  hipError_t r = hipSuccess;
+  for (EnsGroup& q : e->groups)
+    if (r == hipSuccess && nsteps > 0 && q.ops->zz) r = q.ops->zinv(e->d_mem + q.first, q.count, q.stream);
+  for (int s = 0; s < nsteps && r == hipSuccess; ++s)
+    for (EnsGroup& q : e->groups)
+      if (r == hipSuccess) r = hipGraphLaunch(q.ops->zz && s + 1 < nsteps ? q.joined_exec : q.last_exec, q.stream);
+  for (EnsGroup& q : e->groups) {
+    const hipError_t w = hipStreamSynchronize(q.stream);
+    if (r == hipSuccess) r = w;
+  }
+  return r;
 }
 
 }  // namespace
@@ -131,7 +175,7 @@ int pdr_ensemble_create(pdr_ensemble** out, pdr_ctx* const* members, int32_t cou
     for (int32_t q = 0; q < k; ++q)
       if (members[q] == c) return set_error(PDR_ERR_ARG, "pdr_ensemble_create: member listed twice");
     const bool ok = c->prec == prec && c->spec && c->fuse_zf && c->g.zc == c->g.nz && c->g.nx == c->g.ny &&
-                    c->g.ny == c->g.nz && pdr::ens_size_supported(c->g.nx) &&
+                    c->g.ny == c->g.nz && pdr::ens_ops(prec, c->g.nx) &&
                     c->p.f_type == PDR_F_ISOTROPIC && c->p.rk3_timestep == PDR_RK3_TIMESTEP_FIXED &&
                     !c->forcing && c->np == 0 && c->p.dealiasing == PDR_DEALIASING_TWOTHIRD;
     if (!ok)
@@ -161,7 +205,6 @@ int pdr_ensemble_set_split(pdr_ensemble* e, int32_t fpb_y, int32_t fpb_yf) {
   const bool ok = (fpb_y == 0 || fpb_y == 1 || fpb_y == 2 || fpb_y == 3 || fpb_y == 6) &&
                   (fpb_yf == 0 || fpb_yf == 1 || fpb_yf == 3);
   if (!ok) return set_error(PDR_ERR_ARG, "pdr_ensemble_set_split: fields per workgroup must divide 6 / 3");
-  (void)hipStreamSynchronize(e->stream);
   e->fpb_y = fpb_y;
   e->fpb_yf = fpb_yf;
   return ens_build(e);
@@ -201,35 +244,29 @@ int pdr_ensemble_autotune(pdr_ensemble* e, int32_t steps, int32_t* best_y, int32
     return r;
   };
   hipError_t r = copy_state(true);
-  hipEvent_t a = nullptr, b = nullptr;
-  if (r == hipSuccess) r = hipEventCreate(&a);
-  if (r == hipSuccess) r = hipEventCreate(&b);
   const int ys[4] = {1, 2, 3, 6}, yfs[2] = {1, 3};
-  float best = 1e30f;
-  int by = e->fpb_y, byf = e->fpb_yf;
+  double best = 1e30;
+  int by = e->fpb_y ? e->fpb_y : 6, byf = e->fpb_yf ? e->fpb_yf : 3;
+  bool split = false;  // nothing to tune where every member's planes run as one kernel
+  for (const EnsGroup& q : e->groups) split = split || q.ops->split;
   int rc = PDR_OK;
-  for (int iy = 0; iy < 4 && r == hipSuccess && rc == PDR_OK; ++iy)
+  for (int iy = 0; iy < 4 && split && r == hipSuccess && rc == PDR_OK; ++iy)
     for (int iyf = 0; iyf < 2 && r == hipSuccess && rc == PDR_OK; ++iyf) {
       e->fpb_y = ys[iy];
       e->fpb_yf = yfs[iyf];
       rc = ens_build(e);
       if (rc != PDR_OK) break;
-      r = hipGraphLaunch(e->exec, e->stream);  // warm-up
-      if (r == hipSuccess) r = hipEventRecord(a, e->stream);
-      for (int32_t s = 0; s < steps && r == hipSuccess; ++s) r = hipGraphLaunch(e->exec, e->stream);
-      if (r == hipSuccess) r = hipEventRecord(b, e->stream);
-      if (r == hipSuccess) r = hipEventSynchronize(b);
-      float ms = 0.0f;
-      if (r == hipSuccess) r = hipEventElapsedTime(&ms, a, b);
-      if (r == hipSuccess && ms < best) {
-        best = ms;
+      r = ens_steps(e, 1);  // warm-up
+      const auto t0 = std::chrono::steady_clock::now();
+      if (r == hipSuccess) r = ens_steps(e, steps);
+      const double s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+      if (r == hipSuccess && s < best) {
+        best = s;
         by = ys[iy];
         byf = yfs[iyf];
       }
     }
   if (r == hipSuccess) r = copy_state(false);
-  if (a) (void)hipEventDestroy(a);
-  if (b) (void)hipEventDestroy(b);
   (void)hipFree(save);
   if (rc != PDR_OK) return rc;
   if (r != hipSuccess) return set_error(PDR_ERR_HIP, std::string("pdr_ensemble_autotune: ") + hipGetErrorString(r));
@@ -246,17 +283,15 @@ int pdr_ensemble_run(pdr_ensemble* e, int32_t tstep0, int32_t nsteps, double* si
   for (pdr_ctx* c : e->m)  // work queued on the members' own streams comes first
     if (hipStreamSynchronize(c->stream) != hipSuccess)
       return set_error(PDR_ERR_HIP, "pdr_ensemble_run: member stream failed");
-  for (int32_t s = 0; s < nsteps; ++s) {
-    hipError_t r = hipGraphLaunch(e->exec, e->stream);
-    if (r != hipSuccess) return set_error(PDR_ERR_HIP, std::string("pdr_ensemble_run: ") + hipGetErrorString(r));
+  const hipError_t r = ens_steps(e, nsteps);
+  if (r != hipSuccess) return set_error(PDR_ERR_HIP, std::string("pdr_ensemble_run: ") + hipGetErrorString(r));
+  for (int32_t s = 0; s < nsteps; ++s)
     // g_RK3Calc: simtime = t + dt after the third stage (src/pg_rk3.f90:82-129)
     for (size_t k = 0; k < e->m.size(); ++k) {
       pdr_ctx* c = e->m[k];
       c->dt = c->p.rk3_dt;
       simtime[k] = simtime[k] + c->dt;
     }
-  }
-  if (hipStreamSynchronize(e->stream) != hipSuccess) return set_error(PDR_ERR_HIP, "pdr_ensemble_run: step failed");
   return PDR_OK;
 }
 

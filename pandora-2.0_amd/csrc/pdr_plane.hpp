@@ -39,12 +39,12 @@ constexpr int plane_lds_bytes(int n, int s) {
 constexpr int kPlaneLds = 158 * 1024;  // leaves the static arrays of the reductions
 // The longest planes taken this way, and the parts a plane is taken in (0: the
 // separate passes run): the fewest, at least `least`, whose tile fits.
-template <typename T>
+template <typename T, bool ENS = false>
 constexpr int plane_parts(int n, int least) {
-  if (n > PDR_PLANE_MAX) return 0;
+  if (!ENS && n > PDR_PLANE_MAX) return 0;
   for (int s = least; 8 * s <= n + 7; ++s)
     if (n % s == 0 && plane_lds_bytes<T>(n, s) <= kPlaneLds) return s;
-  return least > 1 ? plane_parts<T>(n, 1) : 0;
+  return least > 1 ? plane_parts<T, ENS>(n, 1) : 0;
 }
 // Parts of a single box's planes: enough for the groups below to fill the chip
 // where the planes alone do not.
@@ -323,7 +323,7 @@ __device__ __forceinline__ void plane_body(int z, int gr, int ng, const Geo& g, 
     const int e = tid + NT * q;
     if ((3 * NKI * NKJ) % NT == 0 || e < 3 * NKI * NKJ) {
       const int line = e / NKJ, f = line / NKI;
-      put<kNtYfwd>(reinterpret_cast<cx<T>*>(dz + at(f, line - f * NKI, e - line * NKJ)), out[q]);
+      put<kNtYfwd && !small_store(N)>(reinterpret_cast<cx<T>*>(dz + at(f, line - f * NKI, e - line * NKJ)), out[q]);
     }
   }
   if (want_cfl) {

@@ -170,7 +170,7 @@ __device__ __forceinline__ void zall_body(unsigned bid, const Geo& g, const Coef
       const int e = int(threadIdx.x) + NT * q;
       const int line = e % L, z = (e / L) % N, f = e / (L * N);
       if ((E % NT == 0 || e < E) && line < lines)
-        put<kNtZinv>(&dst[(long long)f * g.m1 + z * g.ldj + line], buf[(f * L + line) * LD + lds_off<T>(z)]);
+        put<kNtZinv && !small_store(N)>(&dst[(long long)f * g.m1 + z * g.ldj + line], buf[(f * L + line) * LD + lds_off<T>(z)]);
     }
   }
 }
