@@ -29,7 +29,7 @@ SPEC_TUS = 8  # kSpecTus of pdr_spec.hpp: pdr_spec.hip is compiled once for each
 # (source, extra defines, object); the costliest first
 SOURCES = [("pdr_ens_passes.hip", [], "pdr_ens_passes.o")]
 SOURCES += [("pdr_spec.hip", [f"-DPDR_SPEC_TU={k}"], f"pdr_spec_{k}.o") for k in range(SPEC_TUS)]
-SOURCES += [(f"{s}.hip", [], f"{s}.o") for s in ("pdr_api", "pdr_kernels", "pdr_spec_dispatch", "pdr_host", "pdr_stats",
+SOURCES += [(f"{s}.hip", [], f"{s}.o") for s in ("pdr_api", "pdr_kernels", "pdr_spec_dispatch", "pdr_host", "pdr_xfer", "pdr_stats",
                                                  "pdr_pstats", "pdr_sort", "pdr_ens")]
 
 

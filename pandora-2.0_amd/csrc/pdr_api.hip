@@ -317,6 +317,7 @@ int pdr_destroy(pdr_ctx* c) {
   if (c->xp0) (void)hipFree(c->xp0);
   if (c->pid) (void)hipFree(c->pid);
   particles_free_sort(c);
+  xfer_free(c);
   if (c->pst_buf) (void)hipFree(c->pst_buf);
   if (c->umax) (void)hipFree(c->umax);
   if (c->red) (void)hipFree(c->red);
@@ -593,67 +594,34 @@ int pdr_kernel_forms(const pdr_ctx* c, int32_t out[8]) {
   return PDR_OK;
 }
 
-static int put_field(pdr_ctx* c, void* dst, const double* src, long long n) {
-  if (!src) return fail(PDR_ERR_ARG, "null host array");
-  if (c->prec == PDR_FP64) {
-    HIPCHK(hipMemcpy(dst, src, size_t(n) * sizeof(double), hipMemcpyHostToDevice));
-  } else {
-    std::vector<float> tmp(static_cast<size_t>(n));
-    for (long long q = 0; q < n; ++q) tmp[size_t(q)] = float(src[q]);
-    HIPCHK(hipMemcpy(dst, tmp.data(), size_t(n) * sizeof(float), hipMemcpyHostToDevice));
-  }
-  return PDR_OK;
+// three wave fields to or from the host
+static int put_fields(pdr_ctx* c, void* const dst[3], const double* a, const double* b, const double* d) {
+  const double* h[3] = {a, b, d};
+  return xfer_from_host(c, 3, dst, h, 2 * c->g.mw, c->prec != PDR_FP64);
 }
-
-static int get_field(pdr_ctx* c, double* dst, const void* src, long long n) {
-  if (!dst) return fail(PDR_ERR_ARG, "null host array");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  if (c->prec == PDR_FP64) {
-    HIPCHK(hipMemcpy(dst, src, size_t(n) * sizeof(double), hipMemcpyDeviceToHost));
-  } else {
-    std::vector<float> tmp(static_cast<size_t>(n));
-    HIPCHK(hipMemcpy(tmp.data(), src, size_t(n) * sizeof(float), hipMemcpyDeviceToHost));
-    for (long long q = 0; q < n; ++q) dst[q] = double(tmp[size_t(q)]);
-  }
-  return PDR_OK;
+static int get_fields(pdr_ctx* c, double* a, double* b, double* d, void* const src[3]) {
+  double* h[3] = {a, b, d};
+  return xfer_to_host(c, 3, src, h, 2 * c->g.mw, c->prec != PDR_FP64);
 }
 
 int pdr_upload_state(pdr_ctx* c, const double* a, const double* b, const double* d) {
   if (!c) return fail(PDR_ERR_ARG, "null context");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  const long long n = 2 * c->g.mw;
-  int rc = put_field(c, c->u[0], a, n);
-  if (rc == PDR_OK) rc = put_field(c, c->u[1], b, n);
-  if (rc == PDR_OK) rc = put_field(c, c->u[2], d, n);
-  return rc;
+  return put_fields(c, c->u, a, b, d);
 }
 
 int pdr_download_state(pdr_ctx* c, double* a, double* b, double* d) {
   if (!c) return fail(PDR_ERR_ARG, "null context");
-  const long long n = 2 * c->g.mw;
-  int rc = get_field(c, a, c->u[0], n);
-  if (rc == PDR_OK) rc = get_field(c, b, c->u[1], n);
-  if (rc == PDR_OK) rc = get_field(c, d, c->u[2], n);
-  return rc;
+  return get_fields(c, a, b, d, c->u);
 }
 
 int pdr_upload_rk3(pdr_ctx* c, const double* a, const double* b, const double* d) {
   if (!c) return fail(PDR_ERR_ARG, "null context");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  const long long n = 2 * c->g.mw;
-  int rc = put_field(c, c->rk[0], a, n);
-  if (rc == PDR_OK) rc = put_field(c, c->rk[1], b, n);
-  if (rc == PDR_OK) rc = put_field(c, c->rk[2], d, n);
-  return rc;
+  return put_fields(c, c->rk, a, b, d);
 }
 
 int pdr_download_rk3(pdr_ctx* c, double* a, double* b, double* d) {
   if (!c) return fail(PDR_ERR_ARG, "null context");
-  const long long n = 2 * c->g.mw;
-  int rc = get_field(c, a, c->rk[0], n);
-  if (rc == PDR_OK) rc = get_field(c, b, c->rk[1], n);
-  if (rc == PDR_OK) rc = get_field(c, d, c->rk[2], n);
-  return rc;
+  return get_fields(c, a, b, d, c->rk);
 }
 
 int pdr_set_frame(pdr_ctx* c, const double bmat[9], const double binv[9]) {
@@ -1174,7 +1142,9 @@ int pdr_debug_prepare(pdr_ctx* c, int32_t field, double* out) {
   const Geo& g = c->g;
   const size_t off = size_t(field) * size_t(g.m1) * c->csz;
   std::vector<double> pad(size_t(2 * g.m1));
-  int rc = get_field(c, pad.data(), (const char*)c->w1 + off, 2 * g.m1);
+  const void* src = (const char*)c->w1 + off;
+  double* dst = pad.data();
+  int rc = xfer_to_host(c, 1, &src, &dst, 2 * g.m1, c->prec != PDR_FP64);
   if (rc != PDR_OK) return rc;
   // drop the padding of the j stride: (0:1, 0:NKJ-1, 0:NZ-1, 0:NKI-1)
   for (long long line = 0; line < (long long)g.nki * g.nz; ++line)

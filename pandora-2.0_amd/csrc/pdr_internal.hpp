@@ -209,6 +209,9 @@ struct pdr_ctx {
   hipStream_t zstream = nullptr;
   void* w2z = nullptr;
   hipEvent_t ev_za = nullptr, ev_zb = nullptr;
+  void* stage = nullptr;  // pinned memory of the host transfers (pdr_xfer.hip), grown on use
+  size_t stage_bytes = 0;
+  long long small_downloads = 0;
   size_t dev_bytes = 0;
   // profiling
   bool prof = false;
@@ -239,6 +242,11 @@ hipError_t launch_tracers(pdr_ctx* c, const TracerFrame& tf, double beta, double
 hipError_t launch_tracers_wrap(pdr_ctx* c, const TracerFrame& tf, hipStream_t s);
 hipError_t launch_remesh(pdr_ctx* c, int bfrot);
 hipError_t launch_remesh_particles(pdr_ctx* c, double lx, double dx);
+// host transfers (pdr_xfer.hip): `fields` (1..3) arrays of n reals each, FP64 on the host,
+// FP32 on the device where f32; in stream order, done on return
+int xfer_to_host(pdr_ctx* c, int fields, const void* const* dev, double* const* host, long long n, bool f32);
+int xfer_from_host(pdr_ctx* c, int fields, void* const* dev, const double* const* host, long long n, bool f32);
+void xfer_free(pdr_ctx* c);
 // tracer order (pdr_sort.hip)
 int particles_sort(pdr_ctx* c);
 int particles_to_host(pdr_ctx* c, const double* dev, double* host);

@@ -144,21 +144,24 @@ int particles_sort(pdr_ctx* c) {
   return PDR_OK;
 }
 
-// dev (3, np) in slot order -> host (3, np) in the caller's numbering
+// slot order to the caller's numbering, three words a tracer
+__global__ void __launch_bounds__(256)
+    k_unsort3(const double* __restrict__ src, double* __restrict__ dst, const uint32_t* __restrict__ pid, long long n) {
+  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < 3 * n) dst[3 * (long long)pid[e / 3] + e % 3] = src[e];
+}
+
+// dev (3, np) in slot order -> host (3, np) in the caller's numbering: put in order on
+// the device, in the sort's spare array (unsorted slots have the caller's order)
 int particles_to_host(pdr_ctx* c, const double* dev, double* host) {
-  const size_t n = size_t(c->np);
-  std::vector<double> tmp(3 * n);
-  std::vector<uint32_t> pid(n);
-  hipError_t e = hipMemcpy(tmp.data(), dev, 24 * n, hipMemcpyDeviceToHost);
-  if (e == hipSuccess) e = hipMemcpy(pid.data(), c->pid, 4 * n, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return set_error(PDR_ERR_HIP, std::string("particle download: ") + hipGetErrorString(e));
-  for (size_t s = 0; s < n; ++s) {
-    const size_t o = pid[s];
-    host[3 * o] = tmp[3 * s];
-    host[3 * o + 1] = tmp[3 * s + 1];
-    host[3 * o + 2] = tmp[3 * s + 2];
+  const double* src = dev;
+  if (c->spare) {
+    k_unsort3<<<dim3(unsigned((3 * c->np + 255) / 256)), 256, 0, c->stream>>>(dev, c->spare, c->pid, c->np);
+    if (hipGetLastError() != hipSuccess) return set_error(PDR_ERR_HIP, "particle download: launch failed");
+    src = c->spare;
   }
-  return PDR_OK;
+  const void* d = src;
+  return xfer_to_host(c, 1, &d, &host, 3 * (long long)c->np, false);
 }
 
 // host (3, np) in the caller's numbering -> dev in slot order
