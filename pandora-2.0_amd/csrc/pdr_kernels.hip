@@ -471,7 +471,10 @@ __global__ void __launch_bounds__(kThreads)
 
 // ---------------------------------------------------------------------------
 // Ornstein-Uhlenbeck forcing update, f_ForceCalc (src/pf_force.f90:106-268).
-// F is [i][j+NK][k+NK][c] complex, i = 0..NK, j, k = -NK..NK.  Thread t < (NK+1)^2
+// F is [i][j+NK][k+NK][c] complex, i = 0..NK, j, k = -NK..NK.  A thread takes one component
+// of an iteration t = thread / 3, since a normal pair, with its rejections, is a chain of a
+// microsecond or two: at NK = 2 the launch takes 6 us, where one thread
+// to an iteration's three components took 14.5, all of them between two passes.  Iteration t < (NK+1)^2
 // runs one (j, k) iteration of the i = 0 loop (j, k = 0..NK) with its
 // conjugate-symmetric copies, in the reference's statement order (for k = 0
 // the (0, -j, 0) update reads the copy just written, as there); the other
@@ -482,35 +485,29 @@ __global__ void __launch_bounds__(kThreads)
 __global__ void __launch_bounds__(kThreads)
     k_force_ou(double2* __restrict__ F, int nk, double om, double sd, unsigned long long seed,
                unsigned long long call) {
-  const int t = int(blockIdx.x * blockDim.x + threadIdx.x);
+  const int e = int(blockIdx.x * blockDim.x + threadIdx.x);
+  const int t = e / 3, c = e - 3 * t;
   const int w = 2 * nk + 1;
   const int n0 = (nk + 1) * (nk + 1);
   const int n1 = nk * w * w;
   if (t >= n0 + n1) return;
-  auto at = [&](int i, int j, int k) { return F + ((i * w + j + nk) * w + k + nk) * 3; };
+  auto at = [&](int i, int j, int k) { return F + ((i * w + j + nk) * w + k + nk) * 3 + c; };
   auto ou = [&](double2* p, unsigned long long key) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      double re, im;
-      pdr::normal_pair(seed, key + unsigned(c), &re, &im);
-      p[c].x = p[c].x * om + re * sd;
-      p[c].y = p[c].y * om + im * sd;
-    }
+    double re, im;
+    pdr::normal_pair(seed, key + unsigned(c), &re, &im);
+    p->x = p->x * om + re * sd;
+    p->y = p->y * om + im * sd;
   };
   const unsigned long long key0 = call << 24;
   if (t < n0) {
     const int j = t / (nk + 1), k = t - (t / (nk + 1)) * (nk + 1);
     double2* p = at(0, j, k);
     ou(p, key0 + 6ull * unsigned(t));
-    double2* m = at(0, -j, -k);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) m[c] = make_double2(p[c].x, -p[c].y);
+    *at(0, -j, -k) = make_double2(p->x, -p->y);
     if (j > 0) {
       double2* q = at(0, -j, k);
       ou(q, key0 + 6ull * unsigned(t) + 3ull);
-      double2* r = at(0, j, -k);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) r[c] = make_double2(q[c].x, -q[c].y);
+      *at(0, j, -k) = make_double2(q->x, -q->y);
     }
   } else {
     const int u = t - n0;
@@ -1151,8 +1148,9 @@ hipError_t launch_force(pdr_ctx* c, int32_t tstep, double dt) {
   } else {
     const double a = dt / c->p.force_tf;  // dt_over_TF
     const double sd = sqrt(2.0 * (c->p.force_sigma * c->p.force_sigma) * a);
-    const int nt = (nk + 1) * (nk + 1) + nk * w * w;
-    k_force_ou<<<dim3(unsigned((nt + kThreads - 1) / kThreads)), kThreads, 0, c->stream>>>(
+    const int nt = 3 * ((nk + 1) * (nk + 1) + nk * w * w);
+    constexpr int kForceThreads = 64;  // few threads: a wave each to its own CU
+    k_force_ou<<<dim3(unsigned((nt + kForceThreads - 1) / kForceThreads)), kForceThreads, 0, c->stream>>>(
         (double2*)c->force, nk, 1.0 - a, sd, (unsigned long long)c->p.force_seed,
         (unsigned long long)c->force_calls);
     ++c->force_calls;

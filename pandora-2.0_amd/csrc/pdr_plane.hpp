@@ -338,7 +338,7 @@ __device__ __forceinline__ void plane_body(int z, int gr, int ng, const Geo& g, 
     if (tid == 0) {
       T r = red[0];
       for (int w = 1; w < NT / 64; ++w) r = red[w] > r ? red[w] : r;
-      atomicMax(umax, (unsigned long long)__double_as_longlong(double(r)));
+      raise_max(umax, (unsigned long long)__double_as_longlong(double(r)));
     }
   }
 }
