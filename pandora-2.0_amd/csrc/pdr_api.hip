@@ -743,7 +743,8 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
   if (pstats) HIPCHK(launch_pstats_primary(c, *dt));
   // spherical / LES truncation on entry to f_RK3PrepareRealSpace (src/pf_rk3.f90:269-277)
   HIPCHK(launch_dealias(c));
-  const Coef cf = make_coef(c);
+  Coef cf = make_coef(c);
+  cf.y3 = z5_fields(c, cf) ? 1 : 0;
   // particles move from tstep = P_TS_RELEASE on (src/pf_rk3.f90:1146): the x pass
   // writes their field, and the stage advances them unless the caller does
   const bool field = c->np > 0 && tstep >= c->ts_release;
@@ -779,7 +780,7 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
         std::swap(c->stream, c->zstream);
         std::swap(c->w2, c->w2z);
       }
-      he = launch_yinv(c, z0, nzc);
+      he = launch_yinv(c, cf, z0, nzc);
       if (he == hipSuccess) he = launch_xpass(c, cf, field, need_cfl, z0, nzc, rsp);
       if (he == hipSuccess) he = launch_yfwd(c, z0, nzc);
       if (alt) {

@@ -56,6 +56,7 @@ struct Coef {
   int fdiv[3];   // projected along the laboratory wavenumber fbm[m] k_m (1 and 1.0
   double fbm[3]; // for the isotropic form); finv = 1 / fdiv
   double finv[3];
+  int y3;        // 1: the z pass leaves the last vorticity component to the y pass (z5_fields)
 };
 
 // B110, B220, B330 (m = 1, 2, 3); values <= 0 stand for the reference default 1
@@ -225,7 +226,7 @@ namespace pdr {
 
 // launchers (pdr_kernels.hip); return hipSuccess or the launch error
 hipError_t launch_zinv(pdr_ctx* c, const Coef& cf);
-hipError_t launch_yinv(pdr_ctx* c, int z0, int nzc);
+hipError_t launch_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc);
 hipError_t launch_xpass(pdr_ctx* c, const Coef& cf, bool tracers, bool cfl, int z0, int nzc,
                         double* rsp = nullptr);
 hipError_t launch_yfwd(pdr_ctx* c, int z0, int nzc);
@@ -281,7 +282,8 @@ void fft_plan(FftPlan* p, int n);
 bool spec_find(pdr_ctx* c);
 void spec_forms(const pdr_ctx* c, int out[4]);
 hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf);
-hipError_t launch2_yinv(pdr_ctx* c, int z0, int nzc);
+hipError_t launch2_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc);
+bool z5_fields(const pdr_ctx* c, const Coef& cf);
 hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tracers, bool cfl, int z0, int nzc, double* rsp);
 int xpass_tiles(const pdr_ctx* c);  // x-pass workgroups per z plane (specialised path)
 Coef make_coef(const pdr_ctx* c);

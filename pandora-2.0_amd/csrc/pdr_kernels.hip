@@ -992,9 +992,9 @@ static hipError_t yinv_t(pdr_ctx* c, const void* w1, void* w2) {
 
 // The generic y/x kernels work on the whole box (the buffer is not chunked
 // for them: zc = NZ); the specialised ones take a chunk of z planes.
-hipError_t launch_yinv(pdr_ctx* c, int z0, int nzc) {
+hipError_t launch_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc) {
   prof_begin(c, K_YINV);
-  hipError_t e = c->spec   ? launch2_yinv(c, z0, nzc)
+  hipError_t e = c->spec   ? launch2_yinv(c, cf, z0, nzc)
                  : c->prec ? yinv_t<float>(c, c->w1, c->w2)
                            : yinv_t<double>(c, c->w1, c->w2);
   prof_end(c, K_YINV);

@@ -278,7 +278,8 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
       }
     }
   };
-  for (int f = 0; f < 6; ++f) {
+  const int nf = cf.y3 ? 5 : 6;  // y3: the inverse y pass forms the last vorticity component
+  for (int f = 0; f < nf; ++f) {
     if (f < 3) {
       load_u(f);
 #pragma unroll
@@ -302,6 +303,14 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
     }
     __syncthreads();
   }
+}
+
+// The thread index of a phase of the z passes: formed anew (fresh_tid) from 256 points up,
+// where the indices of all phases would take registers that a second (zinv) or third (zff)
+// workgroup needs; shorter lines have the registers (128^3 FP64 is 3 us a launch faster so).
+template <int N>
+__device__ __forceinline__ int phase_tid() {
+  return N >= 256 ? fresh_tid() : int(threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -345,8 +354,14 @@ template <typename T, int ZT>
 constexpr int lds_zinv_bytes_t(int n) {
   return (n + zinv_lines_t<T, ZT>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
 }
-#define PDR_ZINV_WAVES_T \
-  __attribute__((amdgpu_waves_per_eu(PDR_ZINV_THREADS > kBlock2 ? PDR_ZINV_THREADS / kBlock2 : waves_for(lds_zinv_bytes<T>(N)))))
+// waves per SIMD declared to the register allocator: two workgroups per CU where the LDS admits
+// them: their indices formed anew in each phase leave the velocity modes room in 128 registers
+// (512^3 FP32-mixed 189 -> 122, one workgroup -> two; spilled before at two)
+template <typename T>
+constexpr int zinv_waves_t(int n) {
+  return PDR_ZINV_THREADS / kBlock2 * waves_for(lds_zinv_bytes_t<T, PDR_ZINV_THREADS>(n));
+}
+#define PDR_ZINV_WAVES_T __attribute__((amdgpu_waves_per_eu(zinv_waves_t<T>(N))))
 
 template <typename T, int N, int ZT = kBlock2>
 __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ u0, const cx<T>* __restrict__ u1,
@@ -384,9 +399,11 @@ __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const
   const double wi = double(i);
 #pragma unroll
   for (int f = 0; f < 6; ++f) {  // unrolled: every field selection is static
+    if (f == 5 && cf.y3) break;  // the inverse y pass forms the last vorticity component
+    const int t0 = phase_tid<N>();
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
-      const int e = int(threadIdx.x) + ZT * q;
+      const int e = t0 + ZT * q;
       if (EM % ZT == 0 || e < EM) {
         const int line = e / NKK;
         const int k = e - line * NKK;
@@ -411,11 +428,11 @@ __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const
         buf[line * LD + lds_off<T>(z)] = v;
       }
     }
-    zero_band_edges<T, N, L, LD, K, ZT>(buf);
+    zero_band_edges<T, N, L, LD, K, ZT>(buf, t0);
     __syncthreads();
-    fft_ip<T, N, L, LD, +1, true, ZT, K>(buf, tw);
+    fft_ip<T, N, L, LD, +1, true, ZT, K>(buf, tw, phase_tid<N>());
     cx<T>* dst = w1 + (long long)f * g.m1 + (long long)i * N * g.ldj + j0;
-    for (int idx = threadIdx.x; idx < L * N; idx += ZT) {
+    for (int idx = phase_tid<N>(); idx < L * N; idx += ZT) {
       const int z = idx / L;
       const int line = idx - z * L;
       if (j0 + line < nkj) put<kNtZinv>(&dst[z * g.ldj + line], buf[line * LD + lds_off<T>(z)]);
@@ -436,9 +453,20 @@ __global__ void __launch_bounds__(PDR_ZINV_THREADS) PDR_ZINV_WAVES_T
 // ---------------------------------------------------------------------------
 // DY: nine fields instead of six, fields 6..8 being d/dy of fields 0..2 (their modes
 // times i k2 on the way in)
-template <typename T, int N, bool PL, bool DY, int YT = kBlock2>
+// W3: the last vorticity component, i sum_n (G[2][n] . k) u_n, has no k3 in it (the
+// frame maps k3 to the third laboratory direction alone), so the z pass need not
+// transform it: this pass forms it from the modes of the three velocity fields that it
+// loads anyway, kept in registers meanwhile.  Five fields then go through the z pass and
+// over memory to this one instead of six (us a launch, z and y: 512^3 FP64 932 + 1457 ->
+// 749 + 1350, 256^3 FP64 105 + 223 -> 99 + 212, 768 x 128 x 1024 FP32-mixed 594 + 605 ->
+// 488 + 590, 512^3 FP32-mixed 542 + 772 -> 441 + 780: 4.3 TB/s, its FP32 transforms and
+// their addresses bound it there).
+struct YVort {
+  double a[3], b[3];  // factors of k1 and k2 for u_1, u_2, u_3
+};
+template <typename T, int N, bool PL, bool DY, int YT = kBlock2, bool W3 = false>
 __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
-            int ntile, int z0, int nzc, int fpb) {
+            int ntile, int z0, int nzc, int fpb, const YVort& vort = YVort()) {
   constexpr int PP = y_planes<T, PL>(N);
   constexpr int L = y_lines<T, PL>(N);
   constexpr int LD = lds_ld<T>(N);
@@ -464,12 +492,15 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
   constexpr int EM = L * NKJ;
   constexpr int QM = PP > 0 ? QE : (EM + YT - 1) / YT;
   cx<T> pre[QM];
+  // (W3 keeps a field in registers: no room for indices kept from phase to phase)
+  auto tid = [&]() { return W3 ? fresh_tid() : int(threadIdx.x); };
   auto load = [&](int f) {
     const cx<T>* src = w1 + (long long)(DY && f >= 6 ? f - 6 : f) * g.m1 + ((long long)i0 * g.nz + z) * g.ldj;
     if constexpr (PP == 0) {
+      const int t0 = tid();
 #pragma unroll
       for (int q = 0; q < QM; ++q) {
-        const int e = int(threadIdx.x) + YT * q;
+        const int e = t0 + YT * q;
         const int line = e / NKJ;
         cx<T> v = czero<T>();
         if ((EM % YT == 0 || e < EM) && i0 + line < nki) v = get<kNrYinv>(&src[line * lstride + (e - line * NKJ)]);
@@ -497,19 +528,50 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
       pre[q] = DY && f >= 6 ? mul_ik<T>(v, j, K) : v;
     }
   };
+  static_assert(!W3 || (PP == 0 && !DY), "W3 is a form of the tiles of i-lines");
+  constexpr int QW = W3 ? QM : 1;
+  cx<T> acc[QW];
   for (int f = fg * fpb; f < (fg + 1) * fpb; ++f) {
-    load(f);
-    if constexpr (PP == 0) {
+    if (W3 && f == 5) {
 #pragma unroll
-      for (int q = 0; q < QM; ++q) {
-        const int e = int(threadIdx.x) + YT * q;
-        if (EM % YT == 0 || e < EM) {
-          const int line = e / NKJ;
-          const int j = e - line * NKJ;
-          buf[line * LD + lds_off<T>((j <= K) ? j : j + (N - NKJ))] = pre[q];
+      for (int q = 0; q < QW; ++q) pre[q] = mk<T>(-acc[q].y, acc[q].x);
+    } else {
+      load(f);
+    }
+    if constexpr (PP == 0) {
+      // into the tile; W3: times factor(line, j) into acc, the z pass's operations
+      auto fill = [&](auto factor) {
+        const int t0 = tid();
+#pragma unroll
+        for (int q = 0; q < QM; ++q) {
+          const int e = t0 + YT * q;
+          if (EM % YT == 0 || e < EM) {
+            const int line = e / NKJ;
+            const int j = e - line * NKJ;
+            buf[line * LD + lds_off<T>((j <= K) ? j : j + (N - NKJ))] = pre[q];
+            if constexpr (W3 && !std::is_same_v<decltype(factor), int>) acc[q] = add(acc[q], scl(pre[q], T(factor(line, j))));
+          }
         }
+        zero_band_edges<T, N, L, LD, K, YT>(buf, t0);
+      };
+      if constexpr (W3) {
+        if (f == 0) {
+#pragma unroll
+          for (int q = 0; q < QW; ++q) acc[q] = czero<T>();
+        }
+        const double ga = f < 3 ? vort.a[f] : 0.0, gb = f < 3 ? vort.b[f] : 0.0;
+        // (a frame has one of the two for most components)
+        if (ga != 0.0 && gb != 0.0)
+          fill([&](int line, int j) { return ga * double(i0 + line) + gb * wvn2(j, K); });
+        else if (ga != 0.0)
+          fill([&](int line, int) { return ga * double(i0 + line); });
+        else if (gb != 0.0)
+          fill([&](int, int j) { return gb * wvn2(j, K); });
+        else
+          fill(0);
+      } else {
+        fill(0);
       }
-      zero_band_edges<T, N, L, LD, K, YT>(buf);
     } else {
       // whole-plane tiles: every position but those of the skipped band blocks
       // (the band's other positions hold the zeros of the load)
@@ -524,9 +586,9 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
       }
     }
     __syncthreads();
-    fft_ip<T, N, L, LD, +1, true, YT, K>(buf, tw);
+    fft_ip<T, N, L, LD, +1, true, YT, K>(buf, tw, tid());
     cx<T>* dst = w2 + (long long)f * g.m2 + (long long)zl * N * g.ldi + i0;
-    for (int idx = threadIdx.x; idx < L * N; idx += YT) {
+    for (int idx = tid(); idx < L * N; idx += YT) {
       const int y = idx / L;
       const int line = idx - y * L;
       if constexpr (PP > 0) {
@@ -569,6 +631,15 @@ __global__ void __launch_bounds__((yinv_threads<T, N, PL>())) __attribute__((amd
     k2_yinv(Geo g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
   k2_yinv_body<T, N, PL, DY, yinv_threads<T, N, PL>()>(xcd_remap(blockIdx.x, gridDim.x), g, w1, w2, twg, ntile, z0, nzc, fpb);
+}
+
+// the five fields of a z pass with y3 (YVort)
+template <typename T, int N>
+__global__ void __launch_bounds__((yinv_threads<T, N, false>())) __attribute__((amdgpu_waves_per_eu(yinv_waves<T, N, false>())))
+    k2_yinv5(Geo g, YVort vort, const cx<T>* __restrict__ w1, cx<T>* __restrict__ w2, const cx<T>* __restrict__ twg,
+             int ntile, int z0, int nzc) {
+  k2_yinv_body<T, N, false, false, yinv_threads<T, N, false>(), true>(xcd_remap(blockIdx.x, gridDim.x), g, w1, w2, twg,
+                                                                    ntile, z0, nzc, 6, vort);
 }
 
 // ---------------------------------------------------------------------------
@@ -1167,9 +1238,10 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
   cx<T> nlv[3][QF];
   auto load = [&](int f) {
     const cx<T>* src = w1 + (long long)f * g.m1 + (long long)i * N * g.ldj + j0;
+    const int t0 = phase_tid<N>();
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + FT * q;
+      const int idx = t0 + FT * q;
       const int z = idx / L;
       const int line = idx - z * L;
       pre[q] = ((L * N % FT == 0 || idx < L * N) && j0 + line < nkj) ? src[z * g.ldj + line] : czero<T>();
@@ -1179,7 +1251,7 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
       src += 3 * g.m1;
 #pragma unroll
       for (int q = 0; q < QE; ++q) {
-        const int idx = int(threadIdx.x) + FT * q;
+        const int idx = t0 + FT * q;
         const int z = idx / L;
         const int line = idx - z * L;
         if ((L * N % FT == 0 || idx < L * N) && j0 + line < nkj) pre[q] = add(pre[q], src[z * g.ldj + line]);
@@ -1194,9 +1266,10 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
 #pragma unroll
   for (int f = 0; f < 3; ++f) {
     if constexpr (!PF) load(f);
+    const int ts = phase_tid<N>();
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + FT * q;
+      const int idx = ts + FT * q;
       if (L * N % FT == 0 || idx < L * N) {
         const int z = idx / L;
         buf[(idx - z * L) * LD + lds_off<T>(z)] = pre[q];
@@ -1206,10 +1279,11 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
     if constexpr (PF) {
       if (f < 2) load(f + 1);
     }
-    fft_ip<T, N, L, LD, -1, true, FT>(buf, tw);
+    fft_ip<T, N, L, LD, -1, true, FT>(buf, tw, phase_tid<N>());
+    const int tm = phase_tid<N>();
 #pragma unroll
     for (int q = 0; q < QF; ++q) {
-      const int idx = int(threadIdx.x) + FT * q;
+      const int idx = tm + FT * q;
       const int line = idx / NKK;
       const int k = idx - line * NKK;
       const int zz = (k <= K) ? k : N - NKK + k;
@@ -1218,9 +1292,10 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
     __syncthreads();
   }
   const long long e0 = ((long long)i * nkj + j0) * NKK;
+  const int te = phase_tid<N>();
 #pragma unroll
   for (int q = 0; q < QF; ++q) {
-    const int idx = int(threadIdx.x) + FT * q;
+    const int idx = te + FT * q;
     if (idx < nl_lines * NKK) {
       const int line = idx / NKK;
       formf_mode<T, FRC>(g, cf, i, j0 + line, idx - line * NKK, e0 + idx, nlv[0][q], nlv[1][q], nlv[2][q], u0, u1, u2,
@@ -1305,6 +1380,24 @@ hipError_t yinv_t(pdr_ctx* c, int z0, int nzc) {
   k2_yinv<T, N, PL, DY>
       <<<dim3(unsigned(nt * (PP ? 1 : nzc) * ((DY ? 9 : 6) / fpb))), yinv_threads<T, N, PL>(), lds, c->stream>>>(
           g, (const cx<T>*)c->w1, (cx<T>*)c->w2, (const cx<T>*)c->tab.twy, nt, z0, nzc, fpb);
+  return hipGetLastError();
+}
+
+template <typename T, int N>
+hipError_t yinv5_n(pdr_ctx* c, const Coef& cf, int z0, int nzc) {
+  const Geo& g = c->g;
+  constexpr int L = y_lines<T, false>(N);
+  const int nt = (g.nki + L - 1) / L;
+  const size_t lds = size_t(lds_y_bytes<T, false>(N));
+  hipError_t e = big_lds((const void*)k2_yinv5<T, N>, lds);
+  if (e != hipSuccess) return e;
+  YVort v;
+  for (int n = 0; n < 3; ++n) {
+    v.a[n] = cf.G[18 + 3 * n];
+    v.b[n] = cf.G[18 + 3 * n + 1];
+  }
+  k2_yinv5<T, N><<<dim3(unsigned(nt * nzc)), yinv_threads<T, N, false>(), lds, c->stream>>>(
+      g, v, (const cx<T>*)c->w1, (cx<T>*)c->w2, (const cx<T>*)c->tab.twy, nt, z0, nzc);
   return hipGetLastError();
 }
 

@@ -22,6 +22,8 @@ SpecOps ops_of() {
   o.prec = sizeof(T) == 4 ? 1 : 0;
   o.n = N;
   o.yinv = yinv_n<T, N, false>;
+  o.yinv5 = yinv5_n<T, N>;
+  o.y_planes = y_planes<T>(N);
   o.yinv_conv = yinv_n<T, N, true>;
   o.xpass_conv = xpass_conv_n<T, N>;
   o.xpass = xpass_n<T, N>;

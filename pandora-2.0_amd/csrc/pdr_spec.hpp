@@ -9,6 +9,9 @@ struct SpecOps {
   int prec, n;
   hipError_t (*zinv)(pdr_ctx*, const Coef&);
   hipError_t (*yinv)(pdr_ctx*, int z0, int nzc);
+  // the same from the five fields of a z pass with Coef::y3
+  hipError_t (*yinv5)(pdr_ctx*, const Coef&, int z0, int nzc);
+  int y_planes;  // > 0: boxes with NX/3 = NY/3 take whole z planes per y-pass workgroup
   hipError_t (*xpass)(pdr_ctx*, const Coef&, bool tr, bool cfl, int z0, int nzc, double* rsp);
   hipError_t (*yinv_conv)(pdr_ctx*, int z0, int nzc);  // NS_R_CONV: also d/dy of the velocity
   hipError_t (*xpass_conv)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);

@@ -54,7 +54,19 @@ int xpass_tiles(const pdr_ctx* c) {
 }
 
 hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf) { return c->ops_z->zinv(c, cf); }
-hipError_t launch2_yinv(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yinv(c, z0, nzc); }
+hipError_t launch2_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc) {
+  return cf.y3 ? c->ops_y->yinv5(c, cf, z0, nzc) : c->ops_y->yinv(c, z0, nzc);
+}
+// Whether five fields go through the z pass and the y pass forms the last vorticity
+// component: where it has no k3 (every frame of the library itself; not one set by hand
+// with k3 in another direction, in NS_R_ROT), and where one y workgroup takes all six
+// fields of its tile of i-lines, so that it has the velocity's modes in any case (with the
+// fields split over workgroups, or whole-plane tiles, they would be read once more).
+bool z5_fields(const pdr_ctx* c, const Coef& cf) {
+  return c->spec && !conv_form(c) && !plane_fused(c) && !c->ops_z->zz && c->fpb_y == 6 &&
+         !(c->ops_y->y_planes > 0 && c->g.nki == c->g.ny / 3 + 1) && cf.G[20] == 0.0 && cf.G[23] == 0.0 &&
+         cf.G[26] == 0.0;
+}
 hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nzc, double* rsp) {
   return c->ops_x->xpass(c, cf, tr, cfl, z0, nzc, rsp);
 }

@@ -782,7 +782,8 @@ int pdr_rs_stats(pdr_ctx* ctx, pdr_rs_stats_t* out) {
   double* dres = part + size_t(nblk) * pdr::kRsWidth;
   // the real-space planes of the current state: pass 1, then the y and x
   // passes with the moments accumulated in the x pass (its outputs are scratch)
-  const pdr::Coef cf = pdr::make_coef(c);
+  pdr::Coef cf = pdr::make_coef(c);
+  cf.y3 = pdr::z5_fields(c, cf) ? 1 : 0;
   hipError_t e = hipSuccess;
   if (pdr::conv_form(c)) {
     e = pdr::launch_conv_front(c, cf, false, false, part);
@@ -793,7 +794,7 @@ int pdr_rs_stats(pdr_ctx* ctx, pdr_rs_stats_t* out) {
     e = pdr::launch_zinv(c, cf);
     for (int z0 = 0; e == hipSuccess && z0 < g.nz; z0 += g.zc) {
       const int nzc = std::min(g.zc, g.nz - z0);
-      e = pdr::launch_yinv(c, z0, nzc);
+      e = pdr::launch_yinv(c, cf, z0, nzc);
       if (e == hipSuccess) e = pdr::launch_xpass(c, cf, false, false, z0, nzc, part);
     }
   }
