@@ -106,10 +106,15 @@ constexpr int y_lines_fwd(int n) {
 }
 
 // Short lines take more rows per workgroup, so that a workgroup still moves
-// about a thousand points (2 rows of 512; 16 rows of 64).
+// about a thousand points (2 rows of 512; 16 rows of 64).  Half of that where it leaves
+// three quarters of the threads a butterfly in every pass and the CU more workgroups at
+// different phases (us a launch, 8 -> 4 rows at 128^3: FP64 39.8 -> 36.4, FP32-mixed
+// 26.3 -> 24.2; 4 -> 2 rows at 256^3: FP64 300 -> 256, FP32-mixed 129.9 / 128.6; but at
+// 160^3 FP32-mixed 42.8 -> 47.8, 192^3 65.7 -> 75.1, 240^3 FP64 251.7 -> 262.4).
 template <typename T>
 constexpr int xrows(int n) {
-  return n <= 64 ? 16 : (n <= 128 ? 8 : (n <= 256 ? 4 : (sizeof(T) == 4 ? (n <= 512 ? PDR_XROWS_F32 : 2)
+  if (sizeof(T) == 8 && n > 144 && n <= 256 && (n & (n - 1)) == 0) return 2;
+  return n <= 64 ? 16 : (n <= 96 ? 8 : n <= 144 ? 4 : (n <= 256 ? 4 : (sizeof(T) == 4 ? (n <= 512 ? PDR_XROWS_F32 : 2)
                                                                         : (n <= 512 ? PDR_XROWS_F64 : 2))));
 }
 
@@ -149,6 +154,18 @@ constexpr int lds_x_bytes(int n) {
   return ((x_tw_global<T>(n) ? 0 : n) + 3 * xrows<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>)) +
          (kBlock2 / 64) * int(sizeof(T));
 }
+// Threads of the x pass: 512 for the FP64 tiles of which the CU's LDS holds fewer than four
+// (512 points 60 KB, 192 points 42 KB), so that it still has sixteen waves (us a launch at
+// 256^3 with such tiles, 256 -> 512 threads: 322 -> 300; 128^3 43.6 -> 39.8).  The moments'
+// reductions are written for 256.
+template <typename T, int RS>
+constexpr int xthreads(int n) {
+  return RS == 0 && sizeof(T) == 8 && n <= 512 && 4 * lds_x_bytes<T>(n) > kLdsPerCu ? 2 * kBlock2 : kBlock2;
+}
+template <typename T, int RS>
+constexpr int xwaves(int n) {
+  return (kLdsPerCu / lds_x_bytes<T>(n) < 2 ? 1 : 2) * (xthreads<T, RS>(n) / kBlock2);
+}
 // Streaming (non-temporal) stores per kernel, bit mask: 1 zinv, 2 yinv,
 // 4 xpass, 8 yfwd, 16 zfwd.  Every pass writes data that only the next pass
 // reads, long after the caches have turned over: streaming stores keep the
@@ -184,8 +201,6 @@ constexpr bool small_store(int n) { return n <= PDR_SMALL_STORE_MAX; }
 }
 #define PDR_LINE_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_lines_bytes<T>(N)))))
 #define PDR_FWD_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_fwd_bytes<T>(N)))))
-#define PDR_X_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_x_bytes<T>(N)))))
-#define PDR_YF_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_yf_bytes<T, PL>(N)))))
 
 // Line kernels issue all global loads of a field (QE elements per thread)
 // before the LDS stores of that field, so that one HBM latency is exposed per
@@ -607,20 +622,35 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
 // The single-box inverse y pass of tiles of i-lines runs 512-thread workgroups
 // over the same tile: half the elements per thread, so the registers of a wave
 // fall below half of what 256 threads need and the CU holds twice the waves
-// (the tile's LDS then bounds it) to keep more loads in flight.  Whole-plane
-// tiles of short lines and the batched ensembles keep 256 threads.
+// (the tile's LDS then bounds it) to keep more loads in flight.  The
+// batched ensembles keep 256 threads.
+// Lines of up to 128 points take 256: their tile is a butterfly or less per thread of
+// 512, and more tiles fit a CU (us a launch, 512 -> 256 threads: 128^3 FP64 31.3 -> 29.0,
+// 128^3 FP32-mixed 20.1 -> 17.9, 768 x 128 x 1024 FP32-mixed 590 -> 551, 120 x 48 x 96 FP64
+// 20.8 -> 15.1; but 160^3 FP32-mixed 33.2 -> 36.9).
 #ifndef PDR_YINV_THREADS
 #define PDR_YINV_THREADS 512
 #endif
+#ifndef PDR_YINV_SHORT
+#define PDR_YINV_SHORT 128
+#endif
+// FP64 whole-plane tiles (some 50 KB of LDS, three to a CU) take 512 as well, in both
+// directions (us a launch, 256 -> 512: inverse at 96^3 22.8 -> 18.2, nine fields 27.7 -> 24.2);
+// the batched ensembles keep 256.
+template <typename T>
+constexpr int yplane_threads() {
+  return sizeof(T) == 8 ? 2 * kBlock2 : kBlock2;
+}
 template <typename T, int N, bool PL>
 constexpr int yinv_threads() {
-  return y_planes<T, PL>(N) ? kBlock2 : PDR_YINV_THREADS;
+  return y_planes<T, PL>(N) ? yplane_threads<T>() : N <= PDR_YINV_SHORT ? kBlock2 : PDR_YINV_THREADS;
 }
 // waves per SIMD declared to the register allocator: as for the other passes
 // (at most two 256-thread workgroups), or the two waves per SIMD of each
 // 512-thread workgroup times the workgroups the LDS admits, at most four
 template <typename T, int N, bool PL>
 constexpr int yinv_waves() {
+  if (!y_planes<T, PL>(N) && N <= PDR_YINV_SHORT) return 4;
   constexpr int wg = kLdsPerCu / lds_y_bytes<T, PL>(N) < 1 ? 1 : kLdsPerCu / lds_y_bytes<T, PL>(N);
   return yinv_threads<T, N, PL>() == kBlock2 ? waves_for(lds_y_bytes<T, PL>(N))
                                           : (wg * (yinv_threads<T, N, PL>() / kBlock2) > 4 ? 4 : wg * (yinv_threads<T, N, PL>() / kBlock2));
@@ -881,11 +911,11 @@ __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const 
 }
 
 template <typename T, int N, int RS>
-__global__ void __launch_bounds__(kBlock2) PDR_X_WAVES
+__global__ void __launch_bounds__((xthreads<T, RS>(N))) __attribute__((amdgpu_waves_per_eu(xwaves<T, RS>(N))))
     k2_xpass(Geo g, Coef cf, cx<T>* __restrict__ w2, T* __restrict__ ur, int want_tr, int want_cfl,
              unsigned long long* __restrict__ umax, const cx<T>* __restrict__ twg, int ntile, int z0,
              double* __restrict__ rsp) {
-  k2_xpass_body<T, N, RS>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w2, ur, want_tr, want_cfl, umax, twg, ntile, z0,
+  k2_xpass_body<T, N, RS, xthreads<T, RS>(N)>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w2, ur, want_tr, want_cfl, umax, twg, ntile, z0,
                           rsp);
 }
 
@@ -904,6 +934,7 @@ __global__ void __launch_bounds__(kBlock2) PDR_X_WAVES
 // ---------------------------------------------------------------------------
 template <typename T>
 constexpr int xrows_conv(int n) {  // half the rows of k2_xpass: twice the lines a row
+  if (sizeof(T) == 4 && n > 96 && n <= 128) return 4;  // (128^3: 33.4 us a launch against 35.7 with 2; FP64 57.3 with 2, 68.6 with 4)
   return xrows<T>(n) > 4 ? xrows<T>(n) / 2 : 2;
 }
 template <typename T>
@@ -1070,7 +1101,7 @@ __global__ void __launch_bounds__(kBlock2) PDR_XC_WAVES
 // ---------------------------------------------------------------------------
 // pass 4: forward y FFT + truncation, (z, i-tile) per block
 // ---------------------------------------------------------------------------
-template <typename T, int N, bool PL>
+template <typename T, int N, bool PL, int YT = kBlock2>
 __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const cx<T>* __restrict__ w2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
   constexpr int PP = y_planes<T, PL>(N);
@@ -1078,7 +1109,7 @@ __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const c
   constexpr int LD = lds_ld<T>(N);
   constexpr int K = N / 3;
   constexpr int NKJ = 2 * K + 1;
-  constexpr int QE = (L * N + kBlock2 - 1) / kBlock2;
+  constexpr int QE = (L * N + YT - 1) / YT;
   extern __shared__ __align__(16) unsigned char smem[];
   cx<T>* tw = reinterpret_cast<cx<T>*>(smem);
   cx<T>* buf = tw + N;
@@ -1090,23 +1121,23 @@ __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const c
   const int i0 = PP ? 0 : tile * L;
   const int nki = g.nki;
   const int lstride = g.nz * g.ldj;
-  load_tw<T, N>(tw, twg);
+  load_tw<T, N, YT>(tw, twg);
   cx<T> pre[QE];
   auto load = [&](int f) {
     const cx<T>* src = w2 + (long long)f * g.m2 + (long long)zl * N * g.ldi + i0;
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + kBlock2 * q;
+      const int idx = int(threadIdx.x) + YT * q;
       const int y = idx / L;
       const int line = idx - y * L;
       if constexpr (PP > 0) {
         const int p = line / (K + 1);
         const int zz = tile * PP + p;
-        pre[q] = ((L * N % kBlock2 == 0 || idx < L * N) && zz < nzc)
+        pre[q] = ((L * N % YT == 0 || idx < L * N) && zz < nzc)
                      ? get<kNrYfwd>(&src[((long long)zz * N + y) * g.ldi + (line - p * (K + 1))])
                      : czero<T>();
       } else {
-        pre[q] = ((L * N % kBlock2 == 0 || idx < L * N) && i0 + line < nki) ? get<kNrYfwd>(&src[y * g.ldi + line])
+        pre[q] = ((L * N % YT == 0 || idx < L * N) && i0 + line < nki) ? get<kNrYfwd>(&src[y * g.ldi + line])
                                                                           : czero<T>();
       }
     }
@@ -1115,16 +1146,16 @@ __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const c
     load(f);
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + kBlock2 * q;
-      if (L * N % kBlock2 == 0 || idx < L * N) {
+      const int idx = int(threadIdx.x) + YT * q;
+      if (L * N % YT == 0 || idx < L * N) {
         const int y = idx / L;
         buf[(idx - y * L) * LD + lds_off<T>(y)] = pre[q];
       }
     }
     __syncthreads();
-    fft_ip<T, N, L, LD, -1>(buf, tw);
+    fft_ip<T, N, L, LD, -1, true, YT>(buf, tw);
     cx<T>* dst = w1 + (long long)f * g.m1 + ((long long)i0 * g.nz + z) * g.ldj;
-    for (int idx = threadIdx.x; idx < L * NKJ; idx += kBlock2) {
+    for (int idx = threadIdx.x; idx < L * NKJ; idx += YT) {
       const int line = idx / NKJ;
       const int j = idx - line * NKJ;
       const int yy = (j <= K) ? j : N - NKJ + j;
@@ -1142,10 +1173,15 @@ __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const c
 }
 
 template <typename T, int N, bool PL>
-__global__ void __launch_bounds__(kBlock2) PDR_YF_WAVES
+constexpr int yfwd_threads() {
+  return y_planes<T, PL>(N) ? yplane_threads<T>() : kBlock2;
+}
+template <typename T, int N, bool PL>
+__global__ void __launch_bounds__((yfwd_threads<T, N, PL>()))
+    __attribute__((amdgpu_waves_per_eu(waves_for(lds_yf_bytes<T, PL>(N)) * (yfwd_threads<T, N, PL>() / kBlock2))))
     k2_yfwd(Geo g, const cx<T>* __restrict__ w2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg,
             int ntile, int z0, int nzc, int fpb) {
-  k2_yfwd_body<T, N, PL>(xcd_remap(blockIdx.x, gridDim.x), g, w2, w1, twg, ntile, z0, nzc, fpb);
+  k2_yfwd_body<T, N, PL, yfwd_threads<T, N, PL>()>(xcd_remap(blockIdx.x, gridDim.x), g, w2, w1, twg, ntile, z0, nzc, fpb);
 }
 
 // ---------------------------------------------------------------------------
@@ -1429,7 +1465,7 @@ hipError_t xpass_n(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nz
     constexpr int RS = decltype(rs_c)::value;
     hipError_t e = big_lds((const void*)k2_xpass<T, N, RS>, lds);
     if (e != hipSuccess) return e;
-    k2_xpass<T, N, RS><<<dim3(unsigned(nt * nzc)), kBlock2, lds, c->stream>>>(
+    k2_xpass<T, N, RS><<<dim3(unsigned(nt * nzc)), xthreads<T, RS>(N), lds, c->stream>>>(
         g, cf, (cx<T>*)c->w2, (T*)c->ur, tr ? 1 : 0, cfl ? 1 : 0, c->umax, (const cx<T>*)c->tab.twx, nt, z0, rsp);
     return hipGetLastError();
   };
@@ -1466,7 +1502,7 @@ hipError_t yfwd_t(pdr_ctx* c, int z0, int nzc) {
   const size_t lds = size_t(lds_yf_bytes<T, PL>(N));
   hipError_t e = big_lds((const void*)k2_yfwd<T, N, PL>, lds);
   if (e != hipSuccess) return e;
-  k2_yfwd<T, N, PL><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (3 / c->fpb_yf))), kBlock2, lds, c->stream>>>(
+  k2_yfwd<T, N, PL><<<dim3(unsigned(nt * (PP ? 1 : nzc) * (3 / c->fpb_yf))), yfwd_threads<T, N, PL>(), lds, c->stream>>>(
       g, (const cx<T>*)c->w2, (cx<T>*)c->w1, (const cx<T>*)c->tab.twy, nt, z0, nzc, c->fpb_yf);
   return hipGetLastError();
 }
