@@ -154,13 +154,14 @@ constexpr int lds_x_bytes(int n) {
   return ((x_tw_global<T>(n) ? 0 : n) + 3 * xrows<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>)) +
          (kBlock2 / 64) * int(sizeof(T));
 }
-// Threads of the x pass: 512 for the FP64 tiles of which the CU's LDS holds fewer than four
-// (512 points 60 KB, 192 points 42 KB), so that it still has sixteen waves (us a launch at
-// 256^3 with such tiles, 256 -> 512 threads: 322 -> 300; 128^3 43.6 -> 39.8).  The moments'
+// Threads of the x pass: 512 for the tiles of which the CU's LDS holds fewer than four (FP64
+// 192 points 42 KB, 512 points 60 KB; FP32-mixed 768 points 45 KB), so that it still has
+// sixteen waves (us a launch, 256 -> 512 threads: 512^3 FP64 2418 -> 2168, 768^3 FP64
+// 16050 -> 12020, 768 x 128 x 1024 FP32-mixed 1206 -> 950, 640^3 2573 -> 2542).  The moments'
 // reductions are written for 256.
 template <typename T, int RS>
 constexpr int xthreads(int n) {
-  return RS == 0 && sizeof(T) == 8 && n <= 512 && 4 * lds_x_bytes<T>(n) > kLdsPerCu ? 2 * kBlock2 : kBlock2;
+  return RS == 0 && 4 * lds_x_bytes<T>(n) > kLdsPerCu ? 2 * kBlock2 : kBlock2;
 }
 template <typename T, int RS>
 constexpr int xwaves(int n) {
@@ -199,7 +200,17 @@ constexpr bool small_store(int n) { return n <= PDR_SMALL_STORE_MAX; }
 [[maybe_unused]] constexpr int waves_for(int lds) {
   return kLdsPerCu / lds < 2 ? 1 : 2;
 }
-#define PDR_LINE_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_lines_bytes<T>(N)))))
+// Threads of the passes of lines above 512 points: 512, since a CU holds two or three of
+// their tiles (us a launch, 256 -> 512: z forward 768 x 128 x 1024 FP32-mixed 243 -> 216,
+// 640^3 625 -> 547, 768^3 FP64 1916 -> 1717; y forward 640^3 FP32-mixed 978 -> 851, 768^3
+// FP64 2812 -> 2601).  The inverse z pass, which keeps the velocity's loads of a field in
+// registers, only where two fit (768 x 128 x 1024 490 -> 435, 768^3 FP64 3632 -> 3305; but
+// 640^3 FP32-mixed 1380 -> 1449).
+constexpr int zthreads(int n) { return n > 512 ? 2 * kBlock2 : kBlock2; }
+template <typename T>
+constexpr int zinv_threads(int n) {
+  return 3 * lds_lines_bytes<T>(n) > kLdsPerCu ? zthreads(n) : kBlock2;
+}
 #define PDR_FWD_WAVES __attribute__((amdgpu_waves_per_eu(waves_for(lds_fwd_bytes<T>(N)))))
 
 // Line kernels issue all global loads of a field (QE elements per thread)
@@ -212,14 +223,15 @@ constexpr bool small_store(int n) { return n <= PDR_SMALL_STORE_MAX; }
 // pass 1: vorticity + inverse z FFT, (i, j-tile) per block
 // ---------------------------------------------------------------------------
 template <typename T, int N>
-__global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
+__global__ void __launch_bounds__((zinv_threads<T>(N))) __attribute__((amdgpu_waves_per_eu(waves_for(lds_lines_bytes<T>(N)) * (zinv_threads<T>(N) / kBlock2))))
     k2_zinv(Geo g, Coef cf, const cx<T>* __restrict__ u0, const cx<T>* __restrict__ u1,
             const cx<T>* __restrict__ u2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg, int ntile) {
+  constexpr int ZT = zinv_threads<T>(N);
   constexpr int L = tile_lines<T>(N);
   constexpr int LD = lds_ld<T>(N);
   constexpr int K = N / 3;
   constexpr int NKK = 2 * K + 1;
-  constexpr int QE = (L * N + kBlock2 - 1) / kBlock2;
+  constexpr int QE = (L * N + ZT - 1) / ZT;
   extern __shared__ __align__(16) unsigned char smem[];
   cx<T>* tw = reinterpret_cast<cx<T>*>(smem);
   cx<T>* buf = tw + N;
@@ -228,7 +240,7 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
   const int i = int(bid / unsigned(ntile));
   const int j0 = tile * L;
   const int nkj = g.nkj;
-  load_tw<T, N>(tw, twg);
+  load_tw<T, N, ZT>(tw, twg);
   const double wi = double(i);
   bool need[3][3];
 #pragma unroll
@@ -245,11 +257,11 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
   auto load_u = [&](int f) {
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + kBlock2 * q;
+      const int idx = int(threadIdx.x) + ZT * q;
       const int line = idx / N;
       const int z = idx - line * N;
       const int k = (z <= K) ? z : ((z >= N - K) ? z - (N - NKK) : -1);
-      pre[q] = ((L * N % kBlock2 == 0 || idx < L * N) && j0 + line < nkj && k >= 0) ? uu[f][line * NKK + k]
+      pre[q] = ((L * N % ZT == 0 || idx < L * N) && j0 + line < nkj && k >= 0) ? uu[f][line * NKK + k]
                                                                                     : czero<T>();
     }
   };
@@ -263,19 +275,19 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
       cx<T> a[VC][3];
 #pragma unroll
       for (int qq = 0; qq < VC; ++qq) {
-        const int idx = int(threadIdx.x) + kBlock2 * (q0 + qq);
+        const int idx = int(threadIdx.x) + ZT * (q0 + qq);
         const int line = idx / N;
         const int z = idx - line * N;
         const int k = (z <= K) ? z : ((z >= N - K) ? z - (N - NKK) : -1);
-        const bool ok = (QE % VC == 0 || q0 + qq < QE) && (L * N % kBlock2 == 0 || idx < L * N) &&
+        const bool ok = (QE % VC == 0 || q0 + qq < QE) && (L * N % ZT == 0 || idx < L * N) &&
                         j0 + line < nkj && k >= 0;
 #pragma unroll
         for (int n = 0; n < 3; ++n) a[qq][n] = (ok && need[c][n]) ? uu[n][line * NKK + k] : czero<T>();
       }
 #pragma unroll
       for (int qq = 0; qq < VC; ++qq) {
-        const int idx = int(threadIdx.x) + kBlock2 * (q0 + qq);
-        if ((QE % VC == 0 || q0 + qq < QE) && (L * N % kBlock2 == 0 || idx < L * N)) {
+        const int idx = int(threadIdx.x) + ZT * (q0 + qq);
+        if ((QE % VC == 0 || q0 + qq < QE) && (L * N % ZT == 0 || idx < L * N)) {
           const int line = idx / N;
           const int z = idx - line * N;
           const int k = (z <= K) ? z : ((z >= N - K) ? z - (N - NKK) : 0);
@@ -299,8 +311,8 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
       load_u(f);
 #pragma unroll
       for (int q = 0; q < QE; ++q) {
-        const int idx = int(threadIdx.x) + kBlock2 * q;
-        if (L * N % kBlock2 == 0 || idx < L * N) {
+        const int idx = int(threadIdx.x) + ZT * q;
+        if (L * N % ZT == 0 || idx < L * N) {
           const int line = idx / N;
           buf[line * LD + lds_off<T>(idx - line * N)] = pre[q];
         }
@@ -309,9 +321,9 @@ __global__ void __launch_bounds__(kBlock2) PDR_LINE_WAVES
       fill_w(f - 3);
     }
     __syncthreads();
-    fft_ip<T, N, L, LD, +1>(buf, tw);
+    fft_ip<T, N, L, LD, +1, true, ZT>(buf, tw);
     cx<T>* dst = w1 + (long long)f * g.m1 + (long long)i * N * g.ldj + j0;
-    for (int idx = threadIdx.x; idx < L * N; idx += kBlock2) {
+    for (int idx = threadIdx.x; idx < L * N; idx += ZT) {
       const int z = idx / L;
       const int line = idx - z * L;
       if (j0 + line < nkj) put<kNtZinv>(&dst[z * g.ldj + line], buf[line * LD + lds_off<T>(z)]);
@@ -1174,7 +1186,7 @@ __device__ __forceinline__ void k2_yfwd_body(unsigned bid, const Geo& g, const c
 
 template <typename T, int N, bool PL>
 constexpr int yfwd_threads() {
-  return y_planes<T, PL>(N) ? yplane_threads<T>() : kBlock2;
+  return y_planes<T, PL>(N) ? yplane_threads<T>() : zthreads(N);
 }
 template <typename T, int N, bool PL>
 __global__ void __launch_bounds__((yfwd_threads<T, N, PL>()))
@@ -1188,14 +1200,15 @@ __global__ void __launch_bounds__((yfwd_threads<T, N, PL>()))
 // pass 5: forward z FFT, normalisation, truncation -> NL [c][i][j][k]
 // ---------------------------------------------------------------------------
 template <typename T, int N>
-__global__ void __launch_bounds__(kBlock2) PDR_FWD_WAVES
+__global__ void __launch_bounds__((zthreads(N))) __attribute__((amdgpu_waves_per_eu(waves_for(lds_fwd_bytes<T>(N)) * (zthreads(N) / kBlock2))))
     k2_zfwd(Geo g, const cx<T>* __restrict__ w1, cx<T>* __restrict__ nl, const cx<T>* __restrict__ twg,
             int ntile, T norm) {
+  constexpr int ZT = zthreads(N);
   constexpr int L = tile_lines_fwd<T>(N);
   constexpr int LD = lds_ld<T>(N);
   constexpr int K = N / 3;
   constexpr int NKK = 2 * K + 1;
-  constexpr int QE = (L * N + kBlock2 - 1) / kBlock2;
+  constexpr int QE = (L * N + ZT - 1) / ZT;
   extern __shared__ __align__(16) unsigned char smem[];
   cx<T>* tw = reinterpret_cast<cx<T>*>(smem);
   cx<T>* buf = tw + N;
@@ -1204,33 +1217,33 @@ __global__ void __launch_bounds__(kBlock2) PDR_FWD_WAVES
   const int i = int(bid / unsigned(ntile));
   const int j0 = tile * L;
   const int nkj = g.nkj;
-  load_tw<T, N>(tw, twg);
+  load_tw<T, N, ZT>(tw, twg);
   cx<T> pre[QE];
   auto load = [&](int f) {
     const cx<T>* src = w1 + (long long)f * g.m1 + (long long)i * N * g.ldj + j0;
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + kBlock2 * q;
+      const int idx = int(threadIdx.x) + ZT * q;
       const int z = idx / L;
       const int line = idx - z * L;
-      pre[q] = ((L * N % kBlock2 == 0 || idx < L * N) && j0 + line < nkj) ? get<kNrZfwd>(&src[z * g.ldj + line]) : czero<T>();
+      pre[q] = ((L * N % ZT == 0 || idx < L * N) && j0 + line < nkj) ? get<kNrZfwd>(&src[z * g.ldj + line]) : czero<T>();
     }
   };
   for (int f = 0; f < 3; ++f) {
     load(f);
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + kBlock2 * q;
-      if (L * N % kBlock2 == 0 || idx < L * N) {
+      const int idx = int(threadIdx.x) + ZT * q;
+      if (L * N % ZT == 0 || idx < L * N) {
         const int z = idx / L;
         buf[(idx - z * L) * LD + lds_off<T>(z)] = pre[q];
       }
     }
     __syncthreads();
-    fft_ip<T, N, L, LD, -1>(buf, tw);
+    fft_ip<T, N, L, LD, -1, true, ZT>(buf, tw);
     cx<T>* dst = nl + (long long)f * g.mw + ((long long)i * nkj + j0) * NKK;
     const int nl_lines = (nkj - j0) < L ? (nkj - j0) : L;
-    for (int idx = threadIdx.x; idx < nl_lines * NKK; idx += kBlock2) {
+    for (int idx = threadIdx.x; idx < nl_lines * NKK; idx += ZT) {
       const int line = idx / NKK;
       const int k = idx - line * NKK;
       const int zz = (k <= K) ? k : N - NKK + k;
@@ -1395,7 +1408,7 @@ hipError_t zinv_n(pdr_ctx* c, const Coef& cf) {
     const size_t lds = lds_lines<T, N>();
     hipError_t e = big_lds((const void*)k2_zinv<T, N>, lds);
     if (e != hipSuccess) return e;
-    k2_zinv<T, N><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
+    k2_zinv<T, N><<<dim3(unsigned(nt * g.nki)), zinv_threads<T>(N), lds, c->stream>>>(
         g, cf, (const cx<T>*)c->u[0], (const cx<T>*)c->u[1], (const cx<T>*)c->u[2], (cx<T>*)c->w1,
         (const cx<T>*)c->tab.twz, nt);
     return hipGetLastError();
@@ -1524,7 +1537,7 @@ hipError_t zfwd_n(pdr_ctx* c) {
   hipError_t e = big_lds((const void*)k2_zfwd<T, N>, lds);
   if (e != hipSuccess) return e;
   const double norm = 1.0 / (double(g.nx) * double(g.ny) * double(g.nz));
-  k2_zfwd<T, N><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
+  k2_zfwd<T, N><<<dim3(unsigned(nt * g.nki)), zthreads(N), lds, c->stream>>>(
       g, (const cx<T>*)c->w1, (cx<T>*)c->nl, (const cx<T>*)c->tab.twz, nt, T(norm));
   return hipGetLastError();
 }
