@@ -37,9 +37,11 @@ def kernel_bytes(g, name, csz, rsz, ntr):
     """Compulsory bytes one launch of each kernel must move (its inputs + outputs)."""
     m2 = g.nz * g.ny * g.nki
     n3 = g.nx * g.ny * g.nz
+    # large boxes: the y inverse forms the last vorticity component itself
+    zf = 5 if g.nz > 128 and (g.nki + 15) // 16 * g.nz >= 1024 else 6
     return {
-        "zinv": (3 * g.mw + 6 * g.m1) * csz,
-        "yinv": (6 * g.m1 + 6 * m2) * csz,
+        "zinv": (3 * g.mw + zf * g.m1) * csz,
+        "yinv": (zf * g.m1 + 6 * m2) * csz,
         "xpass": 9 * m2 * csz + (3 * n3 * rsz if ntr else 0),
         "yfwd": (3 * m2 + 3 * g.m1) * csz,
         "zfwd": (3 * g.m1 + 3 * g.mw) * csz,
@@ -430,7 +432,7 @@ def zstreams_ab(pa, n, ntr, steps=5, repeats=3):
 # this script), written to profiles/; the traffic JSON feeds roofline.traffic.
 # ---------------------------------------------------------------------------
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "rk3_step_512_shear_fp32_traffic.json")
-KERNEL_CLASS = {"zinv": "zinv", "zinv_r": "zinv", "yinv": "yinv", "xpass": "xpass", "yfwd": "yfwd",
+KERNEL_CLASS = {"zinv": "zinv", "zinv_r": "zinv", "yinv": "yinv", "yinv5": "yinv", "xpass": "xpass", "yfwd": "yfwd",
                 "zfwd": "zfwd", "formf": "formf", "zfwd_formf": "zfwdformf", "tracers": "tracers",
                 "tracers_col": "tracers", "copy": "copy"}
 
@@ -462,7 +464,7 @@ def rocpd_summary(trace_db, fetch_db, write_db, out_json, sq_dbs=(), copy_bytes=
         m = re.search(r"k2?_[a-z0-9_]+<(float|double)", name)
         if m:
             base += "<f32>" if m.group(1) == "float" else "<f64>"
-        if re.search(r"k2_xpass<[a-z]+, \d+, true>", name):
+        if re.search(r"k2_xpass<[a-z]+, \d+, [12]>", name):
             base += " with moments"  # the stage-1 x pass of a step with statistics
         a = agg.setdefault(base, [0, 0.0, 1e30, 0.0])
         a[0] += 1
