@@ -709,6 +709,13 @@ static Coef next_coef(pdr_ctx* c, int stage, int32_t tstep, double tstart, doubl
   return f;
 }
 
+// Whether the advance is long enough for a stream of its own.  A short one is about what the
+// two waits between streams cost the device, and their four event calls hold up the host
+// (us a step, beside -> in line: 120 x 48 x 96 FP64 with 5000 tracers 239 -> 198, forced
+// 128^3 FP32-mixed with 16384 260 -> 248, with 60000 280 -> 262, forced 64^3 FP64 with
+// 60000 190 -> 149; but 256^3 FP64 with 60000 2504 -> 2519, whose passes leave the host time).
+static bool tracers_beside(const pdr_ctx* c) { return c->np >= (c->g.nr <= (1 << 22) ? 65536 : 16384); }
+
 static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, StageLink* link);
 
 int pdr_stage(pdr_ctx* c, int32_t stage, int32_t tstep, double time, double* dt) {
@@ -839,13 +846,18 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
   const double gdt = gamma * (*dt);
   if (tracers) {
     // the advance reads the tracer field the x pass wrote and nothing the forward
-    // passes touch: it runs on the tracer stream beside them
-    HIPCHK(hipEventRecord(c->ev_ur, c->stream));
-    HIPCHK(hipStreamWaitEvent(c->tstream, c->ev_ur, 0));
-    if (stage == 1 && tstep == c->ts_release) HIPCHK(tracers_release(c, c->tstream));
-    HIPCHK(launch_tracers(c, c->tf_ur, beta, gdt, c->tstream));
-    if (pstats) HIPCHK(launch_pstats_rel(c, tstep, c->tstream));
-    HIPCHK(hipEventRecord(c->ev_tr, c->tstream));
+    // passes touch: it runs on the tracer stream beside them, or where it is short
+    // (tracers_beside) between them, which saves the two streams' waits
+    const bool beside = tracers_beside(c);
+    const hipStream_t ts = beside ? c->tstream : c->stream;
+    if (beside) {
+      HIPCHK(hipEventRecord(c->ev_ur, c->stream));
+      HIPCHK(hipStreamWaitEvent(c->tstream, c->ev_ur, 0));
+    }
+    if (stage == 1 && tstep == c->ts_release) HIPCHK(tracers_release(c, ts));
+    HIPCHK(launch_tracers(c, c->tf_ur, beta, gdt, ts));
+    if (pstats) HIPCHK(launch_pstats_rel(c, tstep, ts));
+    if (beside) HIPCHK(hipEventRecord(c->ev_tr, c->tstream));
   } else if (pstats && !field) {
     HIPCHK(launch_pstats_rel(c, tstep, c->stream));
   }
@@ -865,7 +877,7 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
   }
   // and at the end of f_RK3SolveNavierStokes (src/pf_rk3.f90:2101-2109)
   HIPCHK(launch_dealias(c));
-  if (tracers) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_tr, 0));
+  if (tracers && tracers_beside(c)) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_tr, 0));
   link->z_ready = link->join;
   return PDR_OK;
 }
