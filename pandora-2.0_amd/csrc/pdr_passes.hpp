@@ -486,8 +486,7 @@ __global__ void __launch_bounds__(PDR_ZINV_THREADS) PDR_ZINV_WAVES_T
 // loads anyway, kept in registers meanwhile.  Five fields then go through the z pass and
 // over memory to this one instead of six (us a launch, z and y: 512^3 FP64 932 + 1457 ->
 // 749 + 1350, 256^3 FP64 105 + 223 -> 99 + 212, 768 x 128 x 1024 FP32-mixed 594 + 605 ->
-// 488 + 590, 512^3 FP32-mixed 542 + 772 -> 441 + 780: 4.3 TB/s, its FP32 transforms and
-// their addresses bound it there).
+// 488 + 590, 512^3 FP32-mixed 542 + 772 -> 441 + 737).
 struct YVort {
   double a[3], b[3];  // factors of k1 and k2 for u_1, u_2, u_3
 };
@@ -521,6 +520,9 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
   cx<T> pre[QM];
   // (W3 keeps a field in registers: no room for indices kept from phase to phase)
   auto tid = [&]() { return W3 ? fresh_tid() : int(threadIdx.x); };
+  // (the transform's and the stores' fit in FP32: formed anew there too, 785 us a launch
+  // at 512^3 against 737)
+  auto tid2 = [&]() { return W3 && sizeof(T) == 8 ? fresh_tid() : int(threadIdx.x); };
   auto load = [&](int f) {
     const cx<T>* src = w1 + (long long)(DY && f >= 6 ? f - 6 : f) * g.m1 + ((long long)i0 * g.nz + z) * g.ldj;
     if constexpr (PP == 0) {
@@ -613,9 +615,9 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
       }
     }
     __syncthreads();
-    fft_ip<T, N, L, LD, +1, true, YT, K>(buf, tw, tid());
+    fft_ip<T, N, L, LD, +1, true, YT, K>(buf, tw, tid2());
     cx<T>* dst = w2 + (long long)f * g.m2 + (long long)zl * N * g.ldi + i0;
-    for (int idx = tid(); idx < L * N; idx += YT) {
+    for (int idx = tid2(); idx < L * N; idx += YT) {
       const int y = idx / L;
       const int line = idx - y * L;
       if constexpr (PP > 0) {
