@@ -58,8 +58,8 @@ using pdr::set_error;
 const double kBeta[3] = {0.0, -5.0 / 9.0, -153.0 / 128.0};
 const double kGamma[3] = {1.0 / 3.0, 15.0 / 16.0, 8.0 / 15.0};
 
-void ens_release(pdr_ensemble* e) {
-  for (EnsGroup& q : e->groups) {
+void ens_release(std::vector<EnsGroup>& groups) {
+  for (EnsGroup& q : groups) {
     if (q.stream) (void)hipStreamSynchronize(q.stream);
     for (hipGraphExec_t x : {q.joined_exec, q.last_exec})
       if (x) (void)hipGraphExecDestroy(x);
@@ -67,7 +67,7 @@ void ens_release(pdr_ensemble* e) {
       if (x) (void)hipGraphDestroy(x);
     if (q.stream) (void)hipStreamDestroy(q.stream);
   }
-  e->groups.clear();
+  groups.clear();
 }
 
 // Captures one RK3 step of a group: 3 stages of the inverse z pass (where the stage
@@ -90,8 +90,11 @@ hipError_t ens_capture(pdr_ensemble* e, EnsGroup& q, int fpb_y, int fpb_yf, bool
   return hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
 }
 
-int ens_build(pdr_ensemble* e) {
-  ens_release(e);
+// The groups' graphs for a split of the y passes (0: each member's own choice).  They are
+// made beside the ones that stand and take their place once all are there, so an
+// ensemble whose rebuild fails keeps its graphs and its split.
+int ens_build(pdr_ensemble* e, int fpb_y, int fpb_yf) {
+  std::vector<EnsGroup> groups;
   const int nm = int(e->m.size());
   std::vector<pdr_ctx*> order = e->m;
   std::stable_sort(order.begin(), order.end(), [](const pdr_ctx* a, const pdr_ctx* b) { return a->g.nx < b->g.nx; });
@@ -103,9 +106,9 @@ int ens_build(pdr_ensemble* e) {
       q.ops = pdr::ens_ops(c->prec, c->g.nx);
       q.first = k;
       if (!q.ops) return set_error(PDR_ERR_UNSUPPORTED, "ensemble: unsupported line length");
-      e->groups.push_back(q);
+      groups.push_back(q);
     }
-    ++e->groups.back().count;
+    ++groups.back().count;
     pdr::EnsMember& d = h[size_t(k)];
     std::memset(&d, 0, sizeof(d));
     d.g = c->g;
@@ -129,9 +132,9 @@ int ens_build(pdr_ensemble* e) {
     return set_error(PDR_ERR_NOMEM, "ensemble: device allocation failed");
   }
   hipError_t r = hipMemcpy(e->d_mem, h.data(), sizeof(pdr::EnsMember) * size_t(nm), hipMemcpyHostToDevice);
-  for (EnsGroup& q : e->groups) {
+  for (EnsGroup& q : groups) {
     const pdr_ctx* c = order[size_t(q.first)];
-    const int fy = e->fpb_y ? e->fpb_y : c->fpb_y, fyf = e->fpb_yf ? e->fpb_yf : c->fpb_yf;
+    const int fy = fpb_y ? fpb_y : c->fpb_y, fyf = fpb_yf ? fpb_yf : c->fpb_yf;
     if (r == hipSuccess) r = q.ops->prepare();
     if (r == hipSuccess) r = hipStreamCreateWithFlags(&q.stream, hipStreamNonBlocking);
     if (r == hipSuccess) r = ens_capture(e, q, fy, fyf, false, &q.last, &q.last_exec);
@@ -139,9 +142,13 @@ int ens_build(pdr_ensemble* e) {
   }
   if (r != hipSuccess) {
     (void)hipGetLastError();
-    ens_release(e);
+    ens_release(groups);
     return set_error(PDR_ERR_HIP, std::string("ensemble set-up: ") + hipGetErrorString(r));
   }
+  ens_release(e->groups);
+  e->groups.swap(groups);
+  e->fpb_y = fpb_y;
+  e->fpb_yf = fpb_yf;
   return PDR_OK;
 }
 
@@ -191,7 +198,7 @@ int pdr_ensemble_create(pdr_ensemble** out, pdr_ctx* const* members, int32_t cou
     delete e;
     return set_error(PDR_ERR_HIP, "pdr_ensemble_create: stream creation failed");
   }
-  int rc = ens_build(e);
+  int rc = ens_build(e, 0, 0);
   if (rc != PDR_OK) {
     pdr_ensemble_destroy(e);
     return rc;
@@ -205,15 +212,14 @@ int pdr_ensemble_set_split(pdr_ensemble* e, int32_t fpb_y, int32_t fpb_yf) {
   const bool ok = (fpb_y == 0 || fpb_y == 1 || fpb_y == 2 || fpb_y == 3 || fpb_y == 6) &&
                   (fpb_yf == 0 || fpb_yf == 1 || fpb_yf == 3);
   if (!ok) return set_error(PDR_ERR_ARG, "pdr_ensemble_set_split: fields per workgroup must divide 6 / 3");
-  e->fpb_y = fpb_y;
-  e->fpb_yf = fpb_yf;
-  return ens_build(e);
+  return ens_build(e, fpb_y, fpb_yf);
 }
 
 // Times `steps` graph steps for each split of the y passes over workgroups
 // (fields per workgroup 1, 2, 3, 6 for the inverse pass and 1, 3 for the
 // forward pass), keeps the fastest, and restores every member's state and RK
-// registers, so the ensemble is where it was before the call.
+// registers, so the ensemble is where it was before the call; after an error it has
+// the split and the graphs of before as well.
 int pdr_ensemble_autotune(pdr_ensemble* e, int32_t steps, int32_t* best_y, int32_t* best_yf) {
   if (!e || steps < 1) return set_error(PDR_ERR_ARG, "pdr_ensemble_autotune: bad argument");
   for (pdr_ctx* c : e->m)
@@ -249,12 +255,14 @@ int pdr_ensemble_autotune(pdr_ensemble* e, int32_t steps, int32_t* best_y, int32
   int by = e->fpb_y ? e->fpb_y : 6, byf = e->fpb_yf ? e->fpb_yf : 3;
   bool split = false;  // nothing to tune where every member's planes run as one kernel
   for (const EnsGroup& q : e->groups) split = split || q.ops->split;
+  const bool saved = r == hipSuccess;
+  std::vector<EnsGroup> before;
+  before.swap(e->groups);
+  const int before_y = e->fpb_y, before_yf = e->fpb_yf;
   int rc = PDR_OK;
   for (int iy = 0; iy < 4 && split && r == hipSuccess && rc == PDR_OK; ++iy)
     for (int iyf = 0; iyf < 2 && r == hipSuccess && rc == PDR_OK; ++iyf) {
-      e->fpb_y = ys[iy];
-      e->fpb_yf = yfs[iyf];
-      rc = ens_build(e);
+      rc = ens_build(e, ys[iy], yfs[iyf]);
       if (rc != PDR_OK) break;
       r = ens_steps(e, 1);  // warm-up
       const auto t0 = std::chrono::steady_clock::now();
@@ -266,15 +274,23 @@ int pdr_ensemble_autotune(pdr_ensemble* e, int32_t steps, int32_t* best_y, int32
         byf = yfs[iyf];
       }
     }
-  if (r == hipSuccess) r = copy_state(false);
+  if (saved) {
+    const hipError_t back = copy_state(false);
+    if (r == hipSuccess) r = back;
+  }
   (void)hipFree(save);
-  if (rc != PDR_OK) return rc;
-  if (r != hipSuccess) return set_error(PDR_ERR_HIP, std::string("pdr_ensemble_autotune: ") + hipGetErrorString(r));
-  e->fpb_y = by;
-  e->fpb_yf = byf;
+  if (r == hipSuccess && rc == PDR_OK) rc = ens_build(e, by, byf);
+  if (r != hipSuccess || rc != PDR_OK) {
+    ens_release(e->groups);
+    e->groups.swap(before);
+    e->fpb_y = before_y;
+    e->fpb_yf = before_yf;
+    return r != hipSuccess ? set_error(PDR_ERR_HIP, std::string("pdr_ensemble_autotune: ") + hipGetErrorString(r)) : rc;
+  }
+  ens_release(before);
   if (best_y) *best_y = by;
   if (best_yf) *best_yf = byf;
-  return ens_build(e);
+  return PDR_OK;
 }
 
 int pdr_ensemble_run(pdr_ensemble* e, int32_t tstep0, int32_t nsteps, double* simtime) {
@@ -283,6 +299,7 @@ int pdr_ensemble_run(pdr_ensemble* e, int32_t tstep0, int32_t nsteps, double* si
   for (pdr_ctx* c : e->m)  // work queued on the members' own streams comes first
     if (hipStreamSynchronize(c->stream) != hipSuccess)
       return set_error(PDR_ERR_HIP, "pdr_ensemble_run: member stream failed");
+  if (e->groups.empty()) return set_error(PDR_ERR_STATE, "pdr_ensemble_run: the ensemble has no graphs");
   const hipError_t r = ens_steps(e, nsteps);
   if (r != hipSuccess) return set_error(PDR_ERR_HIP, std::string("pdr_ensemble_run: ") + hipGetErrorString(r));
   for (int32_t s = 0; s < nsteps; ++s)
@@ -298,7 +315,7 @@ int pdr_ensemble_run(pdr_ensemble* e, int32_t tstep0, int32_t nsteps, double* si
 int pdr_ensemble_destroy(pdr_ensemble* e) {
   if (!e) return PDR_OK;
   if (e->stream) (void)hipStreamSynchronize(e->stream);
-  ens_release(e);
+  ens_release(e->groups);
   if (e->d_mem) (void)hipFree(e->d_mem);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;

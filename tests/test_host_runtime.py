@@ -1,0 +1,69 @@
+"""The library's host code on a stand-in for the HIP runtime (tests/host_runtime): what an
+entry point does when a runtime call fails, and what it asks the runtime for.  Each case runs
+in a process of its own, where the stand-in is loaded first; no GPU is used, kernels do not
+run, so values are checked only where copies alone carry them."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PROLOGUE = """
+import ctypes as C, os, sys
+S = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
+S.stand_in_fail.argtypes = [C.c_char_p, C.c_longlong, C.c_int]
+S.stand_in_count.argtypes, S.stand_in_count.restype = [C.c_char_p], C.c_longlong
+S.stand_in_bytes.argtypes, S.stand_in_bytes.restype = [C.c_int], C.c_longlong
+sys.path.insert(0, {pkg!r})
+import numpy as np
+import pandora_amd as pa
+
+def fail(call, nth=1, error=999):
+    S.stand_in_fail(call.encode(), nth, error)
+def count(call):
+    return S.stand_in_count(call.encode())
+def raises(f, *a):
+    try:
+        f(*a)
+    except pa.PdrError as e:
+        return e.code
+    return 0
+"""
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("host_runtime") / "libhip_stand_in.so")
+    subprocess.run(["g++", "-O1", "-Wall", "-std=c++17", "-shared", "-fPIC",
+                    os.path.join(HERE, "host_runtime", "hip_stand_in.cpp"), "-o", lib], check=True)
+    return lib
+
+
+def _run(lib, body, **env):
+    code = PROLOGUE.format(lib=lib, pkg=os.path.join(os.path.dirname(HERE), "pandora-2.0_amd")) + textwrap.dedent(body)
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                       env={**os.environ, **env})
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+@pytest.mark.parametrize("call", ["hipGraphInstantiate", "hipStreamBeginCapture", "hipStreamCreateWithFlags"])
+@pytest.mark.parametrize("tune", [False, True], ids=["set_split", "autotune"])
+def test_ensemble_keeps_its_graphs_when_a_rebuild_fails(stand_in, call, tune):
+    """Every step that a run reports has been queued, whichever call of whichever rebuild fails."""
+    _run(stand_in, f"""
+    sizes = [32, 96, 32, 128]
+    e = pa.Ensemble([pa.Pandora(n, rk3_timestep=2, rk3_dt=0.25) for n in sizes])
+    for nth in range(1, 60):
+        fail({call!r}, nth)
+        rc = raises(e.autotune, 1) if {tune} else raises(e.set_split, 1, 1)
+        fail({call!r}, 0)
+        before = count("hipGraphLaunch")
+        assert list(e.run(1, 5, [0.0] * 4)) == [1.25] * 4
+        assert count("hipGraphLaunch") - before == 5 * 3  # a graph a step for each of the three lengths
+        if rc == 0:
+            break
+    assert nth > (8 if {tune} else 2)  # the failing cases came first
+    """)
