@@ -54,6 +54,7 @@ hipError_t stage_reserve(pdr_ctx* c, size_t bytes) {
   c->stage_bytes = 0;
   const hipError_t e = hipHostMalloc(&c->stage, bytes, hipHostMallocDefault);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // the caller goes on without: later launch checks read it
     c->stage = nullptr;
     return e;
   }
@@ -78,26 +79,33 @@ void words_in(void* dst, const double* src, size_t n, bool f32) {
   for (size_t q = 0; q < n; ++q) d[q] = float(src[q]);
 }
 
+// Straight to or from the caller's arrays, through the runtime's own buffers.
+template <bool OUT>
+hipError_t pageable(pdr_ctx* c, int fields, void* const* dev, double* const* host, long long n, bool f32) {
+  const size_t fbytes = size_t(n) * (f32 ? sizeof(float) : sizeof(double));
+  hipError_t e = hipStreamSynchronize(c->stream);
+  std::vector<float> tmp(f32 ? size_t(n) : 0);
+  for (int f = 0; f < fields && e == hipSuccess; ++f) {
+    void* h = f32 ? (void*)tmp.data() : (void*)host[f];
+    if (!OUT && f32) words_in(h, host[f], size_t(n), true);
+    e = OUT ? hipMemcpy(h, dev[f], fbytes, hipMemcpyDeviceToHost) : hipMemcpy(dev[f], h, fbytes, hipMemcpyHostToDevice);
+    if (OUT && f32 && e == hipSuccess) words_out(host[f], h, size_t(n), true);
+  }
+  return e;
+}
+
 template <bool OUT>
 hipError_t transfer(pdr_ctx* c, int fields, void* const* dev, double* const* host, long long n, bool f32) {
   const size_t w = f32 ? sizeof(float) : sizeof(double);
   const size_t fbytes = size_t(n) * w, total = fbytes * size_t(fields);
   // Pinning costs 0.3 ms for a small box's fields and up to 4 ms for the chunks: not spent
   // on what is often done once, a small box's uploads and first download and FP64 uploads.
-  if (OUT ? total <= kSmall && c->small_downloads++ == 0 : total <= kSmall || !f32) {
-    hipError_t e = hipStreamSynchronize(c->stream);
-    std::vector<float> tmp(f32 ? size_t(n) : 0);
-    for (int f = 0; f < fields && e == hipSuccess; ++f) {
-      void* h = f32 ? (void*)tmp.data() : (void*)host[f];
-      if (!OUT && f32) words_in(h, host[f], size_t(n), true);
-      e = OUT ? hipMemcpy(h, dev[f], fbytes, hipMemcpyDeviceToHost) : hipMemcpy(dev[f], h, fbytes, hipMemcpyHostToDevice);
-      if (OUT && f32 && e == hipSuccess) words_out(host[f], h, size_t(n), true);
-    }
-    return e;
-  }
+  // Where the host has no pinned memory to give, every transfer goes this way.
+  if (OUT ? total <= kSmall && c->small_downloads++ == 0 : total <= kSmall || !f32)
+    return pageable<OUT>(c, fields, dev, host, n, f32);
   if (OUT && total <= kSmall) {
-    hipError_t e = stage_reserve(c, total);
-    if (e == hipSuccess) e = launch_xfer(c, c->stage, dev, fields, n, f32);
+    if (stage_reserve(c, total) != hipSuccess) return pageable<OUT>(c, fields, dev, host, n, f32);
+    hipError_t e = launch_xfer(c, c->stage, dev, fields, n, f32);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess)
       for (int f = 0; f < fields; ++f) words_out(host[f], (char*)c->stage + fbytes * size_t(f), size_t(n), f32);
@@ -107,9 +115,9 @@ hipError_t transfer(pdr_ctx* c, int fields, void* const* dev, double* const* hos
   const size_t per = (fbytes + kChunk - 1) / kChunk, chunks = per * size_t(fields);
   const int hw = int(std::max(1u, std::thread::hardware_concurrency()));
   const int T = std::max(1, std::min({kMaxThreads, hw, int(chunks / 8)}));
-  hipError_t e = stage_reserve(c, 2 * size_t(T) * kChunk);
+  if (stage_reserve(c, 2 * size_t(T) * kChunk) != hipSuccess) return pageable<OUT>(c, fields, dev, host, n, f32);
   int device = 0;
-  if (e == hipSuccess) e = hipGetDevice(&device);
+  hipError_t e = hipGetDevice(&device);
   // the threads start when there is something to move: waiting for the steps queued
   // before, each would hold a core
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);

@@ -67,3 +67,22 @@ def test_ensemble_keeps_its_graphs_when_a_rebuild_fails(stand_in, call, tune):
             break
     assert nth > (8 if {tune} else 2)  # the failing cases came first
     """)
+
+
+@pytest.mark.parametrize("n,prec", [(32, "PDR_FP64"), (32, "PDR_FP32_MIXED"), (96, "PDR_FP64"), (96, "PDR_FP32_MIXED")])
+def test_transfers_without_pinned_memory(stand_in, n, prec):
+    """Small states and states of several chunks, velocity and RK registers, four times over: they
+    arrive whole where the host has no pinned memory left, and the box is usable afterwards."""
+    _run(stand_in, f"""
+    fail("hipHostMalloc", 1, 2)
+    g = pa.Pandora({n}, precision=pa.{prec})
+    rng = np.random.default_rng(1)
+    for rep in range(4):
+        u = [(rng.integers(-99, 99, g.shape) + 1j * rng.integers(-99, 99, g.shape)).astype(complex) for _ in range(3)]
+        g.set_state(*u)
+        assert all((a == b).all() for a, b in zip(g.get_state(), u))
+        g.set_rk(*u[::-1])
+        assert all((a == b).all() for a, b in zip(g.get_rk(), u[::-1]))
+        g.run(rep + 1, 1, 0.0)  # launches that look at the runtime's last error
+    assert count("hipHostMalloc") > 0 and S.stand_in_bytes(1) == 0
+    """)
