@@ -419,6 +419,7 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     delete c;
     return fail(PDR_ERR_HIP, std::string("no HIP device: ") + hipGetErrorString(he));
   }
+  c->device = dev;
   int lds = 65536;
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) lds = 65536;
   c->lds_max = size_t(lds);

@@ -122,6 +122,7 @@ struct Tables {
 struct pdr_ctx {
   pdr_params p;
   pdr::Geo g;
+  int device = 0;   // the device that was current at pdr_create: its streams and buffers are there
   int prec = 0;     // 0 FP64, 1 FP32-mixed
   size_t csz = 16;  // bytes per complex element
   size_t rsz = 8;   // bytes per real element
@@ -243,6 +244,25 @@ hipError_t launch_tracers(pdr_ctx* c, const TracerFrame& tf, double beta, double
 hipError_t launch_tracers_wrap(pdr_ctx* c, const TracerFrame& tf, hipStream_t s);
 hipError_t launch_remesh(pdr_ctx* c, int bfrot);
 hipError_t launch_remesh_particles(pdr_ctx* c, double lx, double dx);
+// Makes the context's device the current one for a scope: a transfer launches kernels and
+// records events, which take a stream of the current device only, and the caller may have
+// made another device current since pdr_create.
+class OnDevice {
+ public:
+  explicit OnDevice(const pdr_ctx* c) {
+    int now = c->device;
+    if (hipGetDevice(&now) == hipSuccess && now != c->device && hipSetDevice(c->device) == hipSuccess) back_ = now;
+  }
+  ~OnDevice() {
+    if (back_ >= 0) (void)hipSetDevice(back_);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+
+ private:
+  int back_ = -1;
+};
+
 // host transfers (pdr_xfer.hip): `fields` (1..3) arrays of n reals each, FP64 on the host,
 // FP32 on the device where f32; in stream order, done on return
 int xfer_to_host(pdr_ctx* c, int fields, const void* const* dev, double* const* host, long long n, bool f32);

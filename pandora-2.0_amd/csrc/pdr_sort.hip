@@ -155,6 +155,7 @@ __global__ void __launch_bounds__(256)
 // the device, in the sort's spare array (unsorted slots have the caller's order)
 int particles_to_host(pdr_ctx* c, const double* dev, double* host) {
   const double* src = dev;
+  const OnDevice on(c);
   if (c->spare) {
     k_unsort3<<<dim3(unsigned((3 * c->np + 255) / 256)), 256, 0, c->stream>>>(dev, c->spare, c->pid, c->np);
     if (hipGetLastError() != hipSuccess) return set_error(PDR_ERR_HIP, "particle download: launch failed");

@@ -96,6 +96,7 @@ hipError_t pageable(pdr_ctx* c, int fields, void* const* dev, double* const* hos
 
 template <bool OUT>
 hipError_t transfer(pdr_ctx* c, int fields, void* const* dev, double* const* host, long long n, bool f32) {
+  const OnDevice on(c);
   const size_t w = f32 ? sizeof(float) : sizeof(double);
   const size_t fbytes = size_t(n) * w, total = fbytes * size_t(fields);
   // Pinning costs 0.3 ms for a small box's fields and up to 4 ms for the chunks: not spent
@@ -116,15 +117,13 @@ hipError_t transfer(pdr_ctx* c, int fields, void* const* dev, double* const* hos
   const int hw = int(std::max(1u, std::thread::hardware_concurrency()));
   const int T = std::max(1, std::min({kMaxThreads, hw, int(chunks / 8)}));
   if (stage_reserve(c, 2 * size_t(T) * kChunk) != hipSuccess) return pageable<OUT>(c, fields, dev, host, n, f32);
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
   // the threads start when there is something to move: waiting for the steps queued
   // before, each would hold a core
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  hipError_t e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return e;
   std::vector<hipError_t> err(size_t(T), hipSuccess);
   auto work = [&](int t) {
-    hipError_t r = hipSetDevice(device);
+    hipError_t r = hipSetDevice(c->device);
     hipEvent_t ev[2] = {nullptr, nullptr};
     for (hipEvent_t& x : ev)
       if (r == hipSuccess) r = hipEventCreateWithFlags(&x, hipEventDisableTiming);

@@ -86,3 +86,28 @@ def test_transfers_without_pinned_memory(stand_in, n, prec):
         g.run(rep + 1, 1, 0.0)  # launches that look at the runtime's last error
     assert count("hipHostMalloc") > 0 and S.stand_in_bytes(1) == 0
     """)
+
+
+@pytest.mark.parametrize("n,prec", [(32, "PDR_FP64"), (32, "PDR_FP32_MIXED"), (96, "PDR_FP64"), (96, "PDR_FP32_MIXED")])
+def test_transfers_with_another_device_current(stand_in, n, prec):
+    """A program with boxes on two devices reads each whichever device is current, and finds the
+    device that it had made current afterwards."""
+    _run(stand_in, f"""
+    boxes = []
+    for dev in (0, 1):
+        assert S.hipSetDevice(dev) == 0
+        boxes.append(pa.Pandora({n}, precision=pa.{prec}))
+        boxes[-1].set_particle_sort(0)
+        boxes[-1].set_particles(np.linspace(0.1, 6.0, 3 * 70000).reshape(-1, 3))
+    for dev in (1, 0):
+        assert S.hipSetDevice(dev) == 0
+        for g in boxes:
+            u = [np.full(g.shape, 2.0 + k - 3.0j) for k in range(3)]
+            g.set_state(*u)
+            for rep in range(4):
+                v = g.get_state()
+                if {n} == 96:  # a small state's later downloads are a kernel's work
+                    assert all((a == b).all() for a, b in zip(v, u))
+                g.get_particles()
+            assert S.stand_in_device() == dev
+    """)
