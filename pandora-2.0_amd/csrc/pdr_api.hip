@@ -529,8 +529,11 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     if (rc == PDR_OK) rc = dalloc(c, &c->rk[q], wbytes);
   }
   if (rc == PDR_OK) rc = dalloc(c, &c->w1, 6 * size_t(g.m1) * c->csz);
-  if (rc == PDR_OK) rc = dalloc(c, &c->w2, std::max((c->spec && conv_form(c) ? 9 : 6) * size_t(g.m2),
-                                                        3 * size_t(c->nl_parts) * size_t(g.m1)) * c->csz);
+  // the addends of the fused planes are whole boxes; one addend stays in w1, so that the
+  // x-pencil buffer of a chunked box is its chunk
+  const size_t nl_elems = c->nl_parts > 1 ? 3 * size_t(c->nl_parts) * size_t(g.m1) : 0;
+  if (rc == PDR_OK)
+    rc = dalloc(c, &c->w2, std::max((c->spec && conv_form(c) ? 9 : 6) * size_t(g.m2), nl_elems) * c->csz);
   if (rc == PDR_OK && c->zs2) rc = dalloc(c, &c->w2z, 6 * size_t(g.m2) * c->csz);
   if (rc == PDR_OK) c->nl = static_cast<char*>(c->w1) + 3 * size_t(g.m1) * c->csz;
   if (rc == PDR_OK && conv_form(c) && !c->spec) {

@@ -111,3 +111,26 @@ def test_transfers_with_another_device_current(stand_in, n, prec):
                 g.get_particles()
             assert S.stand_in_device() == dev
     """)
+
+
+@pytest.mark.parametrize("prec", ["PDR_FP64", "PDR_FP32_MIXED"])
+@pytest.mark.parametrize("mb,streams", [(1, 1), (2, 1), (2, 2)])
+def test_chunked_box_holds_a_chunk(stand_in, prec, mb, streams):
+    """The x-pencil buffers of a chunked box are one chunk (two with two in flight), the rest of
+    the device memory is that of the whole-box run less its x-pencil buffer."""
+    _run(stand_in, f"""
+    n = (144, 128, 120)
+    csz = 16 if pa.{prec} == pa.PDR_FP64 else 8
+    plane = 6 * n[1] * (-(-(n[0] // 3 + 1) // 16) * 16) * csz
+    size = {{}}
+    for chunked in (False, True):
+        if chunked:
+            os.environ["PDR_ZCHUNK_MB"], os.environ["PDR_ZSTREAMS"] = "{mb}", "{streams}"
+        g = pa.Pandora(nx=n[0], ny=n[1], nz=n[2], precision=pa.{prec})
+        size[chunked] = int(g.sizes()[6])
+        assert S.stand_in_bytes(0) == size[chunked]
+        zc = g.kernel_forms()["zchunk"]
+        assert zc == (max(1, min(n[2], {mb} * 1048576 // plane)) if chunked else n[2])
+        g.close()
+    assert size[True] == size[False] - (n[2] - {streams} * zc) * plane
+    """)
