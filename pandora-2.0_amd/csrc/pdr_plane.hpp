@@ -36,14 +36,24 @@ constexpr int plane_lds_bytes(int n, int s) {
   const int x = 3 * m * lds_ld<T>(n), y = 6 * nki * lds_ld<T>(m);
   return (n + (s > 1 ? n + m : 0) + (x > y ? x : y)) * int(sizeof(cx<T>));
 }
-constexpr int kPlaneLds = 158 * 1024;  // leaves the static arrays of the reductions
+// Threads: the first x pass's butterflies in as few equal rounds as 1024 threads allow.
+constexpr int plane_threads(int n, int s) {
+  const int b = 3 * (n / s) * (n / plan_radix(n, 0));
+  const int rounds = (b + 1023) / 1024;
+  return ((b + rounds - 1) / rounds + 63) / 64 * 64;
+}
+// Bytes of the kernel's own arrays, the CFL maxima and the moments' sums of its waves.
+template <typename T>
+constexpr int plane_static_bytes(int n, int s) {
+  return (plane_threads(n, s) / 64 * (kRsWidth * int(sizeof(double)) + int(sizeof(T))) + 15) / 16 * 16;
+}
 // The longest planes taken this way, and the parts a plane is taken in (0: the
-// separate passes run): the fewest, at least `least`, whose tile fits.
+// separate passes run): the fewest, at least `least`, that the LDS of a CU holds.
 template <typename T, bool ENS = false>
 constexpr int plane_parts(int n, int least) {
   if (!ENS && n > PDR_PLANE_MAX) return 0;
   for (int s = least; 8 * s <= n + 7; ++s)
-    if (n % s == 0 && plane_lds_bytes<T>(n, s) <= kPlaneLds) return s;
+    if (n % s == 0 && plane_lds_bytes<T>(n, s) + plane_static_bytes<T>(n, s) <= kLdsPerCu) return s;
   return least > 1 ? plane_parts<T, ENS>(n, 1) : 0;
 }
 // Parts of a single box's planes: enough for the groups below to fill the chip
@@ -52,12 +62,6 @@ template <typename T>
 constexpr int plane_parts_box(int n) {
   const int want = (256 + n - 1) / n;
   return plane_parts<T>(n, want < 4 ? want : 4);
-}
-// Threads: the first x pass's butterflies in as few equal rounds as 1024 threads allow.
-constexpr int plane_threads(int n, int s) {
-  const int b = 3 * (n / s) * (n / plan_radix(n, 0));
-  const int rounds = (b + 1023) / 1024;
-  return ((b + rounds - 1) / rounds + 63) / 64 * 64;
 }
 
 // Parts gr, gr + ng, ... of plane z, from w1 into the three fields at dst (w1 itself
@@ -86,8 +90,8 @@ __device__ __forceinline__ void plane_body(int z, int gr, int ng, const Geo& g, 
     load_tw<T, M, NT, S>(twy, twg);
     for (int m = threadIdx.x; m < N; m += NT) twp[m] = twg[m];
   }
-  // modes (f, i, j) of the plane at f m1 + i nz ldj + j; 32-bit byte offsets (six fields of
-  // the longest planes hold 30 MB), so that a load in flight holds one register of address
+  // modes (f, i, j) of the plane at f m1 + i nz ldj + j; 32-bit byte offsets (plane_offsets_fit),
+  // so that a load in flight holds one register of address
   const char* const wz = reinterpret_cast<const char*>(w1 + (long long)z * g.ldj);
   char* const dz = reinterpret_cast<char*>(dst + (long long)z * g.ldj);
   const unsigned fstr = unsigned(g.m1), istr = unsigned(g.nz * g.ldj);

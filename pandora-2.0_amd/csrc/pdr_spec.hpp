@@ -23,7 +23,7 @@ struct SpecOps {
   bool zz;
   // passes 2 to 4 of n x n planes in one launch (pdr_plane.hpp), null where they do not fit
   hipError_t (*plane)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
-  size_t lds_plane;
+  size_t lds_plane;  // the kernel's own arrays included
   int plane_parts;
   size_t lds_z, lds_y, lds_x, lds_xc;  // the largest workgroup of the z, y, x and NS_R_CONV x passes
   int xrows, xrows_conv;       // rows of an x tile

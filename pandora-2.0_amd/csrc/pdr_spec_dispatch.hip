@@ -36,11 +36,13 @@ void spec_forms(const pdr_ctx* c, int out[4]) {
   out[3] = c->ops_z->zinv_lines;
 }
 
+// The plane kernel reaches the modes of a plane by 32-bit byte offsets into six fields.
+static bool plane_offsets_fit(const pdr_ctx* c) { return 6 * size_t(c->g.m1) * c->csz <= size_t(UINT32_MAX); }
 // Whether the y and x passes of a plane run as one kernel: square planes of a length
 // that has it, unless the environment asks for the chunked passes or their streams.
 bool plane_fused(const pdr_ctx* c) {
   return c->spec && !conv_form(c) && !c->plane_separate && c->g.nx == c->g.ny && c->ops_x->plane &&
-         c->ops_x->lds_plane <= c->lds_max && c->g.zc == c->g.nz;
+         c->ops_x->lds_plane <= c->lds_max && plane_offsets_fit(c) && c->g.zc == c->g.nz;
 }
 hipError_t launch2_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
   return c->ops_x->plane(c, cf, tr, cfl, rsp);
