@@ -10,6 +10,7 @@ Outputs (git-ignored, shipped with the source tree):
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -25,10 +26,19 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FC = os.environ.get("PDR_FC", "/opt/rocm/bin/amdflang")
 ARCH = "gfx950"
 
-SPEC_TUS = 8  # kSpecTus of pdr_spec.hpp: pdr_spec.hip is compiled once for each group of line lengths
-# (source, extra defines, object); the costliest first
+
+def spec_lengths():
+    """The line lengths of PDR_SPEC_LENGTHS (pdr_spec.hpp)."""
+    with open(os.path.join(CSRC, "pdr_spec.hpp")) as f:
+        rows = re.search(r"#define PDR_SPEC_LENGTHS\(X\)((?:.*\\\n)*.*\n)", f.read()).group(1)
+    return [int(n) for n in re.findall(r"X\((\d+)\)", rows)]
+
+
+# (source, extra defines, object); the costliest first.  pdr_spec.hip is compiled once for
+# each length and precision.
 SOURCES = [("pdr_ens_passes.hip", [], "pdr_ens_passes.o")]
-SOURCES += [("pdr_spec.hip", [f"-DPDR_SPEC_TU={k}"], f"pdr_spec_{k}.o") for k in range(SPEC_TUS)]
+SOURCES += [("pdr_spec.hip", [f"-DPDR_SPEC_N={n}", f"-DPDR_SPEC_FP32={f}"], f"pdr_spec_{n}_f{32 if f else 64}.o")
+            for n in sorted(spec_lengths(), reverse=True) for f in (0, 1)]
 SOURCES += [(f"{s}.hip", [], f"{s}.o") for s in ("pdr_api", "pdr_kernels", "pdr_spec_dispatch", "pdr_host", "pdr_xfer", "pdr_stats",
                                                  "pdr_pstats", "pdr_sort", "pdr_ens")]
 

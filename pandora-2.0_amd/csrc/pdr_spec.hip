@@ -1,13 +1,14 @@
-// pdr_spec.hip -- the pass kernels of pdr_passes.hpp for the lengths of one
-// translation unit; compiled once per PDR_SPEC_TU (build_lib.py), so that the
-// lengths build side by side.
+// pdr_spec.hip -- the pass kernels of pdr_passes.hpp for one line length and precision:
+// compiled once per PDR_SPEC_N and PDR_SPEC_FP32 (build_lib.py), each a code object of
+// its own (pdr_spec.hpp).
 #include "pdr_passes.hpp"
 #include "pdr_plane.hpp"
 #include "pdr_spec.hpp"
 #include "pdr_zall.hpp"
 
-#ifndef PDR_SPEC_TU
-#define PDR_SPEC_TU 0
+#ifndef PDR_SPEC_N
+#define PDR_SPEC_N 32
+#define PDR_SPEC_FP32 0
 #endif
 #define PDR_CAT2(a, b) a##b
 #define PDR_CAT(a, b) PDR_CAT2(a, b)
@@ -56,14 +57,14 @@ SpecOps ops_of() {
 
 }  // namespace
 
-const SpecOps* PDR_CAT(spec_table_, PDR_SPEC_TU)(int* count) {
-  static const SpecOps t[] = {
-#define PDR_ROW(n) ops_of<float, n>(), ops_of<double, n>(),
-      PDR_CAT(PDR_SPEC_SIZES_, PDR_SPEC_TU)(PDR_ROW)
-#undef PDR_ROW
-  };
-  *count = int(sizeof(t) / sizeof(t[0]));
-  return t;
+#if PDR_SPEC_FP32
+const SpecOps* PDR_CAT(spec_ops_f32_, PDR_SPEC_N)() {
+  static const SpecOps o = ops_of<float, PDR_SPEC_N>();
+#else
+const SpecOps* PDR_CAT(spec_ops_f64_, PDR_SPEC_N)() {
+  static const SpecOps o = ops_of<double, PDR_SPEC_N>();
+#endif
+  return &o;
 }
 
 }  // namespace pdr

@@ -35,34 +35,29 @@ struct SpecOps {
 // The specialised path of a line length, or null (pdr_spec_dispatch.hip).
 const SpecOps* spec_ops(int prec, int n);
 
-// Lengths of the translation units that pdr_spec.hip is compiled into, one per
-// PDR_SPEC_TU, the long and costly ones spread over them: every even length of
-// 24 .. 512 points that a 2^a 3^b 5^c box of the reference's form 2^a {1, 3, 5}
-// or with one more factor 3 or 5 has, and 640 .. 1536.  Other lengths, and tiles
-// beyond a workgroup's LDS, run the runtime-radix kernels of pdr_kernels.hip, which
-// ping-pong two LDS buffers with run-time index divisions: twelve FP32 steps of a
-// 160^3 box with the CFL time step, spherical truncation and the state read back
-// take 20.2 ms there and 9.0 ms here, twelve FP64 steps of 120 x 48 x 96 with 5000
-// tracers 7.2 against 3.7 ms.
-#define PDR_SPEC_SIZES_0(X) X(32) X(128) X(512) X(180) X(300)
-#define PDR_SPEC_SIZES_1(X) X(48) X(192) X(384) X(24) X(320)
-#define PDR_SPEC_SIZES_2(X) X(64) X(256) X(768) X(36) X(360)
-#define PDR_SPEC_SIZES_3(X) X(96) X(100) X(1024) X(40) X(200)
-#define PDR_SPEC_SIZES_4(X) X(60) X(108) X(1536) X(400) X(160)
-#define PDR_SPEC_SIZES_5(X) X(72) X(80) X(1280) X(240) X(432)
-#define PDR_SPEC_SIZES_6(X) X(120) X(640) X(288) X(480) X(216)
-#define PDR_SPEC_SIZES_7(X) X(144) X(960) X(150) X(250) X(90) X(30)
-constexpr int kSpecTus = 8;
+// The lengths with specialised kernels, a chosen set: 2^a {1, 3, 5} and 2^a 15 from 24 to
+// 1536 points, and up to 512 points the other even 2^a 3^b 5^c except 50, 54, 162, 270, 324,
+// 450, 486 and 500.  Those, the odd ones, the shorter ones and the rest of the longer ones,
+// and tiles beyond a workgroup's LDS, run the runtime-radix kernels of
+// pdr_kernels.hip, which ping-pong two LDS buffers with run-time index divisions: twelve FP32
+// steps of a 160^3 box with the CFL time step, spherical truncation and the state read back
+// take 20.2 ms there and 7.2 ms here, twelve FP64 steps of 120 x 48 x 96 with 5000 tracers
+// 7.2 against 2.7 ms.
+//
+// pdr_spec.hip is compiled once for each length and precision (build_lib.py reads them
+// here), which makes each a code object of its own: the runtime loads a code object whole at
+// the first launch from it, some 60 us for every kernel in it, so a program pays for the
+// lengths that it steps.  First step of a 32^3 FP32-mixed box in a process 1.3 ms; 11.4 with
+// eight code objects of five lengths in both precisions each, of which boxes of 32, 48, 64 and
+// 96 points then take four (five steps of 64 such boxes, loads included, 53 -> 21 ms).
+#define PDR_SPEC_LENGTHS(X) X(24) X(30) X(32) X(36) X(40) X(48) X(60) X(64) X(72) X(80) X(90) X(96) X(100) \
+   X(108) X(120) X(128) X(144) X(150) X(160) X(180) X(192) X(200) X(216) X(240) X(250) X(256) X(288) X(300) \
+   X(320) X(360) X(384) X(400) X(432) X(480) X(512) X(640) X(768) X(960) X(1024) X(1280) X(1536)
 
-// The table of translation unit K and its length.
-#define PDR_SPEC_TABLE(K) const SpecOps* spec_table_##K(int* count)
-PDR_SPEC_TABLE(0);
-PDR_SPEC_TABLE(1);
-PDR_SPEC_TABLE(2);
-PDR_SPEC_TABLE(3);
-PDR_SPEC_TABLE(4);
-PDR_SPEC_TABLE(5);
-PDR_SPEC_TABLE(6);
-PDR_SPEC_TABLE(7);
+#define PDR_ROW(n)                   \
+  const SpecOps* spec_ops_f32_##n(); \
+  const SpecOps* spec_ops_f64_##n();
+PDR_SPEC_LENGTHS(PDR_ROW)
+#undef PDR_ROW
 
 }  // namespace pdr

@@ -4,16 +4,15 @@
 namespace pdr {
 
 const SpecOps* spec_ops(int prec, int n) {
-  using Table = const SpecOps* (*)(int*);
-  static const Table tables[kSpecTus] = {spec_table_0, spec_table_1, spec_table_2, spec_table_3,
-                                         spec_table_4, spec_table_5, spec_table_6, spec_table_7};
-  for (Table f : tables) {
-    int count = 0;
-    const SpecOps* t = f(&count);
-    for (int q = 0; q < count; ++q)
-      if (t[q].n == n && t[q].prec == prec) return &t[q];
+  switch (n) {
+#define PDR_ROW(n) \
+  case n:          \
+    return prec ? spec_ops_f32_##n() : spec_ops_f64_##n();
+    PDR_SPEC_LENGTHS(PDR_ROW)
+#undef PDR_ROW
+    default:
+      return nullptr;
   }
-  return nullptr;
 }
 
 // Finds the passes of the box's three lengths; false: a length has none, or its

@@ -2,8 +2,8 @@
 // allocations come from malloc, copies are done in place, kernels and graphs are counted
 // and not run.  Loaded before the library (RTLD_GLOBAL), it takes the runtime's place, so
 // that the library's host code runs without a GPU and a test can make any call fail
-// (stand_in_fail), look at what was asked for (stand_in_count, stand_in_bytes) and have
-// two devices.  Streams and events belong to the device that was current when they were
+// (stand_in_fail), look at what was asked for (stand_in_count, stand_in_bytes,
+// stand_in_loaded_kernels) and have two devices.  Streams and events belong to the device that was current when they were
 // made; a launch or a record with another device current fails, as in the runtime.
 #include <cstdlib>
 #include <cstring>
@@ -30,6 +30,12 @@ std::map<std::string, long long> calls;
 std::map<std::string, std::pair<long long, int>> failures;  // call: fail from its n-th on, with this error
 std::unordered_map<void*, Block> blocks;
 size_t live[2] = {0, 0}, largest = 0;  // device, pinned
+struct Module {
+  int kernels = 0;
+  bool loaded = false;
+};
+std::unordered_map<const void*, Module*> kernels;
+long long loaded_kernels = 0;
 thread_local int current = 0;
 thread_local int last = 0;
 
@@ -73,6 +79,14 @@ int drop(void* h) {
   delete static_cast<Handle*>(h);
   return 0;
 }
+// a code object is loaded whole, at the first use of a kernel in it
+void load(const void* kernel) {
+  std::lock_guard<std::mutex> g(lock);
+  auto k = kernels.find(kernel);
+  if (k == kernels.end() || k->second->loaded) return;
+  k->second->loaded = true;
+  loaded_kernels += k->second->kernels;
+}
 int here(void* h) { return h && static_cast<Handle*>(h)->device != current ? done(kInvalidHandle) : 0; }
 
 }  // namespace
@@ -101,6 +115,7 @@ long long stand_in_bytes(int what) {  // 0 device, 1 pinned, 2 the largest devic
   return (long long)(what == 2 ? largest : live[what]);
 }
 int stand_in_device() { return current; }
+long long stand_in_loaded_kernels() { return loaded_kernels; }
 
 // the runtime's
 int hipGetDevice(int* d) {
@@ -236,12 +251,14 @@ int hipGraphDestroy(void* x) {
   ENTER("hipGraphDestroy");
   return drop(x);
 }
-int hipFuncSetAttribute(const void*, int, int) {
+int hipFuncSetAttribute(const void* f, int, int) {
   ENTER("hipFuncSetAttribute");
+  load(f);
   return 0;
 }
-int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
+int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int, size_t) {
   ENTER("hipOccupancyMaxActiveBlocksPerMultiprocessor");
+  load(f);
   *n = 2;
   return 0;
 }
@@ -264,9 +281,18 @@ int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* lds, void** s) {
   *s = pushed.stream;
   return 0;
 }
-int hipLaunchKernel(const void*, Dim3, Dim3, void**, size_t, void* s) {
+int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t, void* s) {
   ENTER("hipLaunchKernel");
+  load(f);
   return here(s);
 }
+void** __hipRegisterFatBinary(const void*) { return reinterpret_cast<void**>(new Module); }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void** m, const void* f, char*, const char*, unsigned, void*, void*, void*, void*, int*) {
+  std::lock_guard<std::mutex> g(lock);
+  kernels[f] = reinterpret_cast<Module*>(m);
+  ++kernels[f]->kernels;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 
 }  // extern "C"

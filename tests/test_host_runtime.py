@@ -17,6 +17,7 @@ S = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
 S.stand_in_fail.argtypes = [C.c_char_p, C.c_longlong, C.c_int]
 S.stand_in_count.argtypes, S.stand_in_count.restype = [C.c_char_p], C.c_longlong
 S.stand_in_bytes.argtypes, S.stand_in_bytes.restype = [C.c_int], C.c_longlong
+S.stand_in_loaded_kernels.restype = C.c_longlong
 sys.path.insert(0, {pkg!r})
 import numpy as np
 import pandora_amd as pa
@@ -133,4 +134,18 @@ def test_chunked_box_holds_a_chunk(stand_in, prec, mb, streams):
         assert zc == (max(1, min(n[2], {mb} * 1048576 // plane)) if chunked else n[2])
         g.close()
     assert size[True] == size[False] - (n[2] - {streams} * zc) * plane
+    """)
+
+
+@pytest.mark.parametrize("shape", [(32, 32, 32), (48, 48, 48), (64, 64, 64), (96, 96, 96), (256, 256, 256), (120, 48, 96)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_a_box_loads_the_code_of_its_lengths(stand_in, shape):
+    """The runtime loads a code object whole, some 60 us for each kernel in it, at the first
+    launch: the steps of a box load at most 32 kernels for each of its different lengths."""
+    _run(stand_in, f"""
+    n = {shape}
+    g = pa.Pandora(nx=n[0], ny=n[1], nz=n[2], precision=pa.PDR_FP32_MIXED)
+    g.run(1, 3, 0.0)
+    print(S.stand_in_loaded_kernels())
+    assert 0 < S.stand_in_loaded_kernels() <= 32 * len(set(n))
     """)
