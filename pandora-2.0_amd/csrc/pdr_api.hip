@@ -260,15 +260,26 @@ static void make_twiddles(int n, std::vector<unsigned char>& out) {
   }
 }
 
-static int upload_tw(pdr_ctx* c, int n, void** dst) {
-  std::vector<unsigned char> h;
-  if (c->prec)
-    make_twiddles<float>(n, h);
-  else
-    make_twiddles<double>(n, h);
-  HIPCHK(hipMalloc(dst, h.size()));
-  c->dev_bytes += h.size();
-  HIPCHK(hipMemcpy(*dst, h.data(), h.size(), hipMemcpyHostToDevice));
+// The twiddle tables of the three lengths, in one allocation and one copy (a copy waits
+// 13 us for the device: three were an eighth of a small box's creation).
+static int upload_tw(pdr_ctx* c) {
+  const int n[3] = {c->g.nz, c->g.ny, c->g.nx};
+  void** const at[3] = {&c->tab.twz, &c->tab.twy, &c->tab.twx};
+  size_t off[4] = {0, 0, 0, 0};
+  std::vector<unsigned char> all, h;
+  for (int q = 0; q < 3; ++q) {
+    if (c->prec)
+      make_twiddles<float>(n[q], h);
+    else
+      make_twiddles<double>(n[q], h);
+    off[q + 1] = off[q] + (h.size() + 255) / 256 * 256;
+    all.resize(off[q + 1]);
+    std::memcpy(all.data() + off[q], h.data(), h.size());
+  }
+  HIPCHK(hipMalloc(&c->tab.all, all.size()));
+  c->dev_bytes += all.size();
+  HIPCHK(hipMemcpy(c->tab.all, all.data(), all.size(), hipMemcpyHostToDevice));
+  for (int q = 0; q < 3; ++q) *at[q] = static_cast<char*>(c->tab.all) + off[q];
   return PDR_OK;
 }
 
@@ -325,9 +336,7 @@ int pdr_destroy(pdr_ctx* c) {
   if (c->stat_buf) (void)hipFree(c->stat_buf);
   if (c->rs_buf) (void)hipFree(c->rs_buf);
   stage_stats_free(c);
-  if (c->tab.twz) (void)hipFree(c->tab.twz);
-  if (c->tab.twy) (void)hipFree(c->tab.twy);
-  if (c->tab.twx) (void)hipFree(c->tab.twx);
+  if (c->tab.all) (void)hipFree(c->tab.all);
   for (auto& e : c->ev_pending) {
     (void)hipEventDestroy(e.second.first);
     (void)hipEventDestroy(e.second.second);
@@ -456,7 +465,8 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     const char* env = std::getenv("PDR_ZCHUNK_MB");
     double mb = env && env[0] ? std::atof(env) : 0.0;
     const double plane = 6.0 * double(ny) * double(g.ldi) * double(c->csz);
-    if (!(env && env[0])) {
+    if (!(env && env[0]) && plane * double(nz) > kZChunkMB * 1048576.0) {
+      // (a smaller box's chunk is the whole box: the query, 19 us, decides nothing there)
       // free device memory; if the query fails, the device's total memory
       size_t free_b = 0, total_b = 0;
       if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
@@ -513,9 +523,6 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
 
   int rc = PDR_OK;
   he = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-  if (he == hipSuccess) he = hipStreamCreateWithFlags(&c->tstream, hipStreamNonBlocking);
-  if (he == hipSuccess) he = hipEventCreateWithFlags(&c->ev_ur, hipEventDisableTiming);
-  if (he == hipSuccess) he = hipEventCreateWithFlags(&c->ev_tr, hipEventDisableTiming);
   if (he == hipSuccess && c->zs2) he = hipStreamCreateWithFlags(&c->zstream, hipStreamNonBlocking);
   if (he == hipSuccess && c->zs2) he = hipEventCreateWithFlags(&c->ev_za, hipEventDisableTiming);
   if (he == hipSuccess && c->zs2) he = hipEventCreateWithFlags(&c->ev_zb, hipEventDisableTiming);
@@ -551,9 +558,7 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     if (rc == PDR_OK && hipMemsetAsync(c->force, 0, fbytes, c->stream) != hipSuccess)
       rc = fail(PDR_ERR_HIP, "zeroing forcing failed");
   }
-  if (rc == PDR_OK) rc = upload_tw(c, nz, &c->tab.twz);
-  if (rc == PDR_OK) rc = upload_tw(c, ny, &c->tab.twy);
-  if (rc == PDR_OK) rc = upload_tw(c, nx, &c->tab.twx);
+  if (rc == PDR_OK) rc = upload_tw(c);
   if (rc == PDR_OK) {
     for (int q = 0; q < 3; ++q) {
       if (hipMemsetAsync(c->u[q], 0, wbytes, c->stream) != hipSuccess ||
@@ -718,7 +723,19 @@ static Coef next_coef(pdr_ctx* c, int stage, int32_t tstep, double tstart, doubl
 // (us a step, beside -> in line: 120 x 48 x 96 FP64 with 5000 tracers 239 -> 198, forced
 // 128^3 FP32-mixed with 16384 260 -> 248, with 60000 280 -> 262, forced 64^3 FP64 with
 // 60000 190 -> 149; but 256^3 FP64 with 60000 2504 -> 2519, whose passes leave the host time).
-static bool tracers_beside(const pdr_ctx* c) { return c->np >= (c->g.nr <= (1 << 22) ? 65536 : 16384); }
+static bool tracers_beside(const pdr_ctx* c, int64_t np) { return np >= (c->g.nr <= (1 << 22) ? 65536 : 16384); }
+
+// Their stream and events, at the first such tracers of a context (a stream costs 20 us to
+// make and 20 to destroy, of the 600 that a 32^3 box's creation, upload, step and end take).
+static int tracer_stream(pdr_ctx* c) {
+  const OnDevice on(c);
+  hipError_t e = c->tstream ? hipSuccess : hipStreamCreateWithFlags(&c->tstream, hipStreamNonBlocking);
+  for (hipEvent_t* ev : {&c->ev_ur, &c->ev_tr})
+    if (e == hipSuccess && !*ev) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
+  if (e == hipSuccess) return PDR_OK;
+  (void)hipGetLastError();  // later launch checks read it
+  return fail(PDR_ERR_HIP, std::string("tracer stream: ") + hipGetErrorString(e));
+}
 
 static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, StageLink* link);
 
@@ -852,7 +869,7 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
     // the advance reads the tracer field the x pass wrote and nothing the forward
     // passes touch: it runs on the tracer stream beside them, or where it is short
     // (tracers_beside) between them, which saves the two streams' waits
-    const bool beside = tracers_beside(c);
+    const bool beside = tracers_beside(c, c->np);
     const hipStream_t ts = beside ? c->tstream : c->stream;
     if (beside) {
       HIPCHK(hipEventRecord(c->ev_ur, c->stream));
@@ -881,7 +898,7 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
   }
   // and at the end of f_RK3SolveNavierStokes (src/pf_rk3.f90:2101-2109)
   HIPCHK(launch_dealias(c));
-  if (tracers && tracers_beside(c)) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_tr, 0));
+  if (tracers && tracers_beside(c, c->np)) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_tr, 0));
   link->z_ready = link->join;
   return PDR_OK;
 }
@@ -1076,6 +1093,10 @@ int pdr_particles_upload(pdr_ctx* c, const double* xp, int64_t np) {
   HIPCHK(hipMemset(c->up, 0, 24 * size_t(np)));
   // particle_xp0 = particle_xp at placement (src/pp_control.f90:405-407)
   if (c->xp0) HIPCHK(hipMemcpy(c->xp0, xp, 24 * size_t(np), hipMemcpyHostToDevice));
+  if (tracers_beside(c, np)) {
+    rc = tracer_stream(c);
+    if (rc != PDR_OK) return rc;
+  }
   c->np = np;
   c->since_sort = 0;
   if (c->sort_every > 0) {

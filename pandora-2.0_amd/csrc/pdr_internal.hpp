@@ -112,6 +112,7 @@ enum KernelClass {
 struct SpecOps;  // pdr_spec.hpp
 
 struct Tables {
+  void* all = nullptr;  // the three in one allocation
   void* twz = nullptr;
   void* twy = nullptr;
   void* twx = nullptr;
@@ -199,9 +200,9 @@ struct pdr_ctx {
   // first use: 0 not yet, -1 unknown)
   mutable int stats_resident = 0;
   hipStream_t stream = nullptr;
-  // the tracer advance runs on its own stream beside the forward passes of the
-  // stage: ev_ur orders it after the x pass that writes the tracer field,
-  // ev_tr orders the next stage after it
+  // a long tracer advance (tracers_beside) runs on its own stream beside the forward
+  // passes of the stage: ev_ur orders it after the x pass that writes the tracer field,
+  // ev_tr orders the next stage after it; made when such tracers are set
   hipStream_t tstream = nullptr;
   hipEvent_t ev_ur = nullptr;
   hipEvent_t ev_tr = nullptr;
