@@ -510,10 +510,22 @@ int pdr_debug_prepare(pdr_ctx* ctx, int32_t field, double* out);
  * specialised kernels, 0 = runtime-radix kernels; out[1] z planes per x-pencil
  * chunk (NZ = whole box); out[2] 1 = two chunks in flight on two streams;
  * out[3] 1 = fused z-forward + FormF kernel; with the specialised kernels
- * out[4] x rows per x-pass workgroup, out[5] 1 = x tile twiddles read from the
- * global table, out[6] 1 = register z inverse (velocity tile loaded once),
- * out[7] lines per z-inverse tile (0 for out[4..7] on the runtime-radix path). */
+ * out[4] x rows that a workgroup takes at a time (of the x pass, or of a part of
+ * a fused plane), out[5] 1 = x tile twiddles read from the global table, out[6]
+ * 1 = z inverse with the velocity tile loaded once and kept in registers (up to
+ * 512 points), out[7] lines per z-inverse tile (0 for out[4..7] on the
+ * runtime-radix path). */
 int pdr_kernel_forms(const pdr_ctx* ctx, int32_t out[8]);
+
+/* Which of the specialised passes this context's steps take together (no
+ * reference counterpart; as pdr_kernel_forms): out[0] workgroups that the parts
+ * of a z plane are spread over where its y and x passes run as one kernel (0 =
+ * separate passes), out[1] parts of such a plane; out[2] 1 = the stages inside
+ * pdr_step and pdr_run are joined, a stage's z forward pass doing the next
+ * one's z inverse; out[3] fields that go through the z inverse with the present
+ * frame (5: the y pass forms the last vorticity component; 6, also on the
+ * runtime-radix path; 18 in its NS_R_CONV). */
+int pdr_kernel_routes(const pdr_ctx* ctx, int32_t out[4]);
 
 /* Measured device copy bandwidth (read + write bytes per second, GB/s) of a
  * plain 16-byte-vector copy of `bytes` bytes, timed over `iters` launches.

@@ -301,6 +301,9 @@ static int dalloc(pdr_ctx* c, void** p, size_t bytes) {
   return PDR_OK;
 }
 
+// Short z lines, no truncation of the state between the stages.
+static bool stages_joined(const pdr_ctx* c) { return zz_fused(c) && c->p.dealiasing == PDR_DEALIASING_TWOTHIRD; }
+
 extern "C" {
 
 const char* pdr_version(void) { return "pandora-amd 0.1 (gfx950, HIP)"; }
@@ -600,6 +603,16 @@ int pdr_kernel_forms(const pdr_ctx* c, int32_t out[8]) {
   out[2] = c->zs2 ? 1 : 0;
   out[3] = (c->spec && c->fuse_zf) ? 1 : 0;
   for (int q = 0; q < 4; ++q) out[4 + q] = f[q];
+  return PDR_OK;
+}
+
+int pdr_kernel_routes(const pdr_ctx* c, int32_t out[4]) {
+  if (!c || !out) return fail(PDR_ERR_ARG, "pdr_kernel_routes: null argument");
+  const bool plane = plane_fused(c);
+  out[0] = plane ? c->nl_parts : 0;
+  out[1] = plane ? c->ops_x->plane_parts : 0;
+  out[2] = stages_joined(c) ? 1 : 0;
+  out[3] = conv_form(c) && !c->spec ? 18 : z5_fields(c, make_coef(c)) ? 5 : 6;
   return PDR_OK;
 }
 
@@ -1006,11 +1019,10 @@ int pdr_update_b(pdr_ctx* c, int32_t tstep, double simtime) {
 }
 
 // g_RK3Calc (src/pg_rk3.f90:82-129).  Its stages are joined where one kernel can end a
-// stage and start the next (short z lines, no truncation of the state between them);
-// more: so is the next step's first stage.
+// stage and start the next (stages_joined); more: so is the next step's first stage.
 static int step_run(pdr_ctx* c, int32_t tstep, double* simtime, StageLink* link, bool more) {
   const double tstart = *simtime;
-  const bool zz = zz_fused(c) && c->p.dealiasing == PDR_DEALIASING_TWOTHIRD;
+  const bool zz = stages_joined(c);
   link->tstart = tstart;
   link->join = zz;
   int rc = stage_run(c, 1, tstep, &c->dt, link);

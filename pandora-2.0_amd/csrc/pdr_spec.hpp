@@ -28,7 +28,7 @@ struct SpecOps {
   size_t lds_z, lds_y, lds_x, lds_xc;  // the largest workgroup of the z, y, x and NS_R_CONV x passes
   int xrows, xrows_conv;       // rows of an x tile
   int x_tw_global;             // 1: the x tile reads its twiddles from the global table
-  int zinv_register;           // 1: register z inverse
+  int zinv_register;           // 1: the velocity tile of a z inverse is kept in registers
   int zinv_lines;              // lines of a z inverse tile
 };
 

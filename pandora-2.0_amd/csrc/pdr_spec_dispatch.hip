@@ -25,11 +25,11 @@ bool spec_find(pdr_ctx* c) {
          c->ops_z->lds_z <= c->lds_max;
 }
 
-// Forms the passes of this box take (pdr_kernel_forms): x rows per x-pass
-// workgroup, 1 if the x tile reads its twiddles from the global table, 1 for the
-// register z inverse (velocity tile loaded once), lines per z-inverse tile.
+// Forms the passes of this box take (pdr_kernel_forms): x rows that a workgroup takes
+// at a time, 1 if the x tile reads its twiddles from the global table, 1 for a z inverse
+// with the velocity tile in registers, lines per z-inverse tile.
 void spec_forms(const pdr_ctx* c, int out[4]) {
-  out[0] = conv_form(c) ? c->ops_x->xrows_conv : c->ops_x->xrows;
+  out[0] = conv_form(c) ? c->ops_x->xrows_conv : plane_fused(c) ? c->g.ny / c->ops_x->plane_parts : c->ops_x->xrows;
   out[1] = c->ops_x->x_tw_global;
   out[2] = c->ops_z->zinv_register;
   out[3] = c->ops_z->zinv_lines;

@@ -155,6 +155,7 @@ def load_library(path: str = LIB_PATH):
         "pdr_spectrum": (C.c_int, [vp, dp, dp, dp, dp]),
         "pdr_debug_prepare": (C.c_int, [vp, i32, dp]),
         "pdr_kernel_forms": (C.c_int, [vp, np.ctypeslib.ndpointer(dtype=np.int32)]),
+        "pdr_kernel_routes": (C.c_int, [vp, np.ctypeslib.ndpointer(dtype=np.int32)]),
         "pdr_profile_enable": (C.c_int, [vp, i32]),
         "pdr_copy_bandwidth": (C.c_int, [i64, i32, C.POINTER(d)]),
         "pdr_hbm_probe": (C.c_int, [i32, i64, i32, C.POINTER(d)]),
@@ -584,6 +585,12 @@ class Pandora:
         keys = ("specialised", "zchunk", "two_chunks", "fused_zformf", "xrows", "x_tw_global",
                 "zinv_register", "zinv_lines")
         return dict(zip(keys, (int(v) for v in out)))
+
+    def kernel_routes(self):
+        """Which passes this box's steps take together (pdr_kernel_routes) as a dict."""
+        out = np.zeros(4, dtype=np.int32)
+        _check(self.L.pdr_kernel_routes(self.h, out))
+        return dict(zip(("plane_groups", "plane_parts", "joined", "z_fields"), (int(v) for v in out)))
 
     def debug_prepare(self, field: int):
         out = np.zeros((self.nki, self.nz, self.nkj), np.complex128)

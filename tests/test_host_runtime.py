@@ -181,3 +181,48 @@ def test_what_a_small_box_is_made_of(stand_in):
     assert S.stand_in_bytes(0) == 0 and S.stand_in_bytes(1) == 0
     assert count("hipStreamCreateWithFlags") == count("hipStreamDestroy")
     """)
+
+
+def test_routes_of_a_box(stand_in):
+    """pdr_kernel_routes and the x rows of pdr_kernel_forms where the rules change: the length that
+    fused planes end at, the groups that a plane's parts are spread over, joined stages (none with
+    a truncation of the state), five fields through z (not with a frame that puts k3 into the last
+    vorticity component, nor with the y pass's fields split), chunks, the runtime-radix kernels."""
+    _run(stand_in, """
+    F64, F32 = pa.PDR_FP64, pa.PDR_FP32_MIXED
+    def routes(nx, ny, nz, prec, **kw):
+        with pa.Pandora(nx=nx, ny=ny, nz=nz, precision=prec, **kw) as g:
+            return tuple(g.kernel_routes().values()) + (g.kernel_forms()["xrows"],)
+    sheared = dict(f_type=2, rk3_timestep=1, deform_s=1.0, remesh_t=4)
+    # groups, parts, joined, fields through z, x rows
+    for args, kw, want in [
+        ((32, 32, 32, F64), {}, (4, 4, 1, 6, 8)),
+        ((64, 64, 64, F64), {}, (4, 4, 1, 6, 16)),
+        ((30, 30, 30, F64), {}, (1, 1, 1, 6, 30)),
+        ((72, 72, 72, F64), {}, (0, 0, 1, 6, 8)),
+        ((64, 64, 96, F64), {}, (3, 4, 1, 6, 16)),
+        ((64, 64, 128, F64), {}, (2, 4, 0, 6, 16)),
+        ((64, 64, 128, F32), {}, (2, 4, 1, 6, 16)),
+        ((64, 64, 256, F64), {}, (1, 4, 0, 6, 16)),
+        ((64, 64, 640, F64), {}, (1, 4, 0, 6, 16)),
+        ((24, 24, 256, F64), {}, (1, 1, 0, 6, 24)),
+        ((64, 60, 64, F64), {}, (0, 0, 1, 6, 16)),
+        ((32, 32, 32, F64), dict(dealiasing=2), (4, 4, 0, 6, 8)),
+        ((32, 32, 32, F64), dict(sheared, ns_deformed=2), (0, 0, 0, 6, 8)),
+        ((50, 50, 50, F64), {}, (0, 0, 0, 6, 0)),
+        ((50, 50, 50, F64), dict(sheared, ns_deformed=2), (0, 0, 0, 18, 0)),
+        ((256, 256, 256, F64), {}, (0, 0, 0, 5, 2)),
+        ((128, 24, 384, F32), sheared, (0, 0, 0, 5, 4)),
+        ((128, 24, 384, F32), dict(sheared, ns_deformed=3), (0, 0, 0, 5, 4)),
+        ((128, 24, 128, F64), sheared, (0, 0, 0, 6, 4)),
+    ]:
+        assert routes(*args, **kw) == want, (args, kw, routes(*args, **kw), want)
+    with pa.Pandora(nx=128, ny=24, nz=384, ns_deformed=3, **sheared) as g:
+        assert g.kernel_routes()["z_fields"] == 5
+        b = np.eye(3)
+        b[2, 0] = 0.25
+        g.set_frame(b.T, np.eye(3))
+        assert g.kernel_routes()["z_fields"] == 6
+    os.environ["PDR_ZCHUNK_MB"] = "0.3"
+    assert routes(32, 32, 32, F64) == (0, 0, 1, 6, 16)
+    """)
