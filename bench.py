@@ -33,12 +33,16 @@ def model_bytes_per_step(g, csz, rsz, ntr):
     return 3 * ((15 * g.mw + 18 * g.m1) * csz + (96 * ntr + 3 * n3 * rsz if ntr else 0))
 
 
-def kernel_bytes(g, name, csz, rsz, ntr):
-    """Compulsory bytes one launch of each kernel must move (its inputs + outputs)."""
+class Profile(dict):
+    """Launches and milliseconds of each kernel, and the fields that the z inverse transformed."""
+    z_fields = 6
+
+
+def kernel_bytes(g, name, csz, rsz, ntr, zf=6):
+    """Compulsory bytes one launch of each kernel must move (its inputs + outputs); zf fields
+    go through the z inverse."""
     m2 = g.nz * g.ny * g.nki
     n3 = g.nx * g.ny * g.nz
-    # large boxes: the y inverse forms the last vorticity component itself
-    zf = 5 if g.nz > 128 and (g.nki + 15) // 16 * g.nz >= 1024 else 6
     return {
         "zinv": (3 * g.mw + zf * g.m1) * csz,
         "yinv": (zf * g.m1 + 6 * m2) * csz,
@@ -77,7 +81,8 @@ def run_gpu(pa, n, precision, steps, warmup, ntr, profile):
     t = g.run(1 + warmup, steps, t)
     g.synchronize()
     t1 = time.perf_counter()
-    prof = g.profile_get() if profile else {}
+    prof = Profile(g.profile_get() if profile else {})
+    prof.z_fields = g.kernel_routes()["z_fields"]
     ok = g.check_finite()
     g.close()
     return (t1 - t0), prof, ok
@@ -649,7 +654,7 @@ def main():
     g.m1 = g.nki * g.nkj * n
     dom, best = None, -1.0
     for k, (cnt, ms) in prof.items():
-        if cnt and ms > best and kernel_bytes(g, k, 8, 4, ntr):
+        if cnt and ms > best and kernel_bytes(g, k, 8, 4, ntr, prof.z_fields):
             dom, best = k, ms
     roof = None
 
@@ -657,7 +662,7 @@ def main():
         out = {}
         for k, (cnt, ms) in pr.items():
             if cnt:
-                b = kernel_bytes(g, k, csz, rsz, ntr)
+                b = kernel_bytes(g, k, csz, rsz, ntr, pr.z_fields)
                 ch = chunks_per_stage(k, cnt, nsteps)
                 if b:
                     b /= ch
@@ -672,7 +677,7 @@ def main():
         cnt, ms = prof[dom]
         avg = ms / cnt * 1e-3
         ch = chunks_per_stage(dom, cnt, rsteps)
-        b = kernel_bytes(g, dom, 8, 4, ntr) / ch
+        b = kernel_bytes(g, dom, 8, 4, ntr, prof.z_fields) / ch
         traffic = measured_traffic(dom, n, ntr)
         if traffic:
             traffic /= ch

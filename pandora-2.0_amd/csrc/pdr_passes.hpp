@@ -535,26 +535,21 @@ __device__ __forceinline__ void k2_yinv_body(unsigned bid, const Geo& g, const c
         if ((EM % YT == 0 || e < EM) && i0 + line < nki) v = get<kNrYinv>(&src[line * lstride + (e - line * NKJ)]);
         pre[q] = DY && f >= 6 ? mul_ik<T>(v, e - line * NKJ, K) : v;
       }
-      return;
-    }
+    } else {
 #pragma unroll
-    for (int q = 0; q < QE; ++q) {
-      const int idx = int(threadIdx.x) + YT * q;
-      const int line = idx / N;
-      const int y = idx - line * N;
-      const int j = (y <= K) ? y : ((y >= N - K) ? y - (N - NKJ) : -1);
-      cx<T> v = czero<T>();
-      if constexpr (PP > 0) {
+      for (int q = 0; q < QE; ++q) {
+        const int idx = int(threadIdx.x) + YT * q;
+        const int line = idx / N;
+        const int y = idx - line * N;
+        const int j = (y <= K) ? y : ((y >= N - K) ? y - (N - NKJ) : -1);
         const int p = line / (K + 1);
         const int i = line - p * (K + 1);
         const int zz = tile * PP + p;
+        cx<T> v = czero<T>();
         if ((L * N % YT == 0 || idx < L * N) && zz < nzc && j >= 0)
           v = get<kNrYinv>(&src[((long long)i * g.nz + zz) * g.ldj + j]);
-      } else {
-        if ((L * N % YT == 0 || idx < L * N) && i0 + line < nki && j >= 0)
-          v = get<kNrYinv>(&src[line * lstride + j]);
+        pre[q] = DY && f >= 6 ? mul_ik<T>(v, j, K) : v;
       }
-      pre[q] = DY && f >= 6 ? mul_ik<T>(v, j, K) : v;
     }
   };
   static_assert(!W3 || (PP == 0 && !DY), "W3 is a form of the tiles of i-lines");
