@@ -313,7 +313,7 @@ const char* pdr_last_error(void) { return g_err.c_str(); }
 int pdr_destroy(pdr_ctx* c) {
   if (!c) return PDR_OK;
   // every stream of the context, before any buffer is freed
-  for (hipStream_t s : {c->stream, c->zstream, c->tstream})
+  for (hipStream_t s : {c->stream, c->zstream})
     if (s) (void)hipStreamSynchronize(s);
   for (int q = 0; q < 3; ++q) {
     if (c->u[q]) (void)hipFree(c->u[q]);
@@ -345,12 +345,9 @@ int pdr_destroy(pdr_ctx* c) {
     (void)hipEventDestroy(e.second.second);
   }
   for (auto& e : c->ev_pool) (void)hipEventDestroy(e);
-  if (c->ev_ur) (void)hipEventDestroy(c->ev_ur);
-  if (c->ev_tr) (void)hipEventDestroy(c->ev_tr);
   if (c->ev_za) (void)hipEventDestroy(c->ev_za);
   if (c->ev_zb) (void)hipEventDestroy(c->ev_zb);
   if (c->zstream) (void)hipStreamDestroy(c->zstream);
-  if (c->tstream) (void)hipStreamDestroy(c->tstream);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return PDR_OK;
@@ -731,25 +728,6 @@ static Coef next_coef(pdr_ctx* c, int stage, int32_t tstep, double tstart, doubl
   return f;
 }
 
-// Whether the advance is long enough for a stream of its own.  A short one is about what the
-// two waits between streams cost the device, and their four event calls hold up the host
-// (us a step, beside -> in line: 120 x 48 x 96 FP64 with 5000 tracers 239 -> 198, forced
-// 128^3 FP32-mixed with 16384 260 -> 248, with 60000 280 -> 262, forced 64^3 FP64 with
-// 60000 190 -> 149; but 256^3 FP64 with 60000 2504 -> 2519, whose passes leave the host time).
-static bool tracers_beside(const pdr_ctx* c, int64_t np) { return np >= (c->g.nr <= (1 << 22) ? 65536 : 16384); }
-
-// Their stream and events, at the first such tracers of a context (a stream costs 20 us to
-// make and 20 to destroy, of the 600 that a 32^3 box's creation, upload, step and end take).
-static int tracer_stream(pdr_ctx* c) {
-  const OnDevice on(c);
-  hipError_t e = c->tstream ? hipSuccess : hipStreamCreateWithFlags(&c->tstream, hipStreamNonBlocking);
-  for (hipEvent_t* ev : {&c->ev_ur, &c->ev_tr})
-    if (e == hipSuccess && !*ev) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
-  if (e == hipSuccess) return PDR_OK;
-  (void)hipGetLastError();  // later launch checks read it
-  return fail(PDR_ERR_HIP, std::string("tracer stream: ") + hipGetErrorString(e));
-}
-
 static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, StageLink* link);
 
 int pdr_stage(pdr_ctx* c, int32_t stage, int32_t tstep, double time, double* dt) {
@@ -879,19 +857,16 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
   rk_coeffs(stage, &beta, &gamma);
   const double gdt = gamma * (*dt);
   if (tracers) {
-    // the advance reads the tracer field the x pass wrote and nothing the forward
-    // passes touch: it runs on the tracer stream beside them, or where it is short
-    // (tracers_beside) between them, which saves the two streams' waits
-    const bool beside = tracers_beside(c, c->np);
-    const hipStream_t ts = beside ? c->tstream : c->stream;
-    if (beside) {
-      HIPCHK(hipEventRecord(c->ev_ur, c->stream));
-      HIPCHK(hipStreamWaitEvent(c->tstream, c->ev_ur, 0));
-    }
-    if (stage == 1 && tstep == c->ts_release) HIPCHK(tracers_release(c, ts));
-    HIPCHK(launch_tracers(c, c->tf_ur, beta, gdt, ts));
-    if (pstats) HIPCHK(launch_pstats_rel(c, tstep, ts));
-    if (beside) HIPCHK(hipEventRecord(c->ev_tr, c->tstream));
+    // the advance reads the tracer field the x pass wrote and nothing the forward passes
+    // touch, but on a stream of its own beside them it takes the device longer than between
+    // them: both are bound by the memory system, and each stage pays two waits (us a step,
+    // beside -> between: 64^3 FP64 with 65536 tracers 178 -> 152, 128^3 FP64 with 262144
+    // 549 -> 503, 256^3 FP64 with 262144 2711 -> 2684, 512^3 FP32-mixed with 1048576
+    // 10548 -> 10509, 512^3 FP64 20934 -> 20928, 1024^3 FP32-mixed with 16777216
+    // 103854 -> 103883)
+    if (stage == 1 && tstep == c->ts_release) HIPCHK(tracers_release(c, c->stream));
+    HIPCHK(launch_tracers(c, c->tf_ur, beta, gdt, c->stream));
+    if (pstats) HIPCHK(launch_pstats_rel(c, tstep, c->stream));
   } else if (pstats && !field) {
     HIPCHK(launch_pstats_rel(c, tstep, c->stream));
   }
@@ -911,7 +886,6 @@ static int stage_run(pdr_ctx* c, int32_t stage, int32_t tstep, double* dt, Stage
   }
   // and at the end of f_RK3SolveNavierStokes (src/pf_rk3.f90:2101-2109)
   HIPCHK(launch_dealias(c));
-  if (tracers && tracers_beside(c, c->np)) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_tr, 0));
   link->z_ready = link->join;
   return PDR_OK;
 }
@@ -1105,10 +1079,6 @@ int pdr_particles_upload(pdr_ctx* c, const double* xp, int64_t np) {
   HIPCHK(hipMemset(c->up, 0, 24 * size_t(np)));
   // particle_xp0 = particle_xp at placement (src/pp_control.f90:405-407)
   if (c->xp0) HIPCHK(hipMemcpy(c->xp0, xp, 24 * size_t(np), hipMemcpyHostToDevice));
-  if (tracers_beside(c, np)) {
-    rc = tracer_stream(c);
-    if (rc != PDR_OK) return rc;
-  }
   c->np = np;
   c->since_sort = 0;
   if (c->sort_every > 0) {

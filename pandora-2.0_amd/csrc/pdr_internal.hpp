@@ -200,12 +200,6 @@ struct pdr_ctx {
   // first use: 0 not yet, -1 unknown)
   mutable int stats_resident = 0;
   hipStream_t stream = nullptr;
-  // a long tracer advance (tracers_beside) runs on its own stream beside the forward
-  // passes of the stage: ev_ur orders it after the x pass that writes the tracer field,
-  // ev_tr orders the next stage after it; made when such tracers are set
-  hipStream_t tstream = nullptr;
-  hipEvent_t ev_ur = nullptr;
-  hipEvent_t ev_tr = nullptr;
   // two z chunks in flight (nz >= 512 unchunked, or PDR_ZSTREAMS=2): odd chunks run their
   // y/x/y passes on zstream with their own x-pencil buffer w2z, beside the even ones
   bool zs2 = false;
