@@ -106,16 +106,17 @@ constexpr int y_lines_fwd(int n) {
 }
 
 // Short lines take more rows per workgroup, so that a workgroup still moves
-// about a thousand points (2 rows of 512; 16 rows of 64).  Half of that where it leaves
-// three quarters of the threads a butterfly in every pass and the CU more workgroups at
-// different phases (us a launch, 8 -> 4 rows at 128^3: FP64 39.8 -> 36.4, FP32-mixed
-// 26.3 -> 24.2; 4 -> 2 rows at 256^3: FP64 300 -> 256, FP32-mixed 129.9 / 128.6; but at
-// 160^3 FP32-mixed 42.8 -> 47.8, 192^3 65.7 -> 75.1, 240^3 FP64 251.7 -> 262.4).
+// about a thousand points (2 rows of 512; 16 rows of 64), and then fewer as soon as the CU
+// gains more by workgroups at different phases than it loses by threads without a
+// butterfly (us a launch, 8 -> 4 rows at 128^3: FP64 39.8 -> 36.4, FP32-mixed 26.3 -> 24.2;
+// 4 -> 2 rows in FP64 at 250^3 362 -> 321, 256^3 300 -> 256, but 240^3 253 -> 264, and at
+// 150^3 to 216^3, where two rows take 0 to 10 % off the pass, the moments no longer fit the
+// tile for their reduction: 216^3 194 -> 184, pdr_rs_stats 548 -> 580; FP32-mixed 160^3
+// 42.8 -> 47.8, 192^3 65.7 -> 75.1, 256^3 129.9 / 128.6).
 template <typename T>
 constexpr int xrows(int n) {
-  if (sizeof(T) == 8 && n > 144 && n <= 256 && (n & (n - 1)) == 0) return 2;
-  return n <= 64 ? 16 : (n <= 96 ? 8 : n <= 144 ? 4 : (n <= 256 ? 4 : (sizeof(T) == 4 ? (n <= 512 ? PDR_XROWS_F32 : 2)
-                                                                        : (n <= 512 ? PDR_XROWS_F64 : 2))));
+  constexpr bool f32 = sizeof(T) == 4;
+  return n <= 64 ? 16 : n <= 96 ? 8 : n <= (f32 ? 256 : 240) ? 4 : n <= 512 ? (f32 ? PDR_XROWS_F32 : PDR_XROWS_F64) : 2;
 }
 
 // LDS bytes of a workgroup, and the waves per SIMD that the 160 KB of LDS of a
