@@ -300,7 +300,7 @@ hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf);
 hipError_t launch2_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc);
 bool z5_fields(const pdr_ctx* c, const Coef& cf);
 hipError_t launch2_xpass(pdr_ctx* c, const Coef& cf, bool tracers, bool cfl, int z0, int nzc, double* rsp);
-int xpass_tiles(const pdr_ctx* c);  // x-pass workgroups per z plane (specialised path)
+int xpass_tiles(const pdr_ctx* c);  // workgroups per z plane of the x pass with moments (specialised path)
 Coef make_coef(const pdr_ctx* c);
 // Rogallo shear run, NS_R_ROT or NS_R_CONV (state = laboratory velocity on the
 // sheared grid; the two share FormF, remesh, tracer and statistics forms)

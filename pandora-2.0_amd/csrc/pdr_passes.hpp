@@ -109,13 +109,16 @@ constexpr int y_lines_fwd(int n) {
 // about a thousand points (2 rows of 512; 16 rows of 64), and then fewer as soon as the CU
 // gains more by workgroups at different phases than it loses by threads without a
 // butterfly (us a launch, 8 -> 4 rows at 128^3: FP64 39.8 -> 36.4, FP32-mixed 26.3 -> 24.2;
-// 4 -> 2 rows in FP64 at 250^3 362 -> 321, 256^3 300 -> 256, but 240^3 253 -> 264, and at
-// 150^3 to 216^3, where two rows take 0 to 10 % off the pass, the moments no longer fit the
-// tile for their reduction: 216^3 194 -> 184, pdr_rs_stats 548 -> 580; FP32-mixed 160^3
-// 42.8 -> 47.8, 192^3 65.7 -> 75.1, 256^3 129.9 / 128.6).
-template <typename T>
+// 4 -> 2 rows in FP64 at 250^3 362 -> 321, 256^3 300 -> 256, but 240^3 253 -> 264;
+// FP32-mixed 160^3 42.8 -> 47.8, 192^3 65.7 -> 75.1, 256^3 129.9 / 128.6).
+// With the moments (RS) the tile keeps the rows where it then holds the threads' sums for
+// their reduction (us a call of pdr_rs_stats, rows as above -> kept: 100^3 FP64 109 -> 101,
+// FP32-mixed 91 -> 81, 128^3 138 -> 130 and 101 -> 86, 144^3 FP32-mixed 167 -> 158, 256^3
+// FP64 724 -> 716; but 144^3 FP64, two tiles of eight rows to a CU, 207 -> 210).
+template <typename T, bool RS = false>
 constexpr int xrows(int n) {
   constexpr bool f32 = sizeof(T) == 4;
+  if (RS && n > 96 && n <= 256) return n <= (f32 ? 144 : 128) ? 8 : 4;
   return n <= 64 ? 16 : n <= 96 ? 8 : n <= (f32 ? 256 : 240) ? 4 : n <= 512 ? (f32 ? PDR_XROWS_F32 : PDR_XROWS_F64) : 2;
 }
 
@@ -150,9 +153,9 @@ constexpr int lds_yf_bytes(int n) {
 #endif
 template <typename T>
 constexpr bool x_tw_global(int n) { return n > PDR_X_TWG_MIN; }
-template <typename T>
+template <typename T, bool RS = false>
 constexpr int lds_x_bytes(int n) {
-  return ((x_tw_global<T>(n) ? 0 : n) + 3 * xrows<T>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>)) +
+  return ((x_tw_global<T>(n) ? 0 : n) + 3 * xrows<T, RS>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>)) +
          (kBlock2 / 64) * int(sizeof(T));
 }
 // Threads of the x pass: 512 for the tiles of which the CU's LDS holds fewer than four (FP64
@@ -166,7 +169,7 @@ constexpr int xthreads(int n) {
 }
 template <typename T, int RS>
 constexpr int xwaves(int n) {
-  return (kLdsPerCu / lds_x_bytes<T>(n) < 2 ? 1 : 2) * (xthreads<T, RS>(n) / kBlock2);
+  return (kLdsPerCu / lds_x_bytes<T, RS != 0>(n) < 2 ? 1 : 2) * (xthreads<T, RS>(n) / kBlock2);
 }
 // Streaming (non-temporal) stores per kernel, bit mask: 1 zinv, 2 yinv,
 // 4 xpass, 8 yfwd, 16 zfwd.  Every pass writes data that only the next pass
@@ -690,7 +693,7 @@ template <typename T, int N, int RS, int XT = kBlock2>
 __device__ __forceinline__ void k2_xpass_body(unsigned bid, const Geo& g, const Coef& cf, cx<T>* __restrict__ w2, T* __restrict__ ur, int want_tr, int want_cfl,
              unsigned long long* __restrict__ umax, const cx<T>* __restrict__ twg, int ntile, int z0,
              double* __restrict__ rsp) {
-  constexpr int RB = xrows<T>(N);
+  constexpr int RB = xrows<T, RS != 0>(N);
   constexpr int LD = lds_ld<T>(N);
   constexpr int KI = N / 3;
   constexpr int NKI = KI + 1;
@@ -1377,9 +1380,9 @@ size_t lds_y() {
     m = size_t(b) > m ? size_t(b) : m;
   return m;
 }
-template <typename T, int N>
+template <typename T, int N, bool RS = false>
 size_t lds_x() {
-  return size_t(lds_x_bytes<T>(N) - (kBlock2 / 64) * int(sizeof(T)));  // dynamic part
+  return size_t(lds_x_bytes<T, RS>(N) - (kBlock2 / 64) * int(sizeof(T)));  // dynamic part
 }
 
 hipError_t big_lds(const void* fn, size_t bytes) {
@@ -1469,11 +1472,11 @@ inline bool rs_fp32_box(const Geo& g) {
 template <typename T, int N>
 hipError_t xpass_n(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, int z0, int nzc, double* rsp) {
   const Geo& g = c->g;
-  constexpr int RB = xrows<T>(N);
-  const int nt = (g.ny + RB - 1) / RB;
-  const size_t lds = lds_x<T, N>();
   auto launch = [&](auto rs_c) -> hipError_t {
     constexpr int RS = decltype(rs_c)::value;
+    constexpr int RB = xrows<T, RS != 0>(N);
+    const int nt = (g.ny + RB - 1) / RB;
+    const size_t lds = lds_x<T, N, RS != 0>();
     hipError_t e = big_lds((const void*)k2_xpass<T, N, RS>, lds);
     if (e != hipSuccess) return e;
     k2_xpass<T, N, RS><<<dim3(unsigned(nt * nzc)), xthreads<T, RS>(N), lds, c->stream>>>(

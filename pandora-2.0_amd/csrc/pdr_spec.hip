@@ -44,9 +44,10 @@ SpecOps ops_of() {
   o.lds_plane = parts ? size_t(plane_lds_bytes<T>(N, parts) + plane_static_bytes<T>(N, parts)) : 0;
   o.lds_z = lds_lines<T, N>() > lds_fwd<T, N>() ? lds_lines<T, N>() : lds_fwd<T, N>();
   o.lds_y = lds_y<T, N>();
-  o.lds_x = lds_x<T, N>();
+  o.lds_x = lds_x<T, N>() > lds_x<T, N, true>() ? lds_x<T, N>() : lds_x<T, N, true>();
   o.lds_xc = size_t(lds_xc_bytes<T>(N));
   o.xrows = xrows<T>(N);
+  o.xrows_rs = xrows<T, true>(N);
   o.xrows_conv = xrows_conv<T>(N);
   o.x_tw_global = x_tw_global<T>(N) ? 1 : 0;
   constexpr bool reg = PDR_ZINV_REG && N <= 512;

@@ -26,7 +26,7 @@ struct SpecOps {
   size_t lds_plane;  // the kernel's own arrays included
   int plane_parts;
   size_t lds_z, lds_y, lds_x, lds_xc;  // the largest workgroup of the z, y, x and NS_R_CONV x passes
-  int xrows, xrows_conv;       // rows of an x tile
+  int xrows, xrows_rs, xrows_conv;  // rows of an x tile; with the moments; NS_R_CONV
   int x_tw_global;             // 1: the x tile reads its twiddles from the global table
   int zinv_register;           // 1: the velocity tile of a z inverse is kept in registers
   int zinv_lines;              // lines of a z inverse tile

@@ -50,7 +50,7 @@ hipError_t launch2_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* 
 // rows of moment partials per z plane: x-pass workgroups, or the parts of a fused plane
 int xpass_tiles(const pdr_ctx* c) {
   if (plane_fused(c)) return c->ops_x->plane_parts;
-  const int rb = conv_form(c) ? c->ops_x->xrows_conv : c->ops_x->xrows;
+  const int rb = conv_form(c) ? c->ops_x->xrows_conv : c->ops_x->xrows_rs;
   return (c->g.ny + rb - 1) / rb;
 }
 
