@@ -192,6 +192,7 @@ struct pdr_ctx {
   // launch shapes
   bool spec = false;  // length-specialised kernels (pdr_passes.hpp)
   const pdr::SpecOps *ops_x = nullptr, *ops_y = nullptr, *ops_z = nullptr;  // theirs for this box
+  bool zall = false;  // z passes with every field of a tile at once (SpecOps::zall_inv)
   bool plane_separate = false;  // y and x passes asked for as separate launches (PDR_ZCHUNK_MB or PDR_ZSTREAMS set)
   bool fuse_zf = true;  // fused z-forward + FormF (specialised path; PDR_FUSE_ZFORMF=0 disables)
   int tj_z = 1, ti_y = 1;

@@ -1544,7 +1544,7 @@ hipError_t zfwd_n(pdr_ctx* c) {
 }
 
 template <typename T, int N>
-hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, const Coef*, double beta, double gdt) {
+hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
   if constexpr (N > 512) {  // not used above 512 points per line (see pdr_create)
     return hipErrorNotSupported;
   } else {

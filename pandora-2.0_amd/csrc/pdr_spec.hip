@@ -30,14 +30,16 @@ SpecOps ops_of() {
   o.xpass = xpass_n<T, N>;
   o.yfwd = yfwd_n<T, N>;
   o.zfwd = zfwd_n<T, N>;
-  o.zz = zall_lines<T>(N) > 0;
+  o.zinv = zinv_n<T, N>;
+  o.zfwd_formf = zfwd_formf_n<T, N>;
+  o.zall_inv = nullptr;
+  o.zall_fwd = nullptr;
   if constexpr (zall_lines<T>(N) > 0) {
-    o.zinv = zall_inv_n<T, N>;
-    o.zfwd_formf = zall_fwd_n<T, N>;
-  } else {
-    o.zinv = zinv_n<T, N>;
-    o.zfwd_formf = zfwd_formf_n<T, N>;
+    o.zall_inv = zall_inv_n<T, N>;
+    o.zall_fwd = zall_fwd_n<T, N>;
   }
+  o.zall_most = zall_most<T>(N);
+  o.zall_lines = zall_lines<T>(N);
   constexpr int parts = plane_parts_box<T>(N);
   o.plane = parts ? plane_n<T, N> : nullptr;
   o.plane_parts = parts;
@@ -52,7 +54,7 @@ SpecOps ops_of() {
   o.x_tw_global = x_tw_global<T>(N) ? 1 : 0;
   constexpr bool reg = PDR_ZINV_REG && N <= 512;
   o.zinv_register = reg ? 1 : 0;
-  o.zinv_lines = zall_lines<T>(N) ? zall_lines<T>(N) : reg ? zinv_lines_t<T, PDR_ZINV_THREADS>(N) : tile_lines<T>(N);
+  o.zinv_lines = reg ? zinv_lines_t<T, PDR_ZINV_THREADS>(N) : tile_lines<T>(N);
   return o;
 }
 

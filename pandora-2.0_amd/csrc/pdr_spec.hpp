@@ -17,10 +17,13 @@ struct SpecOps {
   hipError_t (*xpass_conv)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
   hipError_t (*yfwd)(pdr_ctx*, int z0, int nzc);
   hipError_t (*zfwd)(pdr_ctx*);
-  // next: the operator of the stage that follows, whose inverse z pass is then done in the
-  // same kernel; only where zz is true, else null
-  hipError_t (*zfwd_formf)(pdr_ctx*, const Coef&, const Coef* next, double beta, double gdt);
-  bool zz;
+  hipError_t (*zfwd_formf)(pdr_ctx*, const Coef&, double beta, double gdt);
+  // the z passes of short lines with every field of a tile in LDS (pdr_zall.hpp), null where
+  // there are none; next: the operator of the stage that follows, whose inverse z pass is
+  // then done in the same kernel, or null
+  hipError_t (*zall_inv)(pdr_ctx*, const Coef&);
+  hipError_t (*zall_fwd)(pdr_ctx*, const Coef&, const Coef* next, double beta, double gdt);
+  long long zall_most;  // most z lines of a box that runs them
   // passes 2 to 4 of n x n planes in one launch (pdr_plane.hpp), null where they do not fit
   hipError_t (*plane)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
   size_t lds_plane;  // the kernel's own arrays included
@@ -29,7 +32,7 @@ struct SpecOps {
   int xrows, xrows_rs, xrows_conv;  // rows of an x tile; with the moments; NS_R_CONV
   int x_tw_global;             // 1: the x tile reads its twiddles from the global table
   int zinv_register;           // 1: the velocity tile of a z inverse is kept in registers
-  int zinv_lines;              // lines of a z inverse tile
+  int zinv_lines, zall_lines;  // lines of a z inverse tile
 };
 
 // The specialised path of a line length, or null (pdr_spec_dispatch.hip).

@@ -21,6 +21,7 @@ bool spec_find(pdr_ctx* c) {
   c->ops_x = spec_ops(c->prec, c->g.nx);
   c->ops_y = spec_ops(c->prec, c->g.ny);
   c->ops_z = spec_ops(c->prec, c->g.nz);
+  c->zall = c->ops_z && c->ops_z->zall_inv && (long long)c->g.nki * c->g.nkj <= c->ops_z->zall_most;
   return c->ops_x && c->ops_y && c->ops_z && (conv_form(c) ? c->ops_x->lds_xc : c->ops_x->lds_x) <= c->lds_max && c->ops_y->lds_y <= c->lds_max &&
          c->ops_z->lds_z <= c->lds_max;
 }
@@ -32,7 +33,7 @@ void spec_forms(const pdr_ctx* c, int out[4]) {
   out[0] = conv_form(c) ? c->ops_x->xrows_conv : plane_fused(c) ? c->g.ny / c->ops_x->plane_parts : c->ops_x->xrows;
   out[1] = c->ops_x->x_tw_global;
   out[2] = c->ops_z->zinv_register;
-  out[3] = c->ops_z->zinv_lines;
+  out[3] = c->zall ? c->ops_z->zall_lines : c->ops_z->zinv_lines;
 }
 
 // The plane kernel reaches the modes of a plane by 32-bit byte offsets into six fields.
@@ -54,7 +55,7 @@ int xpass_tiles(const pdr_ctx* c) {
   return (c->g.ny + rb - 1) / rb;
 }
 
-hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf) { return c->ops_z->zinv(c, cf); }
+hipError_t launch2_zinv(pdr_ctx* c, const Coef& cf) { return c->zall ? c->ops_z->zall_inv(c, cf) : c->ops_z->zinv(c, cf); }
 hipError_t launch2_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc) {
   return cf.y3 ? c->ops_y->yinv5(c, cf, z0, nzc) : c->ops_y->yinv(c, z0, nzc);
 }
@@ -64,7 +65,7 @@ hipError_t launch2_yinv(pdr_ctx* c, const Coef& cf, int z0, int nzc) {
 // fields of its tile of i-lines, so that it has the velocity's modes in any case (with the
 // fields split over workgroups, or whole-plane tiles, they would be read once more).
 bool z5_fields(const pdr_ctx* c, const Coef& cf) {
-  return c->spec && !conv_form(c) && !plane_fused(c) && !c->ops_z->zz && c->fpb_y == 6 &&
+  return c->spec && !conv_form(c) && !plane_fused(c) && !c->zall && c->fpb_y == 6 &&
          !(c->ops_y->y_planes > 0 && c->g.nki == c->g.ny / 3 + 1) && cf.G[20] == 0.0 && cf.G[23] == 0.0 &&
          cf.G[26] == 0.0;
 }
@@ -78,9 +79,9 @@ hipError_t launch2_xpass_conv(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, dou
 hipError_t launch2_yfwd(pdr_ctx* c, int z0, int nzc) { return c->ops_y->yfwd(c, z0, nzc); }
 hipError_t launch2_zfwd(pdr_ctx* c) { return c->ops_z->zfwd(c); }
 // Whether the z forward pass can go on with the next stage's z inverse
-bool zz_fused(const pdr_ctx* c) { return c->spec && !conv_form(c) && c->fuse_zf && c->ops_z->zz; }
+bool zz_fused(const pdr_ctx* c) { return c->spec && !conv_form(c) && c->fuse_zf && c->zall; }
 hipError_t launch2_zfwd_formf(pdr_ctx* c, const Coef& cf, const Coef* next, double beta, double gdt) {
-  return c->ops_z->zfwd_formf(c, cf, next, beta, gdt);
+  return c->zall ? c->ops_z->zall_fwd(c, cf, next, beta, gdt) : c->ops_z->zfwd_formf(c, cf, beta, gdt);
 }
 
 }  // namespace pdr

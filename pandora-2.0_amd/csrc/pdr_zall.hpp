@@ -13,10 +13,10 @@
 #pragma once
 #include "pdr_passes.hpp"
 
-// Longest lines: up to here the joined kernel beats the two it replaces (us a launch by
-// events: 64 points 12.4 against 12.3 + 11.8 in FP64 and 11.0 against 12.4 + 11.0 in
-// FP32-mixed, 128 points FP32-mixed 25.5 against 19.1 + 16.5; 128 points FP64 44.0 against
-// 19.0 + 21.5).
+// Longest lines: up to here the joined kernel beats the two it replaces in a box of few
+// lines (us a launch by events: 64 points 12.4 against 12.3 + 11.8 in FP64 and 11.0 against
+// 12.4 + 11.0 in FP32-mixed, 128 points FP32-mixed 25.5 against 19.1 + 16.5; 128 points FP64
+// 44.0 against 19.0 + 21.5); zall_most has the lines.
 #ifndef PDR_ZALL_MAX_F32
 #define PDR_ZALL_MAX_F32 128
 #endif
@@ -32,6 +32,18 @@ namespace {
 template <typename T>
 constexpr int zall_lines(int n) {
   return n > (sizeof(T) == 4 ? PDR_ZALL_MAX_F32 : PDR_ZALL_MAX_F64) ? 0 : (sizeof(T) == 4 && n > 64 ? 8 : 4);
+}
+// Most z lines (i, j) of a single box that takes them.  Up to 80 points they win at any
+// number (us a step, the separate passes -> these: 256 x 256 x 64 FP64 594 -> 539, 256 x 256
+// x 80 FP64 731 -> 720); above, a workgroup's tile is half the LDS of a CU or more, and the
+// separate passes' smaller ones move more at a time once there are lines enough for them
+// (90 to 96 points FP64: 96 x 96 x 96, 2145 lines, 229 / 230, 128 x 128, 3655 lines, 271 ->
+// 296, 256 x 256, 14706 lines, 906 -> 989; FP32-mixed: 96 points 128 x 128 194 -> 178, 192 x
+// 128, 5525 lines, 254 / 254, 256 x 256 512 -> 563, 128 points 192 x 128 304 -> 301, 192 x
+// 192, 8385 lines, 433 -> 446).
+template <typename T>
+constexpr long long zall_most(int n) {
+  return n <= 80 ? (1ll << 40) : sizeof(T) == 4 ? 6000 : 3000;
 }
 template <typename T>
 constexpr int zall_lds_bytes(int n) {

@@ -74,7 +74,10 @@ def test_planes_over_workgroups(oracle_mod, form, n, nz, prec, groups, parts, jo
 
 
 @pytest.mark.parametrize("shape,prec,fields", [((128, 24, 384), F64, 5), ((128, 24, 384), F32, 5), ((100, 30, 512), F64, 5),
-                                               ((32, 36, 1024), F32, 5), ((32, 36, 1024), F64, 6), ((128, 24, 128), F64, 6)],
+                                               ((32, 36, 1024), F32, 5), ((32, 36, 1024), F64, 6), ((128, 24, 128), F64, 6),
+                                               # short z lines in boxes of too many for the joined pass
+                                               ((192, 192, 96), F64, 6), ((192, 192, 96), F32, 6), ((512, 48, 96), F64, 5),
+                                               ((512, 60, 128), F32, 5)],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_fields_through_z(oracle_mod, shape, prec, fields):
     note(f"{shape} bfrot precision {prec}: {fields} fields through z; 3 steps")

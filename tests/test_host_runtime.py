@@ -194,6 +194,12 @@ def test_routes_of_a_box(stand_in):
         ((64, 64, 256, F64), {}, (1, 4, 0, 6, 16)),
         ((64, 64, 640, F64), {}, (1, 4, 0, 6, 16)),
         ((24, 24, 256, F64), {}, (1, 1, 0, 6, 24)),
+        ((96, 96, 96, F64), {}, (0, 0, 1, 6, 8)),
+        ((128, 128, 96, F64), {}, (0, 0, 0, 6, 4)),
+        ((128, 128, 96, F32), {}, (0, 0, 1, 6, 4)),
+        ((192, 192, 96, F32), {}, (0, 0, 0, 6, 4)),
+        ((512, 48, 96, F64), {}, (0, 0, 0, 5, 2)),
+        ((512, 512, 80, F64), {}, (0, 0, 1, 6, 2)),
         ((64, 60, 64, F64), {}, (0, 0, 1, 6, 16)),
         ((32, 32, 32, F64), dict(dealiasing=2), (4, 4, 0, 6, 8)),
         ((32, 32, 32, F64), dict(sheared, ns_deformed=2), (0, 0, 0, 6, 8)),
