@@ -336,13 +336,15 @@ __global__ void __launch_bounds__((zinv_threads<T>(N))) __attribute__((amdgpu_wa
   }
 }
 
-// The thread index of a phase of the z passes: formed anew (fresh_tid) from 256 points up,
-// where the indices of all phases would take registers that a second (zinv) or third (zff)
-// workgroup needs; shorter lines have the registers (128^3 FP64 is 3 us a launch faster so).
-template <int N>
+// The thread index of a phase of the z passes.  FRESH: formed anew (fresh_tid), so that the
+// indices of all phases together do not take the registers that another workgroup on the CU
+// needs; it lengthens a workgroup's own chain, and is for lengths whose registers it brings
+// below that line, in boxes of more workgroups than the CUs hold otherwise.
+template <bool FRESH>
 __device__ __forceinline__ int phase_tid() {
-  return N >= 256 ? fresh_tid() : int(threadIdx.x);
+  return FRESH ? fresh_tid() : int(threadIdx.x);
 }
+constexpr int kCus = 256;
 
 // ---------------------------------------------------------------------------
 // pass 1, register form: the three velocity fields of a tile are loaded once
@@ -385,16 +387,25 @@ template <typename T, int ZT>
 constexpr int lds_zinv_bytes_t(int n) {
   return (n + zinv_lines_t<T, ZT>(n) * lds_ld<T>(n)) * int(sizeof(cx<T>));
 }
-// waves per SIMD declared to the register allocator: two workgroups per CU where the LDS admits
-// them: their indices formed anew in each phase leave the velocity modes room in 128 registers
-// (512^3 FP32-mixed 189 -> 122, one workgroup -> two; spilled before at two)
+// Two workgroups per CU, where the LDS admits them, need the velocity modes and the indices
+// in 128 registers: up to 256 points they fit, above only with FRESH indices (512^3
+// FP32-mixed 189 -> 122), of which 360, 432 and 480 points in FP32 spill.  Up to one
+// workgroup per CU there is no second to make room for (us a launch, FRESH -> not: 64 x 64 x
+// 512 FP32-mixed 45.4 -> 34.4, 96 x 96 x 384 43.0 -> 33.4, 64 x 64 x 384 FP64 33.0 -> 28.0;
+// more workgroups: 512^3 FP32-mixed 440 -> 464, FP64 748 -> 801, 192 x 192 x 384 FP64 101 ->
+// 119; 256^3 FP32-mixed 57.3 -> 50.1, FP64 98.2 -> 88.0; 320 x 320 x 480 FP32-mixed 264 ->
+// 222).
 template <typename T>
-constexpr int zinv_waves_t(int n) {
-  return PDR_ZINV_THREADS / kBlock2 * waves_for(lds_zinv_bytes_t<T, PDR_ZINV_THREADS>(n));
+constexpr bool zinv_fresh(int n) {
+  return n > 256 && !(sizeof(T) == 4 && (n == 360 || n == 432 || n == 480));
 }
-#define PDR_ZINV_WAVES_T __attribute__((amdgpu_waves_per_eu(zinv_waves_t<T>(N))))
+// waves per SIMD declared to the register allocator
+template <typename T, bool FRESH>
+constexpr int zinv_waves_t(int n) {
+  return PDR_ZINV_THREADS / kBlock2 * (FRESH || n < 256 ? waves_for(lds_zinv_bytes_t<T, PDR_ZINV_THREADS>(n)) : 1);
+}
 
-template <typename T, int N, int ZT = kBlock2>
+template <typename T, int N, int ZT = kBlock2, bool FRESH = false>
 __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ u0, const cx<T>* __restrict__ u1,
               const cx<T>* __restrict__ u2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg, int ntile) {
   constexpr int L = zinv_lines_t<T, ZT>(N);
@@ -431,7 +442,7 @@ __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const
 #pragma unroll
   for (int f = 0; f < 6; ++f) {  // unrolled: every field selection is static
     if (f == 5 && cf.y3) break;  // the inverse y pass forms the last vorticity component
-    const int t0 = phase_tid<N>();
+    const int t0 = phase_tid<FRESH>();
 #pragma unroll
     for (int q = 0; q < QM; ++q) {
       const int e = t0 + ZT * q;
@@ -461,9 +472,9 @@ __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const
     }
     zero_band_edges<T, N, L, LD, K, ZT>(buf, t0);
     __syncthreads();
-    fft_ip<T, N, L, LD, +1, true, ZT, K>(buf, tw, phase_tid<N>());
+    fft_ip<T, N, L, LD, +1, true, ZT, K>(buf, tw, phase_tid<FRESH>());
     cx<T>* dst = w1 + (long long)f * g.m1 + (long long)i * N * g.ldj + j0;
-    for (int idx = phase_tid<N>(); idx < L * N; idx += ZT) {
+    for (int idx = phase_tid<FRESH>(); idx < L * N; idx += ZT) {
       const int z = idx / L;
       const int line = idx - z * L;
       if (j0 + line < nkj) put<kNtZinv>(&dst[z * g.ldj + line], buf[line * LD + lds_off<T>(z)]);
@@ -472,11 +483,11 @@ __device__ __forceinline__ void k2_zinv_r_body(unsigned bid, const Geo& g, const
   }
 }
 
-template <typename T, int N>
-__global__ void __launch_bounds__(PDR_ZINV_THREADS) PDR_ZINV_WAVES_T
+template <typename T, int N, bool FRESH>
+__global__ void __launch_bounds__(PDR_ZINV_THREADS) __attribute__((amdgpu_waves_per_eu(zinv_waves_t<T, FRESH>(N))))
     k2_zinv_r(Geo g, Coef cf, const cx<T>* __restrict__ u0, const cx<T>* __restrict__ u1,
               const cx<T>* __restrict__ u2, cx<T>* __restrict__ w1, const cx<T>* __restrict__ twg, int ntile) {
-  k2_zinv_r_body<T, N, PDR_ZINV_THREADS>(xcd_remap(blockIdx.x, gridDim.x), g, cf, u0, u1, u2, w1, twg, ntile);
+  k2_zinv_r_body<T, N, PDR_ZINV_THREADS, FRESH>(xcd_remap(blockIdx.x, gridDim.x), g, cf, u0, u1, u2, w1, twg, ntile);
 }
 
 // ---------------------------------------------------------------------------
@@ -1264,7 +1275,21 @@ __global__ void __launch_bounds__((zthreads(N))) __attribute__((amdgpu_waves_per
 #ifndef PDR_ZFF_PF
 #define PDR_ZFF_PF 1
 #endif
-template <typename T, int N, int FT = kBlock2, int FRC = 2>
+// FRESH indices where they bring the compiled kernel's registers from two workgroups of 256
+// threads per CU to three, which depends on the length and on the forcing's code (FRC as
+// below); in boxes of more than two per CU (us a launch, FRESH -> not: unforced 512^3
+// FP32-mixed 533 -> 568, 320 x 320 x 480 224 -> 252, 192 x 128 x 256 FP64 57.8 -> 64.3, forced
+// 384^3 FP32-mixed 249 -> 267; two per CU 64 x 64 x 512 FP32-mixed 32.5 -> 28.9, 128 x 96 x 256
+// FP64 33.2 -> 30.9; two, or three, in both forms 256^3 FP32-mixed 80.9 -> 75.0, 384^3
+// 252 -> 239, FP64 499 -> 486, forced 512^3 FP32-mixed 584 -> 563).
+template <typename T>
+constexpr bool zff_fresh(int n, int frc) {
+  if (sizeof(T) == 8) return n == 256 && frc == 0;
+  const int longest = frc == 0 ? 512 : frc == 1 ? 432 : 384;
+  const int three = frc == 0 ? 384 : frc == 1 ? 320 : 256;  // multiples of 32 up to here have three
+  return n > 256 && n <= longest && (n % 32 != 0 || n > three);
+}
+template <typename T, int N, int FT = kBlock2, int FRC = 2, bool FRESH = false>
 __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ w1, int parts, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                   cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1, cx<T>* __restrict__ r2,
                   const double2* __restrict__ frc, int fnk, double fkf, double beta, double gdt,
@@ -1288,7 +1313,7 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
   cx<T> nlv[3][QF];
   auto load = [&](int f) {
     const cx<T>* src = w1 + (long long)f * g.m1 + (long long)i * N * g.ldj + j0;
-    const int t0 = phase_tid<N>();
+    const int t0 = phase_tid<FRESH>();
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
       const int idx = t0 + FT * q;
@@ -1316,7 +1341,7 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
 #pragma unroll
   for (int f = 0; f < 3; ++f) {
     if constexpr (!PF) load(f);
-    const int ts = phase_tid<N>();
+    const int ts = phase_tid<FRESH>();
 #pragma unroll
     for (int q = 0; q < QE; ++q) {
       const int idx = ts + FT * q;
@@ -1329,8 +1354,8 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
     if constexpr (PF) {
       if (f < 2) load(f + 1);
     }
-    fft_ip<T, N, L, LD, -1, true, FT>(buf, tw, phase_tid<N>());
-    const int tm = phase_tid<N>();
+    fft_ip<T, N, L, LD, -1, true, FT>(buf, tw, phase_tid<FRESH>());
+    const int tm = phase_tid<FRESH>();
 #pragma unroll
     for (int q = 0; q < QF; ++q) {
       const int idx = tm + FT * q;
@@ -1342,7 +1367,7 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
     __syncthreads();
   }
   const long long e0 = ((long long)i * nkj + j0) * NKK;
-  const int te = phase_tid<N>();
+  const int te = phase_tid<FRESH>();
 #pragma unroll
   for (int q = 0; q < QF; ++q) {
     const int idx = te + FT * q;
@@ -1355,13 +1380,13 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
 }
 
 // FRC: 0 unforced, 1 isotropic forcing, 2 deformed isotropic forcing
-template <typename T, int N, int FRC>
+template <typename T, int N, int FRC, bool FRESH>
 __global__ void __launch_bounds__(kBlock2) PDR_FWD_WAVES
     k2_zfwd_formf(Geo g, Coef cf, const cx<T>* __restrict__ w1, int parts, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                   cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1, cx<T>* __restrict__ r2,
                   const double2* __restrict__ frc, int fnk, double fkf, double beta, double gdt,
                   const cx<T>* __restrict__ twg, int ntile, T norm) {
-  k2_zfwd_formf_body<T, N, kBlock2, FRC>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w1, parts, u0, u1, u2, r0, r1, r2, frc,
+  k2_zfwd_formf_body<T, N, kBlock2, FRC, FRESH>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w1, parts, u0, u1, u2, r0, r1, r2, frc,
                                          fnk, fkf, beta, gdt, twg, ntile, norm);
 }
 
@@ -1397,12 +1422,19 @@ hipError_t zinv_n(pdr_ctx* c, const Coef& cf) {
     constexpr int L = zinv_lines_t<T, PDR_ZINV_THREADS>(N);
     const int nt = (g.nkj + L - 1) / L;
     const size_t lds = size_t(lds_zinv_bytes_t<T, PDR_ZINV_THREADS>(N));
-    hipError_t e = big_lds((const void*)k2_zinv_r<T, N>, lds);
-    if (e != hipSuccess) return e;
-    k2_zinv_r<T, N><<<dim3(unsigned(nt * g.nki)), PDR_ZINV_THREADS, lds, c->stream>>>(
-        g, cf, (const cx<T>*)c->u[0], (const cx<T>*)c->u[1], (const cx<T>*)c->u[2], (cx<T>*)c->w1,
-        (const cx<T>*)c->tab.twz, nt);
-    return hipGetLastError();
+    auto launch = [&](auto fresh_c) -> hipError_t {
+      constexpr bool FRESH = decltype(fresh_c)::value;
+      hipError_t e = big_lds((const void*)k2_zinv_r<T, N, FRESH>, lds);
+      if (e != hipSuccess) return e;
+      k2_zinv_r<T, N, FRESH><<<dim3(unsigned(nt * g.nki)), PDR_ZINV_THREADS, lds, c->stream>>>(
+          g, cf, (const cx<T>*)c->u[0], (const cx<T>*)c->u[1], (const cx<T>*)c->u[2], (cx<T>*)c->w1,
+          (const cx<T>*)c->tab.twz, nt);
+      return hipGetLastError();
+    };
+    if constexpr (zinv_fresh<T>(N)) {
+      if (nt * g.nki > kCus) return launch(std::true_type{});
+    }
+    return launch(std::false_type{});
   } else {
     constexpr int L = tile_lines<T>(N);
     const int nt = (g.nkj + L - 1) / L;
@@ -1553,15 +1585,22 @@ hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
   const int nt = (g.nkj + L - 1) / L;
   const size_t lds = lds_fwd<T, N>();
   const double norm = 1.0 / (double(g.nx) * double(g.ny) * double(g.nz));
-  auto launch = [&](auto frc_c) -> hipError_t {
+  auto launch_f = [&](auto frc_c, auto fresh_c) -> hipError_t {
     constexpr int F = decltype(frc_c)::value;
-    hipError_t e = big_lds((const void*)k2_zfwd_formf<T, N, F>, lds);
+    constexpr bool FRESH = decltype(fresh_c)::value;
+    hipError_t e = big_lds((const void*)k2_zfwd_formf<T, N, F, FRESH>, lds);
     if (e != hipSuccess) return e;
-    k2_zfwd_formf<T, N, F><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
+    k2_zfwd_formf<T, N, F, FRESH><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
         g, cf, (const cx<T>*)(c->nl_parts > 1 ? c->w2 : c->w1), c->nl_parts, (cx<T>*)c->u[0], (cx<T>*)c->u[1],
         (cx<T>*)c->u[2], (cx<T>*)c->rk[0], (cx<T>*)c->rk[1], (cx<T>*)c->rk[2], F ? (const double2*)c->force : nullptr, F ? c->force_nk : 0,
         F ? c->p.force_kf : 0.0, beta, gdt, (const cx<T>*)c->tab.twz, nt, T(norm));
     return hipGetLastError();
+  };
+  auto launch = [&](auto frc_c) -> hipError_t {
+    if constexpr (zff_fresh<T>(N, decltype(frc_c)::value)) {
+      if (nt * g.nki > 2 * kCus) return launch_f(frc_c, std::true_type{});
+    }
+    return launch_f(frc_c, std::false_type{});
   };
   if (!c->forcing) return launch(std::integral_constant<int, 0>{});
   if (cf.fdef) return launch(std::integral_constant<int, 2>{});
