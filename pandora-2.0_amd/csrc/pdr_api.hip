@@ -513,10 +513,10 @@ int pdr_create(pdr_ctx** out, const pdr_params* p) {
     c->fuse_zf = !(env && env[0] == '0') && nz <= 512;
   }
   // fused planes: groups of a plane's parts on their own workgroups until the chip's
-  // 256 CUs have one each (the z forward pass then adds their results; the separate z
-  // forward of long lines reads one).  A step of 64^3 FP64: 180 us with one group, 115
+  // 256 CUs have one each (the z forward pass of all fields at once then adds their
+  // results; the others read one).  A step of 64^3 FP64: 180 us with one group, 115
   // with two, 91 with four; of 32^3 106, 69 and 53.
-  if (plane_fused(c) && c->fuse_zf) c->nl_parts = std::max(1, std::min({kNlParts, c->ops_x->plane_parts, (256 + nz - 1) / nz}));
+  if (plane_fused(c) && c->fuse_zf && c->zall) c->nl_parts = std::max(1, std::min({kNlParts, c->ops_x->plane_parts, (256 + nz - 1) / nz}));
   fft_plan(&c->pz, nz);
   fft_plan(&c->py, ny);
   fft_plan(&c->px, nx);

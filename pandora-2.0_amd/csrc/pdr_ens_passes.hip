@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(kBlock2) k_ens_zfwd_formf(const EnsMember* __r
                                                           double gamma) {
   const unsigned b = xcd_remap(blockIdx.x, gridDim.x), per = unsigned(nt) * (N / 3 + 1);
   const EnsMember& e = mem[b / per];
-  k2_zfwd_formf_body<T, N, kBlock2, 0, zff_fresh<T>(N, 0)>(b % per, e.g, e.cf, (const cx<T>*)e.w1, 1, (cx<T>*)e.u[0], (cx<T>*)e.u[1],
+  k2_zfwd_formf_body<T, N, kBlock2, 0, zff_fresh<T>(N, 0)>(b % per, e.g, e.cf, (const cx<T>*)e.w1, (cx<T>*)e.u[0], (cx<T>*)e.u[1],
                                        (cx<T>*)e.u[2], (cx<T>*)e.rk[0], (cx<T>*)e.rk[1], (cx<T>*)e.rk[2], nullptr, 0,
                                        0.0, beta, gamma * e.dt, (const cx<T>*)e.twz, nt, T(e.norm));
 }

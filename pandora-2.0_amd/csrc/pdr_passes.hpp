@@ -1289,8 +1289,8 @@ constexpr bool zff_fresh(int n, int frc) {
   const int three = frc == 0 ? 384 : frc == 1 ? 320 : 256;  // multiples of 32 up to here have three
   return n > 256 && n <= longest && (n % 32 != 0 || n > three);
 }
-template <typename T, int N, int FT = kBlock2, int FRC = 2, bool FRESH = false, bool MULTI = false>
-__device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ w1, int parts, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
+template <typename T, int N, int FT = kBlock2, int FRC = 2, bool FRESH = false>
+__device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, const Coef& cf, const cx<T>* __restrict__ w1, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                   cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1, cx<T>* __restrict__ r2,
                   const double2* __restrict__ frc, int fnk, double fkf, double beta, double gdt,
                   const cx<T>* __restrict__ twg, int ntile, T norm) {
@@ -1320,19 +1320,6 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
       const int z = idx / L;
       const int line = idx - z * L;
       pre[q] = ((L * N % FT == 0 || idx < L * N) && j0 + line < nkj) ? src[z * g.ldj + line] : czero<T>();
-    }
-    // MULTI: the plane pass left NL as several addends (a form of its own: the loop alone takes
-    // 3 % of a launch, 256 x 256 x 128 FP32-mixed 38.8 -> 37.5 us without)
-#pragma unroll 1
-    for (int p = 1; MULTI && p < parts; ++p) {
-      src += 3 * g.m1;
-#pragma unroll
-      for (int q = 0; q < QE; ++q) {
-        const int idx = t0 + FT * q;
-        const int z = idx / L;
-        const int line = idx - z * L;
-        if ((L * N % FT == 0 || idx < L * N) && j0 + line < nkj) pre[q] = add(pre[q], src[z * g.ldj + line]);
-      }
     }
   };
   // FP32 lines of 256..512 points: the next field's loads are issued before
@@ -1382,13 +1369,13 @@ __device__ __forceinline__ void k2_zfwd_formf_body(unsigned bid, const Geo& g, c
 }
 
 // FRC: 0 unforced, 1 isotropic forcing, 2 deformed isotropic forcing
-template <typename T, int N, int FRC, bool FRESH, bool MULTI>
+template <typename T, int N, int FRC, bool FRESH>
 __global__ void __launch_bounds__(kBlock2) PDR_FWD_WAVES
-    k2_zfwd_formf(Geo g, Coef cf, const cx<T>* __restrict__ w1, int parts, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
+    k2_zfwd_formf(Geo g, Coef cf, const cx<T>* __restrict__ w1, cx<T>* __restrict__ u0, cx<T>* __restrict__ u1,
                   cx<T>* __restrict__ u2, cx<T>* __restrict__ r0, cx<T>* __restrict__ r1, cx<T>* __restrict__ r2,
                   const double2* __restrict__ frc, int fnk, double fkf, double beta, double gdt,
                   const cx<T>* __restrict__ twg, int ntile, T norm) {
-  k2_zfwd_formf_body<T, N, kBlock2, FRC, FRESH, MULTI>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w1, parts, u0, u1, u2, r0, r1, r2, frc,
+  k2_zfwd_formf_body<T, N, kBlock2, FRC, FRESH>(xcd_remap(blockIdx.x, gridDim.x), g, cf, w1, u0, u1, u2, r0, r1, r2, frc,
                                          fnk, fkf, beta, gdt, twg, ntile, norm);
 }
 
@@ -1587,26 +1574,22 @@ hipError_t zfwd_formf_n(pdr_ctx* c, const Coef& cf, double beta, double gdt) {
   const int nt = (g.nkj + L - 1) / L;
   const size_t lds = lds_fwd<T, N>();
   const double norm = 1.0 / (double(g.nx) * double(g.ny) * double(g.nz));
-  auto launch_f = [&](auto frc_c, auto fresh_c, auto multi_c) -> hipError_t {
+  auto launch_f = [&](auto frc_c, auto fresh_c) -> hipError_t {
     constexpr int F = decltype(frc_c)::value;
     constexpr bool FRESH = decltype(fresh_c)::value;
-    constexpr bool MULTI = decltype(multi_c)::value;
-    hipError_t e = big_lds((const void*)k2_zfwd_formf<T, N, F, FRESH, MULTI>, lds);
+    hipError_t e = big_lds((const void*)k2_zfwd_formf<T, N, F, FRESH>, lds);
     if (e != hipSuccess) return e;
-    k2_zfwd_formf<T, N, F, FRESH, MULTI><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
-        g, cf, (const cx<T>*)(c->nl_parts > 1 ? c->w2 : c->w1), c->nl_parts, (cx<T>*)c->u[0], (cx<T>*)c->u[1],
+    k2_zfwd_formf<T, N, F, FRESH><<<dim3(unsigned(nt * g.nki)), kBlock2, lds, c->stream>>>(
+        g, cf, (const cx<T>*)c->w1, (cx<T>*)c->u[0], (cx<T>*)c->u[1],
         (cx<T>*)c->u[2], (cx<T>*)c->rk[0], (cx<T>*)c->rk[1], (cx<T>*)c->rk[2], F ? (const double2*)c->force : nullptr, F ? c->force_nk : 0,
         F ? c->p.force_kf : 0.0, beta, gdt, (const cx<T>*)c->tab.twz, nt, T(norm));
     return hipGetLastError();
   };
   auto launch = [&](auto frc_c) -> hipError_t {
     if constexpr (zff_fresh<T>(N, decltype(frc_c)::value)) {
-      if (nt * g.nki > 2 * kCus) return launch_f(frc_c, std::true_type{}, std::false_type{});
+      if (nt * g.nki > 2 * kCus) return launch_f(frc_c, std::true_type{});
     }
-    if constexpr (N < kCus) {  // (planes in groups: fewer than one for each CU, pdr_create)
-      if (c->nl_parts > 1) return launch_f(frc_c, std::false_type{}, std::true_type{});
-    }
-    return launch_f(frc_c, std::false_type{}, std::false_type{});
+    return launch_f(frc_c, std::false_type{});
   };
   if (!c->forcing) return launch(std::integral_constant<int, 0>{});
   if (cf.fdef) return launch(std::integral_constant<int, 2>{});

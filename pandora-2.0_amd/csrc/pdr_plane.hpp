@@ -36,6 +36,17 @@ constexpr int plane_lds_bytes(int n, int s) {
   const int x = 3 * m * lds_ld<T>(n), y = 6 * nki * lds_ld<T>(m);
   return (n + (s > 1 ? n + m : 0) + (x > y ? x : y)) * int(sizeof(cx<T>));
 }
+// Deepest boxes that take them: with a plane in parts, an under-filled chip's worth of planes
+// (us a step, separate passes -> these: 32 points FP64 64 planes 76 -> 56, 96 planes 87 -> 85,
+// 160 151 -> 150, 256 183 -> 196, 64 points FP64 64 planes 104 -> 91, 72 121 -> 137, 256
+// 254 -> 272, 512 431 -> 495; FP32-mixed 48 points 128 planes 117 -> 105, 144 182 -> 184, 256
+// 222 -> 230, 64 points 80 planes 102 -> 93, 96 107 -> 110, 256 218 -> 238); planes in one
+// part at any depth (24 points FP64 512 planes 259 -> 212).
+template <typename T>
+constexpr int plane_most(int n, int s) {
+  if (s == 1) return 1 << 30;
+  return sizeof(T) == 4 ? (n > 60 ? 80 : 128) : (n > 48 ? 64 : 96);
+}
 // Threads: the first x pass's butterflies in as few equal rounds as 1024 threads allow.
 constexpr int plane_threads(int n, int s) {
   const int b = 3 * (n / s) * (n / plan_radix(n, 0));

@@ -43,6 +43,7 @@ SpecOps ops_of() {
   constexpr int parts = plane_parts_box<T>(N);
   o.plane = parts ? plane_n<T, N> : nullptr;
   o.plane_parts = parts;
+  o.plane_most = parts ? plane_most<T>(N, parts) : 0;
   o.lds_plane = parts ? size_t(plane_lds_bytes<T>(N, parts) + plane_static_bytes<T>(N, parts)) : 0;
   o.lds_z = lds_lines<T, N>() > lds_fwd<T, N>() ? lds_lines<T, N>() : lds_fwd<T, N>();
   o.lds_y = lds_y<T, N>();

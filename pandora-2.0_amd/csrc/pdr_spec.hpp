@@ -28,6 +28,7 @@ struct SpecOps {
   hipError_t (*plane)(pdr_ctx*, const Coef&, bool tr, bool cfl, double* rsp);
   size_t lds_plane;  // the kernel's own arrays included
   int plane_parts;
+  int plane_most;  // most planes of a box that takes them
   size_t lds_z, lds_y, lds_x, lds_xc;  // the largest workgroup of the z, y, x and NS_R_CONV x passes
   int xrows, xrows_rs, xrows_conv;  // rows of an x tile; with the moments; NS_R_CONV
   int x_tw_global;             // 1: the x tile reads its twiddles from the global table

@@ -42,7 +42,8 @@ static bool plane_offsets_fit(const pdr_ctx* c) { return 6 * size_t(c->g.m1) * c
 // that has it, unless the environment asks for the chunked passes or their streams.
 bool plane_fused(const pdr_ctx* c) {
   return c->spec && !conv_form(c) && !c->plane_separate && c->g.nx == c->g.ny && c->ops_x->plane &&
-         c->ops_x->lds_plane <= c->lds_max && plane_offsets_fit(c) && c->g.zc == c->g.nz;
+         c->g.nz <= c->ops_x->plane_most && c->ops_x->lds_plane <= c->lds_max && plane_offsets_fit(c) &&
+         c->g.zc == c->g.nz;
 }
 hipError_t launch2_plane(pdr_ctx* c, const Coef& cf, bool tr, bool cfl, double* rsp) {
   return c->ops_x->plane(c, cf, tr, cfl, rsp);

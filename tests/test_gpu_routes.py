@@ -1,7 +1,7 @@
 """The passes that a box's steps take together (pdr_kernel_routes) at the sizes where the rule
 changes, each against the FP64 oracle: fused planes over four workgroups down to one, a
-workgroup with several of a plane's parts among them, before the joined z pass and before the
-separate z forward + FormF, which add the groups' results; and five or six fields through z."""
+workgroup with several of a plane's parts among them, whose results the joined z pass adds;
+boxes too deep for them; and five or six fields through z."""
 import sys
 
 import numpy as np
@@ -17,15 +17,15 @@ F64, F32 = pa.PDR_FP64, pa.PDR_FP32_MIXED
 PLANES = [
     (32, 32, F64, 4, 4, 1),
     (32, 72, F32, 4, 4, 1),
-    (64, 96, F64, 3, 4, 1),    # a group has two of the four parts
-    (64, 96, F32, 3, 4, 1),
-    (64, 128, F64, 2, 4, 0),   # z forward + FormF adds two results
-    (48, 192, F32, 2, 4, 0),
-    (48, 192, F64, 2, 4, 0),
-    (60, 100, F64, 3, 4, 0),   # and three
-    (24, 256, F64, 1, 1, 0),   # one group, its result in place: a plane whole
-    (32, 256, F64, 1, 4, 0),   # and in four parts
-    (64, 300, F32, 1, 4, 0),
+    (48, 96, F64, 3, 4, 1),    # a group has two of the four parts
+    (60, 100, F32, 3, 4, 1),
+    (60, 128, F32, 2, 4, 1),   # each has two
+    (64, 80, F32, 4, 4, 1),
+    (24, 256, F64, 1, 1, 0),   # a plane whole, its result in place
+    (30, 128, F32, 1, 1, 1),
+    (64, 96, F64, 0, 0, 1),    # too deep for planes in parts
+    (64, 128, F64, 0, 0, 0),
+    (48, 192, F32, 0, 0, 0),
 ]
 
 

@@ -188,12 +188,16 @@ def test_routes_of_a_box(stand_in):
         ((64, 64, 64, F64), {}, (4, 4, 1, 6, 16)),
         ((30, 30, 30, F64), {}, (1, 1, 1, 6, 30)),
         ((72, 72, 72, F64), {}, (0, 0, 1, 6, 8)),
-        ((64, 64, 96, F64), {}, (3, 4, 1, 6, 16)),
-        ((64, 64, 128, F64), {}, (2, 4, 0, 6, 16)),
-        ((64, 64, 128, F32), {}, (2, 4, 1, 6, 16)),
-        ((64, 64, 256, F64), {}, (1, 4, 0, 6, 16)),
-        ((64, 64, 640, F64), {}, (1, 4, 0, 6, 16)),
+        ((48, 48, 96, F64), {}, (3, 4, 1, 6, 12)),
+        ((48, 48, 100, F64), {}, (0, 0, 0, 6, 16)),
+        ((64, 64, 72, F64), {}, (0, 0, 1, 6, 16)),
+        ((64, 64, 80, F32), {}, (4, 4, 1, 6, 16)),
+        ((64, 64, 96, F32), {}, (0, 0, 1, 6, 16)),
+        ((60, 60, 128, F32), {}, (2, 4, 1, 6, 15)),
+        ((60, 60, 144, F32), {}, (0, 0, 0, 6, 16)),
         ((24, 24, 256, F64), {}, (1, 1, 0, 6, 24)),
+        ((24, 24, 640, F64), {}, (1, 1, 0, 6, 24)),
+        ((64, 60, 64, F64), {}, (0, 0, 1, 6, 16)),
         ((96, 96, 96, F64), {}, (0, 0, 1, 6, 8)),
         ((128, 128, 96, F64), {}, (0, 0, 0, 6, 4)),
         ((128, 128, 96, F32), {}, (0, 0, 1, 6, 4)),
