@@ -3,12 +3,12 @@
 //
 // A pageable hipMemcpy stages through the runtime's own buffers on one thread, and an
 // FP32-mixed field was converted after it on the same thread, which also took the page
-// faults of the caller's array: 512^3 FP32-mixed velocity read back in 175 ms, 955 MB of
-// host array at 5.5 GB/s.  Here chunks of 1 MB go by DMA into pinned slots and as many
+// faults of the caller's array.  Here chunks of 1 MB go by DMA into pinned slots and as many
 // threads as the size warrants copy or convert them out, two slots each, so that DMA,
-// conversion and page faults overlap: 14 ms there, 12.1 -> 3.7 ms for 256^3 FP64.  A small box's fields go in one kernel
-// that writes them into the pinned memory: one launch and one wait instead of three copies
-// (32^3 FP64 0.13 -> 0.03 ms).
+// conversion and page faults overlap: 512^3 FP32-mixed velocity read back into arrays in use
+// 145 -> 15.3 ms, 324 -> 190 into fresh pages, 256^3 FP64 7.0 -> 3.9 and 33 -> 21.  A small
+// box's fields go in one kernel that writes them into the pinned memory: one launch and one
+// wait instead of three copies (32^3 FP64 0.05 to 0.13 -> 0.03 ms, 48^3 0.074 -> 0.054).
 #include <algorithm>
 #include <cstring>
 #include <string>
